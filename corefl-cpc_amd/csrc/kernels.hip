@@ -5,6 +5,8 @@
 // NS so that they live in VGPRs; NS == 0 selects the Air perfect gas.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "corefl_internal.h"
 #include "fastmath.h"
 
@@ -26,6 +28,8 @@ __constant__ double c_rk_b[3] = {0.0, 0.25, 2.0 / 3.0};
 __constant__ double c_rk_c[3] = {1.0, 0.25, 2.0 / 3.0};
 
 constexpr int kBlock = 256;
+// one wave per block over boundary faces: a face holds few sites, so small blocks reach more compute units
+constexpr int kFaceBlock = 64;
 constexpr int kMaxNv = 5 + COREFL_MAX_SPEC + 1;  // conservative variables: 5, species, E_ve
 
 // Thermochemical model code of the species-templated kernels: species count in
@@ -3522,9 +3526,10 @@ DEV void btype_flags(const Zone &z, int i, int j, int k, bool *ct) {
 // two temperatures Tve (field tve_f), into
 // zg[field] at interior nodes.  A thread owns KC consecutive k of one column
 // and slides a nine-node window along them, so each field is read
-// (KC + 8) / KC times instead of nine by the flux kernel.
+// (KC + 8) / KC times instead of nine by the flux kernel; blockIdx.y takes
+// fpb consecutive fields (column_split).
 template <int KC>
-__global__ __launch_bounds__(kBlock) void k_zeta_grad(Zone z, int ns, int nfield, int tve_f, long ncol) {
+__global__ __launch_bounds__(kBlock) void k_zeta_grad(Zone z, int ns, int nfield, int fpb, int tve_f, long ncol) {
   const long t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (t >= ncol) return;
   const int mx = z.mx, my = z.my, mz = z.mz;
@@ -3536,8 +3541,9 @@ __global__ __launch_bounds__(kBlock) void k_zeta_grad(Zone z, int ns, int nfield
   const long sz = z.sz, sk = z.sxy, dsz = z.dsz, dk = static_cast<long>(mx) * my;
   const bool kl = z.bt_kl[i + j * mx] != 0, kr = z.bt_kr[i + j * mx] != 0;
   const long p0 = z.ix(i, j, k0), q0 = z.dx(i, j, k0);
+  const int f0 = blockIdx.y * fpb, f1 = min(nfield, f0 + fpb);
 #pragma unroll 1
-  for (int f = 0; f < nfield; ++f) {
+  for (int f = f0; f < f1; ++f) {
     const double *src = f == tve_f ? z.tve
                                    : (f < 3 ? z.bv + (f + 1) * sz
                                             : (f == 3 ? z.bv + 5 * sz : (f < 4 + ns ? z.sv + (f - 4) * sz : z.bv + 4 * sz)));
@@ -3736,8 +3742,11 @@ __global__ __launch_bounds__(kBlock) void k_viscous_flux(Zone z, const Tab *__re
 // them, so H is read (KC + 8) / KC times instead of nine.
 // STORE: the derivative is the stage's first contribution to dq and replaces
 // it (a stage recorded without the separate clearing of dq); else it adds.
-template <int NV, int KC, bool STORE>
-__global__ __launch_bounds__(kBlock) void k_viscous_derivative(Zone z, long ncol) {
+// blockIdx.y takes cpb of the components 1 .. nv - 1 (column_split).  With
+// ALL (every component in one block) the chunk's boundary flags and Jacobians
+// are read once and held, else each component reads them for itself.
+template <int KC, bool STORE, bool ALL>
+__global__ __launch_bounds__(kBlock) void k_viscous_derivative(Zone z, int nv, int cpb, long ncol) {
   const long t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (t >= ncol) return;
   const int mx = z.mx, my = z.my, mz = z.mz;
@@ -3750,22 +3759,24 @@ __global__ __launch_bounds__(kBlock) void k_viscous_derivative(Zone z, long ncol
   const bool kl = z.bt_kl[i + j * mx] != 0, kr = z.bt_kr[i + j * mx] != 0;
   const long p0 = z.ix(i, j, k0), q0 = z.dx(i, j, k0);
   static_assert(KC <= 16, "four flag bits per node of a chunk");
-  // the i / j boundary flags of the chunk's nodes, four bits per node, read once for all components
+  // the i / j boundary flags of the chunk's nodes, four bits per node
   unsigned long long fl = 0;
-  __shared__ double jac_s[KC][kBlock];  // the chunk's J, each thread's own column
+  __shared__ double jac_s[ALL ? KC : 1][ALL ? kBlock : 1];  // the chunk's J, each thread's own column
   for (int c = 0; c < nk; ++c) {
     const int k = k0 + c;
     const unsigned b = (z.bt_il[j + k * my] != 0 ? 1u : 0u) | (z.bt_ir[j + k * my] != 0 ? 2u : 0u) |
                        (z.bt_jl[i + k * mx] != 0 ? 4u : 0u) | (z.bt_jr[i + k * mx] != 0 ? 8u : 0u);
     fl |= static_cast<unsigned long long>(b) << (4 * c);
-    jac_s[c][threadIdx.x] = z.jac[p0 + c * sk];
+    if constexpr (ALL) jac_s[c][threadIdx.x] = z.jac[p0 + c * sk];
   }
   if constexpr (STORE) {
     // the continuity equation has no viscous term: its dq starts at 0 here
-    for (int c = 0; c < nk; ++c) z.dq[q0 + c * dk] = 0.0;
+    if (blockIdx.y == 0)
+      for (int c = 0; c < nk; ++c) z.dq[q0 + c * dk] = 0.0;
   }
+  const int l0 = 1 + blockIdx.y * cpb, l1 = min(nv, l0 + cpb);
 #pragma unroll 1
-  for (int l = 1; l < NV; ++l) {
+  for (int l = l0; l < l1; ++l) {
     // nodes k0-4 .. k0+nk+3 lie inside the padded extent (ngg >= 4)
     double w[9];
 #pragma unroll
@@ -3777,13 +3788,14 @@ __global__ __launch_bounds__(kBlock) void k_viscous_derivative(Zone z, long ncol
       w[8] = z.hf[p + 4 * sk + l * sz];
       const unsigned b = static_cast<unsigned>(fl >> (4 * c));
       const bool il = (b & 1u) != 0, ir = (b & 2u) != 0, jl = (b & 4u) != 0, jr = (b & 8u) != 0;
+      const double jac = ALL ? jac_s[ALL ? c : 0][ALL ? threadIdx.x : 0] : z.jac[p];
       const double dxi = d8(z.ff, p + l * sz, si, i, mx, il, ir);
       const double deta = d8(z.gf, p + l * sz, sj, j, my, jl, jr);
       const double dzeta = d8g([&](int o) { return w[4 + o]; }, k, mz, kl, kr);
       if constexpr (STORE)
-        z.dq[q0 + c * dk + l * dsz] = (dxi + deta + dzeta) * jac_s[c][threadIdx.x];
+        z.dq[q0 + c * dk + l * dsz] = (dxi + deta + dzeta) * jac;
       else
-        z.dq[q0 + c * dk + l * dsz] += (dxi + deta + dzeta) * jac_s[c][threadIdx.x];
+        z.dq[q0 + c * dk + l * dsz] += (dxi + deta + dzeta) * jac;
 #pragma unroll
       for (int m = 0; m < 8; ++m) w[m] = w[m + 1];
     }
@@ -4025,7 +4037,13 @@ __global__ void k_periodic_flux(Zone z, corefl_boundary b, int nv) {
 // in sequence average the same coincident nodes twice, the second time to the
 // same values, and copy disjoint ghost layers): threads over the low face's
 // sites; layer 0 averages the coincident pair once, layer g fills both ghosts.
-__global__ void k_periodic_flux_pair(Zone z, corefl_boundary lo, int nv) {
+// A thread takes kFluxGroup of the variables (blockIdx.y): on an i-face every
+// access of a wave is to 64 lines of its own, so all the variables in one
+// thread were a chain of up to 168 such accesses on a few compute units
+// (14 variables, average of the three axes: 33x25x19 21.6 -> 6.1 us,
+// 256x128x128 52 -> 36 us).
+constexpr int kFluxGroup = 4;
+__global__ __launch_bounds__(kFaceBlock) void k_periodic_flux_pair(Zone z, corefl_boundary lo, int nv) {
   FaceSite f;
   if (!face_site(z, lo, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, f)) return;
   const int a = lo.face;
@@ -4033,21 +4051,23 @@ __global__ void k_periodic_flux_pair(Zone z, corefl_boundary lo, int nv) {
   int o[3] = {f.i, f.j, f.k};
   o[a] = n - 1;
   const long sz = z.sz;
+  const int l0 = blockIdx.y * kFluxGroup;
   double *arrs[3] = {z.ff, z.gf, z.hf};
-  double va[kMaxNv], vb[kMaxNv];
+  double va[kFluxGroup], vb[kFluxGroup];
   if (f.layer == 0) {
-    const long p = z.ix(f.i, f.j, f.k), po = z.ix(o[0], o[1], o[2]);
+    const long p = z.ix(f.i, f.j, f.k) + l0 * sz, po = z.ix(o[0], o[1], o[2]) + l0 * sz;
+#pragma unroll
     for (int c = 0; c < 3; ++c) {
       double *fa = arrs[c];
 #pragma unroll
-      for (int l = 0; l < kMaxNv; ++l)
-        if (l < nv) {
+      for (int l = 0; l < kFluxGroup; ++l)
+        if (l0 + l < nv) {
           va[l] = fa[p + l * sz];
           vb[l] = fa[po + l * sz];
         }
 #pragma unroll
-      for (int l = 0; l < kMaxNv; ++l)
-        if (l < nv) {
+      for (int l = 0; l < kFluxGroup; ++l)
+        if (l0 + l < nv) {
           const double ave = 0.5 * (va[l] + vb[l]);
           fa[p + l * sz] = ave;
           fa[po + l * sz] = ave;
@@ -4060,18 +4080,18 @@ __global__ void k_periodic_flux_pair(Zone z, corefl_boundary lo, int nv) {
     li[a] = n - 1 - g;
     hg[a] = n - 1 + g;
     hi[a] = g;
-    double *fa = arrs[a];
+    double *fa = arrs[a] + l0 * sz;
     const long plg = z.ix(lg[0], lg[1], lg[2]), pli = z.ix(li[0], li[1], li[2]);
     const long phg = z.ix(hg[0], hg[1], hg[2]), phi = z.ix(hi[0], hi[1], hi[2]);
 #pragma unroll
-    for (int l = 0; l < kMaxNv; ++l)
-      if (l < nv) {
+    for (int l = 0; l < kFluxGroup; ++l)
+      if (l0 + l < nv) {
         va[l] = fa[pli + l * sz];
         vb[l] = fa[phi + l * sz];
       }
 #pragma unroll
-    for (int l = 0; l < kMaxNv; ++l)
-      if (l < nv) {
+    for (int l = 0; l < kFluxGroup; ++l)
+      if (l0 + l < nv) {
         fa[plg + l * sz] = va[l];
         fa[phg + l * sz] = vb[l];
       }
@@ -4605,7 +4625,7 @@ __global__ void k_bc_periodic(Zone z, const Tab *__restrict__ tb, corefl_boundar
 // layer 0 averages the coincident nodes once and forms both nodes'
 // conservative variables, layer g fills the low and the high ghost.
 template <int M>
-__global__ void k_bc_periodic_pair(Zone z, const Tab *__restrict__ tb, corefl_boundary lo) {
+__global__ __launch_bounds__(kFaceBlock) void k_bc_periodic_pair(Zone z, const Tab *__restrict__ tb, corefl_boundary lo) {
   FaceSite f;
   if (!face_site(z, lo, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, f)) return;
   const int a = lo.face;
@@ -5079,15 +5099,43 @@ hipError_t launch_shock_sensor(const Zone &z, const Run &r, hipStream_t s) {
   return hipGetLastError();
 }
 
+// How the column kernels (k_zeta_grad, k_viscous_derivative) split their work:
+// the k nodes a thread slides its window along and the fields one block takes.
+// A long chunk re-reads less of the k halo ((KC + 8) / KC) and a block with
+// every field reads the column's flags and Jacobians once, but both leave few
+// threads, each with a long serial chain.  So the fields are spread over
+// blocks (and, on the smallest grids, the chunk shortened) until the launch
+// holds kColumnWaves waves, about eight per SIMD of the 256 CUs.  Measured per
+// launch with all fields in 16-node columns -> split: 33x25x19, derivative 250
+// -> 10 us, zeta 70 -> 5 us (4-node chunks); 101x67x53, 285 -> 74 us and 78 ->
+// 18 us; 256x128x128 has the waves without it and stays at 0.61 ms and 0.20 ms.
+struct ColumnSplit {
+  int kc, per_block;
+  long ncol;
+};
+constexpr long kColumnWaves = 8192;
+inline ColumnSplit column_split(const Zone &z, int fields) {
+  ColumnSplit c{16, fields, 0};
+  auto columns = [&](int kc) { return static_cast<long>(z.mx) * z.my * ((z.mz + kc - 1) / kc); };
+  auto waves = [&](int kc) { return (columns(kc) + 63) / 64; };
+  if (waves(16) * 2 < kColumnWaves)
+    c.per_block = static_cast<int>(std::max<long>(1, waves(16) * fields / kColumnWaves));
+  if (c.per_block == 1 && waves(16) * fields < kColumnWaves / 2) c.kc = 4;
+  c.ncol = columns(c.kc);
+  return c;
+}
+
 hipError_t launch_viscous_flux(const Zone &z, const Run &r, const Tab *tb, hipStream_t s) {
-  constexpr int KC = 16;
-  const long ncol = static_cast<long>(z.mx) * z.my * ((z.mz + KC - 1) / KC);
   const int ns = r.mixture ? r.ns : 0;
   // zeta-derivative fields: u, v, w, T, Y_l, (p with the pressure-gradient term), (Tve)
   const int nf = 4 + ns + (r.gradp && ns > 0 ? 1 : 0);
-  const int tve_f = r.tt ? nf : -1;
-  hipLaunchKernelGGL((k_zeta_grad<KC>), dim3(blocks_for(ncol)), dim3(kBlock), 0, s, z, ns, nf + (r.tt ? 1 : 0),
-                     tve_f, ncol);
+  const int tve_f = r.tt ? nf : -1, fields = nf + (r.tt ? 1 : 0);
+  const ColumnSplit c = column_split(z, fields);
+  const dim3 grid(blocks_for(c.ncol), (fields + c.per_block - 1) / c.per_block);
+  if (c.kc == 16)
+    hipLaunchKernelGGL((k_zeta_grad<16>), grid, dim3(kBlock), 0, s, z, ns, fields, c.per_block, tve_f, c.ncol);
+  else
+    hipLaunchKernelGGL((k_zeta_grad<4>), grid, dim3(kBlock), 0, s, z, ns, fields, c.per_block, tve_f, c.ncol);
   const long n = interior_points(z);
   COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_viscous_flux<MV>), dim3(blocks_for(n)), dim3(kBlock), 0, s, z,
                                               tb, r.prandtl, r.gradp, tve_f, n));
@@ -5119,17 +5167,21 @@ hipError_t launch_viscous2(const Zone &z, const Run &r, const Tab *tb, hipStream
   return hipSuccess;
 }
 
-hipError_t launch_viscous_derivative(const Zone &z, const Run &r, hipStream_t s, bool store) {
-  constexpr int KC = 16;
-  const long ncol = static_cast<long>(z.mx) * z.my * ((z.mz + KC - 1) / KC);
-  if (store) {
-    COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_viscous_derivative<kNv(MV), KC, true>),
-                                                dim3(blocks_for(ncol)), dim3(kBlock), 0, s, z, ncol));
-  } else {
-    COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_viscous_derivative<kNv(MV), KC, false>),
-                                                dim3(blocks_for(ncol)), dim3(kBlock), 0, s, z, ncol));
-  }
+template <bool STORE>
+hipError_t launch_derivative_t(const Zone &z, int nv, hipStream_t s) {
+  const ColumnSplit c = column_split(z, nv - 1);
+  const dim3 grid(blocks_for(c.ncol), (nv - 1 + c.per_block - 1) / c.per_block);
+  if (c.kc != 16)
+    hipLaunchKernelGGL((k_viscous_derivative<4, STORE, false>), grid, dim3(kBlock), 0, s, z, nv, c.per_block, c.ncol);
+  else if (c.per_block < nv - 1)
+    hipLaunchKernelGGL((k_viscous_derivative<16, STORE, false>), grid, dim3(kBlock), 0, s, z, nv, c.per_block, c.ncol);
+  else
+    hipLaunchKernelGGL((k_viscous_derivative<16, STORE, true>), grid, dim3(kBlock), 0, s, z, nv, c.per_block, c.ncol);
   return hipGetLastError();
+}
+
+hipError_t launch_viscous_derivative(const Zone &z, const Run &r, hipStream_t s, bool store) {
+  return store ? launch_derivative_t<true>(z, r.nv, s) : launch_derivative_t<false>(z, r.nv, s);
 }
 
 hipError_t launch_periodic_flux(const Zone &z, const Run &r, const corefl_boundary &b, hipStream_t s) {
@@ -5178,14 +5230,15 @@ hipError_t launch_bc_periodic(const Zone &z, const Run &r, const Tab *tb, const 
 hipError_t launch_bc_periodic_pair(const Zone &z, const Run &r, const Tab *tb, const corefl_boundary &lo,
                                   hipStream_t s) {
   const long n = face_points(lo) * (z.ngg + 1);
-  COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_bc_periodic_pair<MV>), dim3(blocks_for(n)), dim3(kBlock), 0, s, z,
-                                              tb, lo));
+  COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_bc_periodic_pair<MV>), dim3(blocks_for(n, kFaceBlock)), dim3(kFaceBlock), 0,
+                                              s, z, tb, lo));
   return hipGetLastError();
 }
 
 hipError_t launch_periodic_flux_pair(const Zone &z, const Run &r, const corefl_boundary &lo, hipStream_t s) {
   const long n = face_points(lo) * (z.ngg + 1);
-  hipLaunchKernelGGL(k_periodic_flux_pair, dim3(blocks_for(n)), dim3(kBlock), 0, s, z, lo, r.nv);
+  hipLaunchKernelGGL(k_periodic_flux_pair, dim3(blocks_for(n, kFaceBlock), (r.nv + kFluxGroup - 1) / kFluxGroup),
+                     dim3(kFaceBlock), 0, s, z, lo, r.nv);
   return hipGetLastError();
 }
 

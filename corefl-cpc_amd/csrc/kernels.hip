@@ -2057,92 +2057,117 @@ __global__ void k_reactor_admit(ReactorPool P, const Tab *__restrict__ tb, const
 // ---------------------------------------------------------------------------
 // WENO5-JS / WENO7-Z (shock branch), src/WENO.cu:3033-3196
 // ---------------------------------------------------------------------------
-// One half of WENO5-JS on the upwind-ordered values v[0..4] (v[2] is the
-// point left of the face), in the differences d_k = v_{k+1} - v_k and their
-// differences D_k: each candidate stencil's beta is u^2 + 13/12 D^2 and its
-// face value v2 + p / 2, with u and p of two terms each, so the flux is v2
-// plus half the weighted mean of the p.  The nonlinear weights d_k /
-// (eps + beta_k)^2 are normalised by their sum, so they are scaled by
-// prod_{m} (eps + beta_m)^2 first: one division per side instead of four.
-// (eps + beta) lies between eps >= 1e-40 (rho v)^2 and the square of the
-// largest characteristic flux, so the products of two squared terms stay
-// inside the double range.  42 FP64 instructions, and a third of the rounding
-// error of the candidate values formed from the v themselves.
-DEV double weno5_half(double v0, double v1, double v2, double v3, double v4, double eps) {
-  constexpr double third = 1.0 / 3, d12 = 13.0 / 12;
-  const double d0 = v1 - v0, d1 = v2 - v1, d2 = v3 - v2, d3 = v4 - v3;
-  const double D0 = d1 - d0, D1 = d2 - d1, D2 = d3 - d2;
-  const double u0 = fma(-0.5, D2, d2), u1 = fma(-0.5, D1, d2), u2 = fma(0.5, D0, d1);
-  const double e0 = fma(u0, u0, fma(d12 * D2, D2, eps));
-  const double e1 = fma(u1, u1, fma(d12 * D1, D1, eps));
-  const double e2 = fma(u2, u2, fma(d12 * D0, D0, eps));
+// The nonlinear weights d_k / (eps + beta_k)^2 are normalised by their sum,
+// so they are scaled by prod_{m} (eps + beta_m)^2 first: one division per
+// side instead of four.  (eps + beta) lies between eps >= 1e-40 (rho v)^2 and
+// the square of the largest characteristic flux, so the products of two
+// squared terms stay inside the double range.
+DEV double weno5_side(double q0, double q1, double q2, double b0, double b1, double b2, double d0, double d1,
+                      double d2, double eps) {
+  const double e0 = eps + b0, e1 = eps + b1, e2 = eps + b2;
   const double e12 = e1 * e2, e02 = e0 * e2, e01 = e0 * e1;
-  // the linear weights 3, 6, 1 (over 10, which cancels in the mean)
-  const double a0 = 3.0 * (e12 * e12), a1 = 6.0 * (e02 * e02), a2 = e01 * e01;
-  const double p0 = fma(-third, D2, d2), p1 = fma(-third, D1, d2), p2 = fma(2 * third, D0, d1);
-  const double num = fma(a0, p0, fma(a1, p1, a2 * p2));
-  return fma(0.5 * num, fast_rcp(a0 + a1 + a2), v2);
+  const double a0 = d0 * (e12 * e12), a1 = d1 * (e02 * e02), a2 = d2 * (e01 * e01);
+  return (a0 * q0 + a1 * q1 + a2 * q2) * fast_rcp(a0 + a1 + a2);
 }
 
-// The left-biased half at the face right of vp[2] (vp = the values at
-// i-2 .. i+2) and the right-biased half at the face left of vm[2] (vm = the
-// values at i-1 .. i+3).
-DEV double weno5_left(const double *vp, double eps) { return weno5_half(vp[0], vp[1], vp[2], vp[3], vp[4], eps); }
-DEV double weno5_right(const double *vm, double eps) { return weno5_half(vm[4], vm[3], vm[2], vm[1], vm[0], eps); }
-DEV double weno5(const double *vp, const double *vm, double eps) { return weno5_left(vp, eps) + weno5_right(vm, eps); }
+// The left-biased half of WENO5-JS at the face right of vp[2] (vp = the
+// values at i-2 .. i+2) and the right-biased half at the face left of vm[2]
+// (vm = the values at i-1 .. i+3), as the two halves of weno5 below.
+DEV double weno5_left(const double *vp, double eps) {
+  constexpr double one6th = 1.0 / 6, thirteen12th = 13.0 / 12;
+  const double v0 = one6th * (2 * vp[2] + 5 * vp[3] - vp[4]);
+  const double v1 = one6th * (-vp[1] + 5 * vp[2] + 2 * vp[3]);
+  const double v2 = one6th * (2 * vp[0] - 7 * vp[1] + 11 * vp[2]);
+  const double beta0 = thirteen12th * (vp[2] + vp[4] - 2 * vp[3]) * (vp[2] + vp[4] - 2 * vp[3]) +
+                       0.25 * (3 * vp[2] - 4 * vp[3] + vp[4]) * (3 * vp[2] - 4 * vp[3] + vp[4]);
+  const double beta1 = thirteen12th * (vp[1] + vp[3] - 2 * vp[2]) * (vp[1] + vp[3] - 2 * vp[2]) +
+                       0.25 * (vp[1] - vp[3]) * (vp[1] - vp[3]);
+  const double beta2 = thirteen12th * (vp[0] + vp[2] - 2 * vp[1]) * (vp[0] + vp[2] - 2 * vp[1]) +
+                       0.25 * (vp[0] - 4 * vp[1] + 3 * vp[2]) * (vp[0] - 4 * vp[1] + 3 * vp[2]);
+  return weno5_side(v0, v1, v2, beta0, beta1, beta2, 0.3, 0.6, 0.1, eps);
+}
+
+DEV double weno5_right(const double *vm, double eps) {
+  constexpr double one6th = 1.0 / 6, thirteen12th = 13.0 / 12;
+  const double v0 = one6th * (11 * vm[2] - 7 * vm[3] + 2 * vm[4]);
+  const double v1 = one6th * (2 * vm[1] + 5 * vm[2] - vm[3]);
+  const double v2 = one6th * (-vm[0] + 5 * vm[1] + 2 * vm[2]);
+  const double beta0 = thirteen12th * (vm[2] + vm[4] - 2 * vm[3]) * (vm[2] + vm[4] - 2 * vm[3]) +
+                       0.25 * (3 * vm[2] - 4 * vm[3] + vm[4]) * (3 * vm[2] - 4 * vm[3] + vm[4]);
+  const double beta1 = thirteen12th * (vm[1] + vm[3] - 2 * vm[2]) * (vm[1] + vm[3] - 2 * vm[2]) +
+                       0.25 * (vm[1] - vm[3]) * (vm[1] - vm[3]);
+  const double beta2 = thirteen12th * (vm[0] + vm[2] - 2 * vm[1]) * (vm[0] + vm[2] - 2 * vm[1]) +
+                       0.25 * (vm[0] - 4 * vm[1] + 3 * vm[2]) * (vm[0] - 4 * vm[1] + 3 * vm[2]);
+  return weno5_side(v0, v1, v2, beta0, beta1, beta2, 0.1, 0.6, 0.3, eps);
+}
+
+DEV double weno5(const double *vp, const double *vm, double eps) {
+  constexpr double one6th = 1.0 / 6, thirteen12th = 13.0 / 12;
+  double v0 = one6th * (2 * vp[2] + 5 * vp[3] - vp[4]);
+  double v1 = one6th * (-vp[1] + 5 * vp[2] + 2 * vp[3]);
+  double v2 = one6th * (2 * vp[0] - 7 * vp[1] + 11 * vp[2]);
+  double beta0 = thirteen12th * (vp[2] + vp[4] - 2 * vp[3]) * (vp[2] + vp[4] - 2 * vp[3]) +
+                 0.25 * (3 * vp[2] - 4 * vp[3] + vp[4]) * (3 * vp[2] - 4 * vp[3] + vp[4]);
+  double beta1 = thirteen12th * (vp[1] + vp[3] - 2 * vp[2]) * (vp[1] + vp[3] - 2 * vp[2]) +
+                 0.25 * (vp[1] - vp[3]) * (vp[1] - vp[3]);
+  double beta2 = thirteen12th * (vp[0] + vp[2] - 2 * vp[1]) * (vp[0] + vp[2] - 2 * vp[1]) +
+                 0.25 * (vp[0] - 4 * vp[1] + 3 * vp[2]) * (vp[0] - 4 * vp[1] + 3 * vp[2]);
+  const double fPlus = weno5_side(v0, v1, v2, beta0, beta1, beta2, 0.3, 0.6, 0.1, eps);
+  v0 = one6th * (11 * vm[2] - 7 * vm[3] + 2 * vm[4]);
+  v1 = one6th * (2 * vm[1] + 5 * vm[2] - vm[3]);
+  v2 = one6th * (-vm[0] + 5 * vm[1] + 2 * vm[2]);
+  beta0 = thirteen12th * (vm[2] + vm[4] - 2 * vm[3]) * (vm[2] + vm[4] - 2 * vm[3]) +
+          0.25 * (3 * vm[2] - 4 * vm[3] + vm[4]) * (3 * vm[2] - 4 * vm[3] + vm[4]);
+  beta1 = thirteen12th * (vm[1] + vm[3] - 2 * vm[2]) * (vm[1] + vm[3] - 2 * vm[2]) +
+          0.25 * (vm[1] - vm[3]) * (vm[1] - vm[3]);
+  beta2 = thirteen12th * (vm[0] + vm[2] - 2 * vm[1]) * (vm[0] + vm[2] - 2 * vm[1]) +
+          0.25 * (vm[0] - 4 * vm[1] + 3 * vm[2]) * (vm[0] - 4 * vm[1] + 3 * vm[2]);
+  const double fMinus = weno5_side(v0, v1, v2, beta0, beta1, beta2, 0.1, 0.6, 0.3, eps);
+  return fPlus + fMinus;
+}
+
+DEV double w7beta(double s1, double s2, double s3) {
+  constexpr double d12 = 13.0 / 12.0, d13 = 1043.0 / 960, d14 = 1.0 / 12;
+  // s1^2 + d12 s2^2 + d13 s3^2 + d14 s1 s3
+  return fma(d13 * s3, s3, fma(d12 * s2, s2, s1 * fma(d14, s3, s1)));
+}
 
 // One half of WENO7-Z on the upwind-ordered values v[0..6] (v[3] is the
-// point left of the face), in the differences d_k = v_{k+1} - v_k, their
-// second differences D_k and third differences T_k.  A candidate stencil's
-// derivative estimates s1, s2, s3 (the reference's polynomials,
-// src/WENO.cu:3094-3117) are combinations of these, e.g. the left stencil's
-// s1 = (-2 v0 + 9 v1 - 18 v2 + 11 v3) / 6 is d2 + D1 / 2 + T0 / 3, and
-//   beta = s1^2 + 13/12 s2^2 + 1043/960 s3^2 + s1 s3 / 12
-//        = u^2 + 13/12 s2^2 + d13 s3^2,  u = s1 + s3 / 24,
-//          d13 = 1043/960 - 1/576 = 781/720,
-// while its face value is v3 + p / 2 with p = s1 + s2 / 6, so the flux is v3
-// plus half the weighted mean of the p.  eps joins the sums of squares as
-// they start (tau takes differences of the beta only).
-//
-// Bound by FP64 issue: 98 instructions against 113 with the candidate fluxes
-// formed from the values and the betas from their products s1 s3; two such
-// halves per row and face are 60% of a sweep's FP64 instructions (256x128x128,
-// nine species: x 1.21 -> 1.15 ms, y and z 1.27 -> 1.20 ms).  Its rounding
-// error against exact arithmetic is a third of that form's (largest over
-// smooth, stepped and random values: 1.1e-16 against 5.4e-16 of max |v|, and
-// 4.2e-16 against 5.4e-16 on noise).
-DEV double weno7_half(double v0, double v1, double v2, double v3, double v4, double v5, double v6, double eps) {
-  constexpr double third = 1.0 / 3, sixth = 1.0 / 6, d12 = 13.0 / 12, d13 = 781.0 / 720;
-  const double d0 = v1 - v0, d1 = v2 - v1, d2 = v3 - v2, d3 = v4 - v3, d4 = v5 - v4, d5 = v6 - v5;
-  const double D0 = d1 - d0, D1 = d2 - d1, D2 = d3 - d2, D3 = d4 - d3, D4 = d5 - d4;
+// point left of the face).  The three derivative estimates s1, s2, s3 of
+// each candidate stencil (the reference's polynomials, src/WENO.cu:3094-3117)
+// are formed from the shared differences d_k = v_{k+1} - v_k, their second
+// differences D_k and third differences T_k: e.g. the left stencil's
+// (-2 v0 + 9 v1 - 18 v2 + 11 v3) / 6 is d2 + D1 / 2 + T0 / 3.
+DEV double weno7_half(double v0_, double v1_, double v2_, double v3_, double v4_, double v5_, double v6_,
+                      double eps) {
+  constexpr double one12th = 1.0 / 12, third = 1.0 / 3, sixth = 1.0 / 6;
+  constexpr double c0 = 1.0 / 35, c1 = 12.0 / 35, c2 = 18.0 / 35, c3 = 4.0 / 35;
+  const double d2 = v3_ - v2_, d3 = v4_ - v3_;
+  const double D0 = fma(-2.0, v1_, v0_ + v2_), D1 = fma(-2.0, v2_, v1_ + v3_), D2 = fma(-2.0, v3_, v2_ + v4_),
+               D3 = fma(-2.0, v4_, v3_ + v5_), D4 = fma(-2.0, v5_, v4_ + v6_);
   const double T0 = D1 - D0, T1 = D2 - D1, T2 = D3 - D2, T3 = D4 - D3;
-  // u of the four stencils: s1's T coefficient 1/3, -1/6, -1/6, 1/3 plus 1/24
-  const double u0 = fma(0.375, T0, fma(0.5, D1, d2)), u1 = fma(-0.125, T1, fma(0.5, D2, d2));
-  const double u2 = fma(-0.125, T2, fma(-0.5, D2, d3)), u3 = fma(0.375, T3, fma(-0.5, D3, d3));
-  const double s20 = D1 + T0, s23 = D3 - T3;
-  const double mid = fma(d12 * D2, D2, eps);
-  const double e0 = fma(u0, u0, fma(d12 * s20, s20, fma(d13 * T0, T0, eps)));
-  const double e1 = fma(u1, u1, fma(d13 * T1, T1, mid));
-  const double e2 = fma(u2, u2, fma(d13 * T2, T2, mid));
-  const double e3 = fma(u3, u3, fma(d12 * s23, s23, fma(d13 * T3, T3, eps)));
-  double tau = fma(3.0, e1 - e2, e0 - e3);
+  const double beta0 = w7beta(fma(third, T0, fma(0.5, D1, d2)), D1 + T0, T0);
+  const double beta1 = w7beta(fma(-sixth, T1, fma(0.5, D2, d2)), D2, T1);
+  const double beta2 = w7beta(fma(-sixth, T2, fma(-0.5, D2, d3)), D2, T2);
+  const double beta3 = w7beta(fma(third, T3, fma(-0.5, D3, d3)), D3 - T3, T3);
+  double tau = beta0 + 3 * beta1 - 3 * beta2 - beta3;
   tau *= tau;
   // 1/(eps + beta_k) from one division of the product of the four terms
   // (each lies between eps >= 1e-40 (rho v)^2 and the square of the largest
   // characteristic flux, so the product stays inside the double range).
+  const double e0 = eps + beta0, e1 = eps + beta1, e2 = eps + beta2, e3 = eps + beta3;
   const double e01 = e0 * e1, e23 = e2 * e3;
   const double inv = fast_rcp(e01 * e23);
-  const double i01 = inv * e23, i23 = inv * e01;
-  const double r0 = i01 * e1, r1 = i01 * e0, r2 = i23 * e3, r3 = i23 * e2;
-  // the linear weights 1, 12, 18, 4 (over 35, which cancels in the mean)
-  const double a0 = fma(tau, r0 * r0, 1.0);
-  const double a1 = fma(12.0 * tau, r1 * r1, 12.0);
-  const double a2 = fma(18.0 * tau, r2 * r2, 18.0);
-  const double a3 = fma(4.0 * tau, r3 * r3, 4.0);
-  const double p0 = fma(0.5, T0, fma(2 * third, D1, d2)), p1 = fma(-sixth, T1, fma(2 * third, D2, d2));
-  const double p2 = fma(-sixth, T2, fma(-third, D2, d3)), p3 = fma(sixth, T3, fma(-third, D3, d3));
-  const double num = fma(a3, p3, fma(a2, p2, fma(a1, p1, a0 * p0)));
-  return fma(0.5 * num, fast_rcp((a0 + a1) + (a2 + a3)), v3);
+  const double r0 = inv * (e1 * e23), r1 = inv * (e0 * e23), r2 = inv * (e01 * e3), r3 = inv * (e01 * e2);
+  const double a0 = c0 + c0 * tau * (r0 * r0);
+  const double a1 = c1 + c1 * tau * (r1 * r1);
+  const double a2 = c2 + c2 * tau * (r2 * r2);
+  const double a3 = c3 + c3 * tau * (r3 * r3);
+  const double q0 = -3 * v0_ + 13 * v1_ - 23 * v2_ + 25 * v3_;
+  const double q1 = v1_ - 5 * v2_ + 13 * v3_ + 3 * v4_;
+  const double q2 = -v2_ + 7 * v3_ + 7 * v4_ - v5_;
+  const double q3 = 3 * v3_ + 13 * v4_ - 5 * v5_ + v6_;
+  return one12th * (a0 * q0 + a1 * q1 + a2 * q2 + a3 * q3) * fast_rcp(a0 + a1 + a2 + a3);
 }
 
 DEV double weno7(const double *vp, const double *vm, double eps) {

@@ -37,8 +37,8 @@ void emit_gibbs(std::ostringstream &o, const Tab &tb, int i) {
   auto g_expr = [&](const double *c, const char *t, const char *t2, const char *t3, const char *t4, const char *ti,
                     const char *lt) {
     std::ostringstream e;
-    e << lit(c[0]) << " * (1.0 - " << lt << ") - 0.5 * " << lit(c[1]) << " * " << t << " - " << lit(c[2]) << " * "
-      << t2 << " / 6.0 - " << lit(c[3]) << " * " << t3 << " / 12.0 - " << lit(c[4]) << " * " << t4 << " * 0.05 + "
+    e << lit(c[0]) << " * (1.0 - " << lt << ") - 0.5 * " << lit(c[1]) << " * " << t << " - div_by(" << lit(c[2])
+      << " * " << t2 << ", 6.0, 1.0 / 6) - div_by(" << lit(c[3]) << " * " << t3 << ", 12.0, 1.0 / 12) - " << lit(c[4]) << " * " << t4 << " * 0.05 + "
       << lit(c[5]) << " * " << ti << " - " << lit(c[6]);
     return e.str();
   };
@@ -149,8 +149,8 @@ void emit_rates(std::ostringstream &o, const Tab &tb, int ns) {
 void emit_h_cp(std::ostringstream &o, const Tab &tb, int ns) {
   auto h_expr = [&](const double *c, const char *t, const char *t2, const char *t3, const char *t4, const char *t5) {
     std::ostringstream e;
-    e << lit(c[0]) << " * " << t << " + 0.5 * " << lit(c[1]) << " * " << t2 << " + " << lit(c[2]) << " * " << t3
-      << " / 3 + 0.25 * " << lit(c[3]) << " * " << t4 << " + 0.2 * " << lit(c[4]) << " * " << t5 << " + "
+    e << lit(c[0]) << " * " << t << " + 0.5 * " << lit(c[1]) << " * " << t2 << " + div_by(" << lit(c[2])
+      << " * " << t3 << ", 3.0, 1.0 / 3) + 0.25 * " << lit(c[3]) << " * " << t4 << " + 0.2 * " << lit(c[4]) << " * " << t5 << " + "
       << lit(c[5]);
     return e.str();
   };
@@ -307,6 +307,9 @@ void emit_wu_kernel(std::ostringstream &o, const Tab &tb, int ns) {
 
 std::string generate(const Tab &tb, int ns) {
   std::ostringstream o;
+  // x / d for a constant d (y = 1 / d rounded), the IEEE quotient's bits (div_by in kernels.hip)
+  o << "__device__ __forceinline__ double div_by(double x, double d, double y) {\n"
+       "  const double q = x * y;\n  return fma(fma(-d, q, x), y, q);\n}\n\n";
   emit_rates(o, tb, ns);
   emit_h_cp(o, tb, ns);
   emit_chem_kernel(o, tb, ns);

@@ -133,6 +133,7 @@ struct Tab : corefl_chem_tables {
   double pw_lj[COREFL_MAX_SPEC];                    // LJ_potent_inv^-0.145
   double pw_kbe[COREFL_MAX_SPEC][COREFL_MAX_SPEC];  // 1.0548 kb_over_eps_jk^-0.15504
   double inv_bdc[COREFL_MAX_SPEC][COREFL_MAX_SPEC]; // 1 / binary_diffusivity_coeff
+  double rcp_imw[COREFL_MAX_SPEC], mol_conv[COREFL_MAX_SPEC];  // 1 / imw, 1e3 / imw
   Reac reac[COREFL_MAX_REAC];
 };
 void derive_tables(const corefl_chem_tables &in, Tab &out);

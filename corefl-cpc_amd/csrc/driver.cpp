@@ -735,6 +735,8 @@ void derive_tables(const corefl_chem_tables &in, Tab &out) {
   for (int l = 0; l < in.n_spec; ++l) {
     const double ln_lj = in.LJ_potent_inv[l] > 0 ? std::log(in.LJ_potent_inv[l]) : 0.0;
     out.pw_lj[l] = std::exp(-0.145 * ln_lj);
+    out.rcp_imw[l] = 1.0 / in.imw[l];
+    out.mol_conv[l] = 1e+3 / in.imw[l];
     for (int k = 0; k < in.n_spec; ++k) {
       const double ln_kbe = in.kb_over_eps_jk[l][k] > 0 ? std::log(in.kb_over_eps_jk[l][k]) : 0.0;
       out.pw_kbe[l][k] = 1.0548 * std::exp(-0.15504 * ln_kbe);

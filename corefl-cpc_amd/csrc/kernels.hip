@@ -44,34 +44,63 @@ constexpr int kNv(int m) { return 5 + kNsc(m); }                  // n_var
 
 DEV double norm3(double a, double b, double c) { return sqrt(a * a + b * b + c * c); }
 
+// x / d for a constant d, correctly rounded: one multiplication by the rounded
+// 1/d and one exact-remainder correction (P. Markstein, Computation of
+// elementary functions on the IBM RISC System/6000 processor, 1990) give the
+// IEEE quotient's bits in 3 instructions instead of a division's eleven, for
+// normal x whose quotient is normal.
+template <int D>
+DEV double div_by(double x) {
+  constexpr double d = D, y = 1.0 / D;
+  const double q = x * y;
+  return fma(fma(-d, q, x), y, q);
+}
+
 // ---------------------------------------------------------------------------
 // NASA-7 thermodynamics (two ranges, linear extrapolation outside), the
 // Combustion2Part branch of src/Thermo.cu:386-631.
 // ---------------------------------------------------------------------------
 DEV double nasa_h(const double *c, double t, double t2, double t3, double t4, double t5) {
-  return c[0] * t + 0.5 * c[1] * t2 + c[2] * t3 / 3 + 0.25 * c[3] * t4 + 0.2 * c[4] * t5 + c[5];
+  return c[0] * t + 0.5 * c[1] * t2 + div_by<3>(c[2] * t3) + 0.25 * c[3] * t4 + 0.2 * c[4] * t5 + c[5];
 }
 DEV double nasa_cp(const double *c, double t, double t2, double t3, double t4) {
   return c[0] + c[1] * t + c[2] * t2 + c[3] * t3 + c[4] * t4;
+}
+DEV double nasa_g(const double *c, double t, double t2, double t3, double t4, double t_inv, double log_t) {
+  return c[0] * (1.0 - log_t) - 0.5 * c[1] * t - div_by<6>(c[2] * t2) - div_by<12>(c[3] * t3) - c[4] * t4 * 0.05 +
+         c[5] * t_inv - c[6];
 }
 
 // NASA-9 (src/Thermo.cu:426-456, 501-521, 573-596, 628-653): the range of
 // species i at t is the first j with t_cut[j] <= t <= t_cut[j+1]; outside
 // [t_cut[0], t_cut[n]] the enthalpy is extrapolated linearly with the bound's
 // cp, cp is held and G/RT is taken at the bound.  Values are per unit R_i.
-DEV double nasa9_h_at(const double *c, double tt) {
-  const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt5 = tt4 * tt, itt = 1.0 / tt;
-  return -c[0] * itt + c[1] * log(tt) + c[2] * tt + 0.5 * c[3] * tt2 + c[4] * tt3 / 3 + 0.25 * c[5] * tt4 +
-         0.2 * c[6] * tt5 + c[7];
+// The terms in T that every species shares, formed once per temperature.
+struct Nasa9T {
+  double t, t2, t3, t4, t5, it, it2, ln_t;
+};
+DEV Nasa9T nasa9_terms(double t) {
+  Nasa9T T;
+  T.t = t;
+  T.t2 = t * t;
+  T.t3 = T.t2 * t;
+  T.t4 = T.t3 * t;
+  T.t5 = T.t4 * t;
+  T.it = 1.0 / t;
+  T.it2 = T.it * T.it;
+  T.ln_t = log(t);
+  return T;
 }
-DEV double nasa9_cp_at(const double *c, double tt) {
-  const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, itt2 = 1.0 / tt2, itt = 1.0 / tt;
-  return c[0] * itt2 + c[1] * itt + c[2] + c[3] * tt + c[4] * tt2 + c[5] * tt3 + c[6] * tt4;
+DEV double nasa9_h_at(const double *c, const Nasa9T &T) {
+  return -c[0] * T.it + c[1] * T.ln_t + c[2] * T.t + 0.5 * c[3] * T.t2 + div_by<3>(c[4] * T.t3) + 0.25 * c[5] * T.t4 +
+         0.2 * c[6] * T.t5 + c[7];
 }
-DEV double nasa9_g_at(const double *c, double tt) {
-  const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, itt = 1 / tt, lntt = log(tt), itt2 = itt * itt;
-  return -0.5 * c[0] * itt2 + c[1] * itt * (lntt + 1) + c[2] * (1.0 - lntt) - 0.5 * c[3] * tt - c[4] * tt2 / 6.0 -
-         c[5] * tt3 / 12.0 - c[6] * tt4 * 0.05 + c[7] * itt - c[8];
+DEV double nasa9_cp_at(const double *c, const Nasa9T &T) {
+  return c[0] * T.it2 + c[1] * T.it + c[2] + c[3] * T.t + c[4] * T.t2 + c[5] * T.t3 + c[6] * T.t4;
+}
+DEV double nasa9_g_at(const double *c, const Nasa9T &T) {
+  return -0.5 * c[0] * T.it2 + c[1] * T.it * (T.ln_t + 1) + c[2] * (1.0 - T.ln_t) - 0.5 * c[3] * T.t -
+         div_by<6>(c[4] * T.t2) - div_by<12>(c[5] * T.t3) - c[6] * T.t4 * 0.05 + c[7] * T.it - c[8];
 }
 // range index inside [t_cut[0], t_cut[n]] (the interior cuts below t)
 DEV int nasa9_range(const Tab *__restrict__ tb, int i, double t) {
@@ -83,28 +112,28 @@ DEV int nasa9_range(const Tab *__restrict__ tb, int i, double t) {
 }
 // h_i / R_i and cp_i / R_i (either may be skipped)
 template <bool WANT_H, bool WANT_CP>
-DEV void nasa9_h_cp(const Tab *__restrict__ tb, int i, double t, double &h, double &cp) {
+DEV void nasa9_h_cp(const Tab *__restrict__ tb, int i, const Nasa9T &T, double &h, double &cp) {
   const int n = tb->n_range[i];
-  const double lo = tb->t_cut[i][0], hi = tb->t_cut[i][n];
+  const double t = T.t, lo = tb->t_cut[i][0], hi = tb->t_cut[i][n];
   if (t < lo || t > hi) {
-    const double tt = t < lo ? lo : hi;
+    const Nasa9T B = nasa9_terms(t < lo ? lo : hi);
     const double *c = tb->poly9[i][t < lo ? 0 : n - 1];
-    const double cb = nasa9_cp_at(c, tt);
-    if (WANT_H) h = nasa9_h_at(c, tt) + cb * (t - tt);
+    const double cb = nasa9_cp_at(c, B);
+    if (WANT_H) h = nasa9_h_at(c, B) + cb * (t - B.t);
     if (WANT_CP) cp = cb;
   } else {
     const double *c = tb->poly9[i][nasa9_range(tb, i, t)];
-    const double t2 = t * t, t3 = t2 * t, t4 = t3 * t, it = 1.0 / t;
-    if (WANT_H) {
-      const double t5 = t4 * t, lnT = log(t);
-      h = -c[0] * it + c[1] * lnT + c[2] * t + 0.5 * c[3] * t2 + c[4] * t3 / 3 + 0.25 * c[5] * t4 +
-          0.2 * c[6] * t5 + c[7];
-    }
-    if (WANT_CP) {
-      const double it2 = it * it;
-      cp = c[0] * it2 + c[1] * it + c[2] + c[3] * t + c[4] * t2 + c[5] * t3 + c[6] * t4;
-    }
+    if (WANT_H) h = nasa9_h_at(c, T);
+    if (WANT_CP) cp = nasa9_cp_at(c, T);
   }
+}
+
+// G/RT of species i (the bound's value outside the ranges)
+DEV double nasa9_g1(const Tab *__restrict__ tb, int i, const Nasa9T &T) {
+  const int n = tb->n_range[i];
+  const double lo = tb->t_cut[i][0], hi = tb->t_cut[i][n];
+  if (T.t < lo || T.t > hi) return nasa9_g_at(tb->poly9[i][T.t < lo ? 0 : n - 1], nasa9_terms(T.t < lo ? lo : hi));
+  return nasa9_g_at(tb->poly9[i][nasa9_range(tb, i, T.t)], T);
 }
 
 template <int M>
@@ -112,9 +141,10 @@ DEV void thermo_h(const Tab *__restrict__ tb, double t, double *h) {
   [[maybe_unused]] constexpr int NS = kNs(M);
   if constexpr (kNasa9(M)) {
     double cp;
+    const Nasa9T T = nasa9_terms(t);
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
-      nasa9_h_cp<true, false>(tb, i, t, h[i], cp);
+      nasa9_h_cp<true, false>(tb, i, T, h[i], cp);
       h[i] *= tb->gas_const[i];
     }
     return;
@@ -146,9 +176,10 @@ DEV void thermo_cp(const Tab *__restrict__ tb, double t, double *cp) {
   [[maybe_unused]] constexpr int NS = kNs(M);
   if constexpr (kNasa9(M)) {
     double h;
+    const Nasa9T T = nasa9_terms(t);
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
-      nasa9_h_cp<false, true>(tb, i, t, h, cp[i]);
+      nasa9_h_cp<false, true>(tb, i, T, h, cp[i]);
       cp[i] *= tb->gas_const[i];
     }
     return;
@@ -178,9 +209,10 @@ template <int M>
 DEV void thermo_h_cp(const Tab *__restrict__ tb, double t, double *h, double *cp) {
   [[maybe_unused]] constexpr int NS = kNs(M);
   if constexpr (kNasa9(M)) {
+    const Nasa9T T = nasa9_terms(t);
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
-      nasa9_h_cp<true, true>(tb, i, t, h[i], cp[i]);
+      nasa9_h_cp<true, true>(tb, i, T, h[i], cp[i]);
       h[i] *= tb->gas_const[i];
       cp[i] *= tb->gas_const[i];
     }
@@ -216,7 +248,7 @@ template <int M>
 DEV double thermo_h1(const Tab *__restrict__ tb, int i, double t, double t2, double t3, double t4, double t5) {
   if constexpr (kNasa9(M)) {
     double h, cp;
-    nasa9_h_cp<true, false>(tb, i, t, h, cp);
+    nasa9_h_cp<true, false>(tb, i, nasa9_terms(t), h, cp);
     return h * tb->gas_const[i];
   }
   const double tl = tb->t_low[i], th = tb->t_high[i];
@@ -242,15 +274,9 @@ template <int M>
 DEV void thermo_gibbs(const Tab *__restrict__ tb, double t, double *g) {
   [[maybe_unused]] constexpr int NS = kNs(M);
   if constexpr (kNasa9(M)) {
+    const Nasa9T T = nasa9_terms(t);
 #pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      const int n = tb->n_range[i];
-      const double lo = tb->t_cut[i][0], hi = tb->t_cut[i][n];
-      if (t < lo || t > hi)
-        g[i] = nasa9_g_at(tb->poly9[i][t < lo ? 0 : n - 1], t < lo ? lo : hi);
-      else
-        g[i] = nasa9_g_at(tb->poly9[i][nasa9_range(tb, i, t)], t);
-    }
+    for (int i = 0; i < NS; ++i) g[i] = nasa9_g1(tb, i, T);
     return;
   }
   const double t2 = t * t, t3 = t2 * t, t4 = t3 * t, t_inv = 1 / t, log_t = log(t);
@@ -261,15 +287,13 @@ DEV void thermo_gibbs(const Tab *__restrict__ tb, double t, double *g) {
       const double tt = t < tl ? tl : th;
       const double *c = t < tl ? tb->low_coeff[i] : tb->high_coeff[i];
       const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt_inv = 1 / tt, log_tt = log(tt);
-      g[i] = c[0] * (1.0 - log_tt) - 0.5 * c[1] * tt - c[2] * tt2 / 6.0 - c[3] * tt3 / 12.0 - c[4] * tt4 * 0.05 +
-             c[5] * tt_inv - c[6];
+      g[i] = nasa_g(c, tt, tt2, tt3, tt4, tt_inv, log_tt);
     } else {
       const bool lo = t < tb->t_mid[i];
       double c[7];
 #pragma unroll
       for (int k = 0; k < 7; ++k) c[k] = lo ? tb->low_coeff[i][k] : tb->high_coeff[i][k];
-      g[i] = c[0] * (1.0 - log_t) - 0.5 * c[1] * t - c[2] * t2 / 6.0 - c[3] * t3 / 12.0 - c[4] * t4 * 0.05 +
-             c[5] * t_inv - c[6];
+      g[i] = nasa_g(c, t, t2, t3, t4, t_inv, log_t);
     }
   }
 }
@@ -715,7 +739,7 @@ DEV void transport(const Tab *__restrict__ tb, double temperature, double mw_tot
     double s = 0;
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      const double tmp = (X[l] + eps) * (1.0 / tb->imw[l]);
+      const double tmp = (X[l] + eps) * tb->rcp_imw[l];
       num[l] = tmp;
       s += tmp;
       den[l] = 0;
@@ -1028,10 +1052,7 @@ DEV double reaction_temperature(double t, double tve, double a, double b) {
 template <int M>
 DEV double gibbs1(const Tab *__restrict__ tb, int i, double t) {
   if constexpr (kNasa9(M)) {
-    const int n = tb->n_range[i];
-    const double lo = tb->t_cut[i][0], hi = tb->t_cut[i][n];
-    if (t < lo || t > hi) return nasa9_g_at(tb->poly9[i][t < lo ? 0 : n - 1], t < lo ? lo : hi);
-    return nasa9_g_at(tb->poly9[i][nasa9_range(tb, i, t)], t);
+    return nasa9_g1(tb, i, nasa9_terms(t));
   } else {
     const double tl = tb->t_low[i], th = tb->t_high[i];
     const bool out = t < tl || t > th;
@@ -1039,8 +1060,7 @@ DEV double gibbs1(const Tab *__restrict__ tb, int i, double t) {
     const double *c = out ? (t < tl ? tb->low_coeff[i] : tb->high_coeff[i])
                           : (t < tb->t_mid[i] ? tb->low_coeff[i] : tb->high_coeff[i]);
     const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt_inv = 1 / tt, log_tt = log(tt);
-    return c[0] * (1.0 - log_tt) - 0.5 * c[1] * tt - c[2] * tt2 / 6.0 - c[3] * tt3 / 12.0 - c[4] * tt4 * 0.05 +
-           c[5] * tt_inv - c[6];
+    return nasa_g(c, tt, tt2, tt3, tt4, tt_inv, log_tt);
   }
 }
 
@@ -1255,7 +1275,7 @@ __global__ __launch_bounds__(kBlock) void k_chemistry(Zone z, const Tab *__restr
   double time_scale = 1e+6;
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
-    const double conv = 1e+3 / tb->imw[l];
+    const double conv = tb->mol_conv[l];
     const double cr = creation[l] * conv;
     const double od = omega_d[l] * conv;
     const double om = cr - od;
@@ -1269,7 +1289,7 @@ __global__ __launch_bounds__(kBlock) void k_chemistry(Zone z, const Tab *__restr
     double src = 0.0;
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      const double conv = 1e+3 / tb->imw[l];
+      const double conv = tb->mol_conv[l];
       src += (creation[l] * conv - omega_d[l] * conv) * ve_energy1<false>(tb, l, tv, nullptr);
     }
     z.dq[t + (5 + NS) * dsz] += jac * src;
@@ -1320,7 +1340,7 @@ DEV void reactor_source(const Tab *__restrict__ tb, double rho, double t, const 
     chem_rates<M, false>(tb, rho, t, t, yk, cr, od, nullptr);
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
-    const double conv = 1e+3 / tb->imw[l];
+    const double conv = tb->mol_conv[l];
     omega[l] = cr[l] * conv - od[l] * conv;
   }
 }
@@ -1629,7 +1649,7 @@ constexpr int kWave = 64;
 template <int M>
 DEV void thermo_h_cp1(const Tab *__restrict__ tb, int i, double t, double &h, double &cp) {
   if constexpr (kNasa9(M)) {
-    nasa9_h_cp<true, true>(tb, i, t, h, cp);
+    nasa9_h_cp<true, true>(tb, i, nasa9_terms(t), h, cp);
     h *= tb->gas_const[i];
     cp *= tb->gas_const[i];
   } else {
@@ -1743,7 +1763,7 @@ DEV void wave_source(const Tab *__restrict__ tb, ReactorWaveLds<M> &L, double rh
   __syncthreads();
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
-    const double conv = 1e+3 / tb->imw[l];
+    const double conv = tb->mol_conv[l];
     omega[l] = L.cr[l] * conv - L.od[l] * conv;
   }
 }
@@ -3596,9 +3616,9 @@ __global__ __launch_bounds__(kBlock) void k_viscous_flux(Zone z, const Tab *__re
   const double w_y = w_xi * xi_y + w_eta * eta_y + w_zeta * zeta_y;
   const double w_z = w_xi * xi_z + w_eta * eta_z + w_zeta * zeta_z;
   const double mul = z.mul[p];
-  const double tau_xx = mul * (4 * u_x - 2 * v_y - 2 * w_z) / 3.0;
-  const double tau_yy = mul * (4 * v_y - 2 * u_x - 2 * w_z) / 3.0;
-  const double tau_zz = mul * (4 * w_z - 2 * u_x - 2 * v_y) / 3.0;
+  const double tau_xx = div_by<3>(mul * (4 * u_x - 2 * v_y - 2 * w_z));
+  const double tau_yy = div_by<3>(mul * (4 * v_y - 2 * u_x - 2 * w_z));
+  const double tau_zz = div_by<3>(mul * (4 * w_z - 2 * u_x - 2 * v_y));
   const double tau_xy = mul * (u_y + v_x);
   const double tau_xz = mul * (u_z + w_x);
   const double tau_yz = mul * (v_z + w_y);
@@ -3849,9 +3869,9 @@ __global__ __launch_bounds__(kBlock) void k_visc2_flux(Zone z, const Tab *__rest
   grad(pv, 3, w_x, w_y, w_z);
   grad(pv, 5, t_x, t_y, t_z);
   const double mul = 0.5 * (z.mul[p] + z.mul[pe]);
-  const double tau_xx = mul * (4 * u_x - 2 * v_y - 2 * w_z) / 3.0;
-  const double tau_yy = mul * (4 * v_y - 2 * u_x - 2 * w_z) / 3.0;
-  const double tau_zz = mul * (4 * w_z - 2 * u_x - 2 * v_y) / 3.0;
+  const double tau_xx = div_by<3>(mul * (4 * u_x - 2 * v_y - 2 * w_z));
+  const double tau_yy = div_by<3>(mul * (4 * v_y - 2 * u_x - 2 * w_z));
+  const double tau_zz = div_by<3>(mul * (4 * w_z - 2 * u_x - 2 * v_y));
   const double tau_xy = mul * (u_y + v_x), tau_xz = mul * (u_z + w_x), tau_yz = mul * (v_z + w_y);
   const double kx = 0.5 * (mt[p + (3 * DIR) * sz] * z.jac[p] + mt[pe + (3 * DIR) * sz] * z.jac[pe]);
   const double ky = 0.5 * (mt[p + (3 * DIR + 1) * sz] * z.jac[p] + mt[pe + (3 * DIR + 1) * sz] * z.jac[pe]);
@@ -5683,7 +5703,7 @@ DEV void wu_substep(const Tab *__restrict__ tb, double *cv, const double *cn, do
       double ts = 1e+6;
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
-        const double conv = 1e+3 / tb->imw[l];
+        const double conv = tb->mol_conv[l];
         const double odl = od[l] * conv, om = cr[l] * conv - odl;
         if (cv[5 + l] > 1e-25 && fabs(odl) > 1e-25) ts = fmin(ts, fabs(cv[5 + l] / odl));
         cv[5 + l] = a * qn[5 + l] + b * cv[5 + l] + c * h * (om + cn[5 + l] * iJac);
@@ -5699,14 +5719,14 @@ DEV void wu_substep(const Tab *__restrict__ tb, double *cv, const double *cn, do
     chem_rates<M, true>(tb, 1.0, T, T, cv + 5, cr, od, zz);
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      const double conv = 1e+3 / tb->imw[l];
+      const double conv = tb->mol_conv[l];
       om[l] = cr[l] * conv - od[l] * conv;
     }
     // (I - h J) x = omega, J[m][n] = 1e3 / imw_m * zz[m][n] / (rho Y_n) where rho Y_n > 1e-25
     // (rho Y_n as the reference forms it back from the concentration)
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
-      const double ry = cv[5 + n] * tb->imw[n] * 1e-3 * (1e+3 / tb->imw[n]);
+      const double ry = cv[5 + n] * tb->imw[n] * 1e-3 * tb->mol_conv[n];
 #pragma unroll
       for (int m = 0; m < NS; ++m) {
         double jmn = 0;
@@ -5721,7 +5741,7 @@ DEV void wu_substep(const Tab *__restrict__ tb, double *cv, const double *cn, do
     chem_rates<M, false>(tb, 1.0, T, T, cv + 5, cr, od, nullptr);
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      const double conv = 1e+3 / tb->imw[l];
+      const double conv = tb->mol_conv[l];
       om[l] = cr[l] * conv - od[l] * conv;
     }
   }
@@ -5730,7 +5750,7 @@ DEV void wu_substep(const Tab *__restrict__ tb, double *cv, const double *cn, do
   double ts = 1e+6;
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
-    const double odl = od[l] * (1e+3 / tb->imw[l]);
+    const double odl = od[l] * tb->mol_conv[l];
     if (cv[5 + l] > 1e-25 && fabs(odl) > 1e-25) ts = fmin(ts, fabs(cv[5 + l] / odl));
     cv[5 + l] += (om[l] + cn[5 + l] * iJac) * h;
   }

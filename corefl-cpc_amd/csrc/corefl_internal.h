@@ -199,10 +199,11 @@ constexpr int kWenoShapes = 2;
 hipError_t launch_inviscid(const Zone &z, const Run &r, const Tab *tb, int dir, hipStream_t s, int shape = 0);
 hipError_t launch_shock_sensor(const Zone &z, const Run &r, hipStream_t s);
 hipError_t launch_reactors(const ReactorPool &p, int model, const Tab *tb, int max_steps, hipStream_t s);
-// the same step with one wave per slot, over slots [0, n_slots); the servers take it while at most
-// kReactorWaveSlots slots are in flight (one lane per slot is the faster choice beyond: a wave per slot
-// costs about 18 times the SIMD time of a lane per slot, and wins only while lanes would idle)
-constexpr int kReactorWaveSlots = 2048;
+// the same step with one wave per slot, over slots [0, n_slots).  The servers take it while at most
+// kReactorWaveSlots slots are in flight: a wave per slot steps about 80 reactors a microsecond once the
+// GPU is full, a lane per slot takes 212 us a step however few of its lanes are used (up to 65,536), so
+// the lines cross near 16,000 slots (5000: 58 us against 212).
+constexpr int kReactorWaveSlots = 16384;
 hipError_t launch_reactors_wave(const ReactorPool &p, int model, const Tab *tb, int max_steps, int n_slots,
                                 hipStream_t s);
 hipError_t launch_reactor_admit(const ReactorPool &p, int model, const Tab *tb, const double *req, int n_req,

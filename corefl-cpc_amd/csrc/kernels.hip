@@ -56,19 +56,30 @@ DEV double div_by(double x) {
   return fma(fma(-d, q, x), y, q);
 }
 
+// a x + b y and a x + b y + c z with the fused operations written out: where two
+// products meet, which one the compiler fuses depends on the code around them,
+// and the two reactor kernels have to agree in every bit.
+DEV double dot2(double a, double x, double b, double y) {
+#pragma clang fp contract(off)
+  const double p = b * y;
+  return fma(a, x, p);
+}
+DEV double dot3(double a, double x, double b, double y, double c, double z) { return fma(c, z, dot2(a, x, b, y)); }
+
 // ---------------------------------------------------------------------------
 // NASA-7 thermodynamics (two ranges, linear extrapolation outside), the
 // Combustion2Part branch of src/Thermo.cu:386-631.
 // ---------------------------------------------------------------------------
 DEV double nasa_h(const double *c, double t, double t2, double t3, double t4, double t5) {
-  return c[0] * t + 0.5 * c[1] * t2 + div_by<3>(c[2] * t3) + 0.25 * c[3] * t4 + 0.2 * c[4] * t5 + c[5];
+  const double a = dot2(c[0], t, 0.5 * c[1], t2) + div_by<3>(c[2] * t3);
+  return fma(0.2 * c[4], t5, fma(0.25 * c[3], t4, a)) + c[5];
 }
 DEV double nasa_cp(const double *c, double t, double t2, double t3, double t4) {
-  return c[0] + c[1] * t + c[2] * t2 + c[3] * t3 + c[4] * t4;
+  return fma(c[4], t4, fma(c[3], t3, fma(c[2], t2, fma(c[1], t, c[0]))));
 }
 DEV double nasa_g(const double *c, double t, double t2, double t3, double t4, double t_inv, double log_t) {
-  return c[0] * (1.0 - log_t) - 0.5 * c[1] * t - div_by<6>(c[2] * t2) - div_by<12>(c[3] * t3) - c[4] * t4 * 0.05 +
-         c[5] * t_inv - c[6];
+  const double a = dot2(c[0], 1.0 - log_t, -(0.5 * c[1]), t) - div_by<6>(c[2] * t2) - div_by<12>(c[3] * t3);
+  return fma(c[5], t_inv, fma(-(c[4] * t4), 0.05, a)) - c[6];
 }
 
 // NASA-9 (src/Thermo.cu:426-456, 501-521, 573-596, 628-653): the range of
@@ -159,7 +170,7 @@ DEV void thermo_h(const Tab *__restrict__ tb, double t, double *h) {
       const double *c = t < tl ? tb->low_coeff[i] : tb->high_coeff[i];
       const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt5 = tt4 * tt;
       v = nasa_h(c, tt, tt2, tt3, tt4, tt5);
-      v += nasa_cp(c, tt, tt2, tt3, tt4) * (t - tt);
+      v = fma(nasa_cp(c, tt, tt2, tt3, tt4), t - tt, v);
     } else {
       const bool lo = t < tb->t_mid[i];
       double c[6];
@@ -229,7 +240,7 @@ DEV void thermo_h_cp(const Tab *__restrict__ tb, double t, double *h, double *cp
       const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt5 = tt4 * tt;
       vh = nasa_h(c, tt, tt2, tt3, tt4, tt5);
       vc = nasa_cp(c, tt, tt2, tt3, tt4);
-      vh += vc * (t - tt);
+      vh = fma(vc, t - tt, vh);
     } else {
       const bool lo = t < tb->t_mid[i];
       double c[6];
@@ -258,7 +269,7 @@ DEV double thermo_h1(const Tab *__restrict__ tb, int i, double t, double t2, dou
     const double *c = t < tl ? tb->low_coeff[i] : tb->high_coeff[i];
     const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt5 = tt4 * tt;
     v = nasa_h(c, tt, tt2, tt3, tt4, tt5);
-    v += nasa_cp(c, tt, tt2, tt3, tt4) * (t - tt);
+    v = fma(nasa_cp(c, tt, tt2, tt3, tt4), t - tt, v);
   } else {
     const bool lo = t < tb->t_mid[i];
     double c[6];
@@ -1066,14 +1077,16 @@ DEV double gibbs1(const Tab *__restrict__ tb, int i, double t) {
 
 DEV double ipow(double c, int e) {
   if (e == 0) return 1.0;
-  if (e == 1) return c;
-  if (e == 2) return c * c;
-  return pow(c, static_cast<double>(e));
+  double p = c;
+  for (int k = 1; k < e; ++k) p *= c;
+  return p;
 }
 
 // Arrhenius A T^b exp(-Ea/T) as one exponential of b log T - Ea/T.
 DEV double arrhenius_ln(double ln_t, double inv_t, double A, double b, double Ea) {
-  return A * exp(b * ln_t - Ea * inv_t);
+#pragma clang fp contract(off)
+  const double e = exp(dot2(b, ln_t, -Ea, inv_t));
+  return A * e;
 }
 
 // Forward and backward rates of progress q1, q2 of reaction r at T (and Tve
@@ -1108,7 +1121,7 @@ DEV void reaction_progress(const Tab *__restrict__ tb, int r, double T, double t
   } else if (type > 3) {
     double cc = 0;
 #pragma unroll
-    for (int l = 0; l < NS; ++l) cc += c[l] * tb->third_body[r][l];
+    for (int l = 0; l < NS; ++l) cc = fma(c[l], tb->third_body[r][l], cc);
     if (type == 4) {
       kf *= cc;
     } else {
@@ -1121,15 +1134,15 @@ DEV void reaction_progress(const Tab *__restrict__ tb, int r, double T, double t
         const double reduced_pressure = kf_low * cc / kf_high;
         double F = 1.0;
         if (type > 5) {
-          double f_cent = (1 - tb->troe_alpha[r]) * exp(-thf / tb->troe_t3[r]) +
-                          tb->troe_alpha[r] * exp(-thf / tb->troe_t1[r]);
+          double f_cent = dot2(1 - tb->troe_alpha[r], exp(-thf / tb->troe_t3[r]), tb->troe_alpha[r],
+                               exp(-thf / tb->troe_t1[r]));
           if (type == 7) f_cent += exp(-tb->troe_t2[r] * it);
           const double logFc = log(f_cent) * kInvLn10;
-          const double cT = -0.4 - 0.67 * logFc;
-          const double nn = 0.75 - 1.27 * logFc;
-          const double logPr = log(reduced_pressure) * kInvLn10;
-          const double tempo = (logPr + cT) / (nn - 0.14 * (logPr + cT));
-          F = exp(kLn10 * (logFc / (1.0 + tempo * tempo)));
+          const double cT = fma(-0.67, logFc, -0.4);
+          const double nn = fma(-1.27, logFc, 0.75);
+          const double lp = fma(log(reduced_pressure), kInvLn10, cT);  // log10 Pr + c
+          const double tempo = lp / fma(-0.14, lp, nn);
+          F = exp(kLn10 * (logFc / fma(tempo, tempo, 1.0)));
         }
         kf = kf_high * reduced_pressure / (1.0 + reduced_pressure) * F;
       }
@@ -1149,7 +1162,7 @@ DEV void reaction_progress(const Tab *__restrict__ tb, int r, double T, double t
       if (type == 4) {
         double cc = 0;
 #pragma unroll
-        for (int l = 0; l < NS; ++l) cc += c[l] * tb->third_body[r][l];
+        for (int l = 0; l < NS; ++l) cc = fma(c[l], tb->third_body[r][l], cc);
         kb *= cc;
       }
     } else {
@@ -1163,7 +1176,7 @@ DEV void reaction_progress(const Tab *__restrict__ tb, int r, double T, double t
       if (type == 4) {
         double cc = 0;
 #pragma unroll
-        for (int l = 0; l < NS; ++l) cc += c[l] * tb->third_body[r][l];
+        for (int l = 0; l < NS; ++l) cc = fma(c[l], tb->third_body[r][l], cc);
         kb *= cc;
       }
     }
@@ -1174,9 +1187,9 @@ DEV void reaction_progress(const Tab *__restrict__ tb, int r, double T, double t
       double d_gibbs = 0;
 #pragma unroll
       for (int l = 0; l < NS; ++l)
-        if (sb[l] != sf[l]) d_gibbs += g[l] * static_cast<double>(sb[l] - sf[l]);
+        if (sb[l] != sf[l]) d_gibbs = fma(g[l], static_cast<double>(sb[l] - sf[l]), d_gibbs);
       // kb = kf / Kc with Kc = (p_atm / R_u T)^order exp(-dG/RT)
-      kb = kf * exp(d_gibbs - static_cast<double>(tb->order[r]) * ln_temp_t);
+      kb = kf * exp(fma(-static_cast<double>(tb->order[r]), ln_temp_t, d_gibbs));
     }
   }
   // rate of progress, src/FiniteRateChem.cu:1638-1663 (reactants and products in index order)
@@ -1243,13 +1256,15 @@ DEV void chem_rates(const Tab *__restrict__ tb, double density, double T, double
     for (int l = 0; l < NS; ++l) {
       if (sfi[l] == 0 && sbi[l] == 0) continue;
       const double sf = sfi[l], sb = sbi[l];
-      creation[l] += q2 * sf + q1 * sb;
-      omega_d[l] += q1 * sf + q2 * sb;
+      creation[l] += dot2(q2, sf, q1, sb);
+      omega_d[l] += dot2(q1, sf, q2, sb);
       if constexpr (JAC) {
 #pragma unroll
         for (int l2 = 0; l2 < NS; ++l2) {
           if (sfi[l2] == 0 && sbi[l2] == 0) continue;
-          zz[(l * NS + l2) * ZST] += (sb - sf) * (static_cast<double>(sfi[l2]) * q1 - static_cast<double>(sbi[l2]) * q2);
+          zz[(l * NS + l2) * ZST] =
+              fma(sb - sf, dot2(static_cast<double>(sfi[l2]), q1, -static_cast<double>(sbi[l2]), q2),
+                  zz[(l * NS + l2) * ZST]);
         }
       }
     }
@@ -1318,10 +1333,10 @@ DEV double reactor_temperature(const Tab *__restrict__ tb, double t0, double imw
     double cp_tot = 0, hm = 0;
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      cp_tot += cp[l] * yk[l];
-      hm += h[l] * yk[l];
+      cp_tot = fma(cp[l], yk[l], cp_tot);
+      hm = fma(h[l], yk[l], hm);
     }
-    const double t1 = t - (hm - r * t - e) / (cp_tot - r);
+    const double t1 = t - (fma(-r, t, hm) - e) / (cp_tot - r);
     err = fabs(1 - t1 / t);
     t = t1;
   }
@@ -1341,7 +1356,7 @@ DEV void reactor_source(const Tab *__restrict__ tb, double rho, double t, const 
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
     const double conv = tb->mol_conv[l];
-    omega[l] = cr[l] * conv - od[l] * conv;
+    omega[l] = dot2(cr[l], conv, -od[l], conv);
   }
 }
 
@@ -1356,7 +1371,8 @@ DEV void lu_factor(double *a, int *ipiv) {
 #pragma unroll
     for (int m = n; m < NS; ++m)
 #pragma unroll
-      for (int t = 0; t < n; ++t) a[(m * NS + n) * ST] -= a[(m * NS + t) * ST] * a[(t * NS + n) * ST];
+      for (int t = 0; t < n; ++t)
+        a[(m * NS + n) * ST] = fma(-a[(m * NS + t) * ST], a[(t * NS + n) * ST], a[(m * NS + n) * ST]);
     int ik = n;
     double best = fabs(a[(n * NS + n) * ST]);
 #pragma unroll
@@ -1381,7 +1397,8 @@ DEV void lu_factor(double *a, int *ipiv) {
 #pragma unroll
     for (int q = n + 1; q < NS; ++q)
 #pragma unroll
-      for (int t = 0; t < n; ++t) a[(n * NS + q) * ST] -= a[(n * NS + t) * ST] * a[(t * NS + q) * ST];
+      for (int t = 0; t < n; ++t)
+        a[(n * NS + q) * ST] = fma(-a[(n * NS + t) * ST], a[(t * NS + q) * ST], a[(n * NS + q) * ST]);
 #pragma unroll
     for (int m = n + 1; m < NS; ++m) a[(m * NS + n) * ST] /= a[(n * NS + n) * ST];
   }
@@ -1402,13 +1419,14 @@ DEV void lu_apply(const double *a, const int *ipiv, double *b) {
 #pragma unroll
   for (int m = 1; m < NS; ++m)
 #pragma unroll
-    for (int t = 0; t < m; ++t) b[m] -= a[(m * NS + t) * ST] * b[t];
-  b[NS - 1] /= a[(NS * NS - 1) * ST];
+    for (int t = 0; t < m; ++t) b[m] = fma(-a[(m * NS + t) * ST], b[t], b[m]);
+  // back substitution column by column (each b[m] takes its terms from the last column down), the order
+  // in which a wave holding a row per lane can take them
 #pragma unroll
-  for (int m = NS - 2; m >= 0; --m) {
-#pragma unroll
-    for (int t = m + 1; t < NS; ++t) b[m] -= a[(m * NS + t) * ST] * b[t];
+  for (int m = NS - 1; m >= 0; --m) {
     b[m] /= a[(m * NS + m) * ST];
+#pragma unroll
+    for (int q = 0; q < m; ++q) b[q] = fma(-a[(q * NS + m) * ST], b[m], b[q]);
   }
 }
 
@@ -1480,7 +1498,7 @@ __global__ __launch_bounds__(kReactorBlock) void k_reactors(ReactorPool P, const
         for (int n = 0; n < NS; ++n) {
           const int e = (m * NS + n) * kReactorBlock;
           const double jmn = rhoY[n] > 1e-30 ? a[e] / rhoY[n] * 1e+3 / tb->imw[m] : 0.0;
-          a[e] = (m == n ? 1.0 : 0.0) - hs * kRkGamma * jmn;
+          a[e] = fma(-(hs * kRkGamma), jmn, m == n ? 1.0 : 0.0);
         }
       lu_factor<NS, kReactorBlock>(a, ipiv);
 #pragma unroll
@@ -1489,44 +1507,44 @@ __global__ __launch_bounds__(kReactorBlock) void k_reactors(ReactorPool P, const
       double imw = 0;
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
-        ys[l] = rhoY[l] + hs * kRkA21 * k1[l];
+        ys[l] = fma(hs * kRkA21, k1[l], rhoY[l]);
         yk[l] = ys[l] / rho;
-        imw += yk[l] * tb->imw[l];
+        imw = fma(yk[l], tb->imw[l], imw);
       }
       double ts = reactor_temperature<M>(tb, t, imw, yk, e);
       reactor_source<M>(tb, rho, ts, yk, omega, nullptr);
 #pragma unroll
-      for (int l = 0; l < NS; ++l) k2[l] = omega[l] + kRkG21 * k1[l];
+      for (int l = 0; l < NS; ++l) k2[l] = fma(kRkG21, k1[l], omega[l]);
       lu_apply<NS, kReactorBlock>(a, ipiv, k2);
 #pragma unroll
-      for (int l = 0; l < NS; ++l) k2[l] -= kRkG21 * k1[l];
+      for (int l = 0; l < NS; ++l) k2[l] = fma(-kRkG21, k1[l], k2[l]);
       imw = 0;
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
-        ys[l] = rhoY[l] + hs * (kRkA31 * k1[l] + kRkA32 * k2[l]);
+        ys[l] = fma(hs, dot2(kRkA31, k1[l], kRkA32, k2[l]), rhoY[l]);
         yk[l] = ys[l] / rho;
-        imw += yk[l] * tb->imw[l];
+        imw = fma(yk[l], tb->imw[l], imw);
       }
       ts = reactor_temperature<M>(tb, ts, imw, yk, e);
       reactor_source<M>(tb, rho, ts, yk, omega, nullptr);
 #pragma unroll
-      for (int l = 0; l < NS; ++l) k3[l] = omega[l] + kRkG31 * k1[l] + kRkG32 * k2[l];
+      for (int l = 0; l < NS; ++l) k3[l] = omega[l] + dot2(kRkG31, k1[l], kRkG32, k2[l]);
       lu_apply<NS, kReactorBlock>(a, ipiv, k3);
 #pragma unroll
-      for (int l = 0; l < NS; ++l) k3[l] -= kRkG31 * k1[l] + kRkG32 * k2[l];
+      for (int l = 0; l < NS; ++l) k3[l] -= dot2(kRkG31, k1[l], kRkG32, k2[l]);
 #pragma unroll
-      for (int l = 0; l < NS; ++l) k4[l] = omega[l] + kRkG41 * k1[l] + kRkG42 * k2[l] + kRkG43 * k3[l];
+      for (int l = 0; l < NS; ++l) k4[l] = omega[l] + dot3(kRkG41, k1[l], kRkG42, k2[l], kRkG43, k3[l]);
       lu_apply<NS, kReactorBlock>(a, ipiv, k4);
 #pragma unroll
-      for (int l = 0; l < NS; ++l) k4[l] -= kRkG41 * k1[l] + kRkG42 * k2[l] + kRkG43 * k3[l];
+      for (int l = 0; l < NS; ++l) k4[l] -= dot3(kRkG41, k1[l], kRkG42, k2[l], kRkG43, k3[l]);
       if (adaptive) {
         double rn[NS], err = 0;
 #pragma unroll
         for (int l = 0; l < NS; ++l) {
-          rn[l] = rhoY[l] + hs * (kRkB1 * k1[l] + kRkB2 * k2[l] + kRkB4 * k4[l]);
-          double dy = hs * (kRkE1 * k1[l] + kRkE2 * k2[l] + kRkE3 * k3[l] + kRkE4 * k4[l]);
-          dy /= rtol * rn[l] + atol;
-          err += dy * dy;
+          rn[l] = fma(hs, dot3(kRkB1, k1[l], kRkB2, k2[l], kRkB4, k4[l]), rhoY[l]);
+          double dy = hs * fma(kRkE4, k4[l], dot3(kRkE1, k1[l], kRkE2, k2[l], kRkE3, k3[l]));
+          dy /= fma(rtol, rn[l], atol);
+          err = fma(dy, dy, err);
         }
         err = sqrt(err / NS);
         double hstar = hs;
@@ -1552,7 +1570,7 @@ __global__ __launch_bounds__(kReactorBlock) void k_reactors(ReactorPool P, const
       } else {
 #pragma unroll
         for (int l = 0; l < NS; ++l) {
-          rhoY[l] += hs * (kRkB1 * k1[l] + kRkB2 * k2[l] + kRkB4 * k4[l]);
+          rhoY[l] = fma(hs, dot3(kRkB1, k1[l], kRkB2, k2[l], kRkB4, k4[l]), rhoY[l]);
           yk[l] = rhoY[l] / rho;
         }
         time += hs;
@@ -1563,24 +1581,24 @@ __global__ __launch_bounds__(kReactorBlock) void k_reactors(ReactorPool P, const
       reactor_source<M>(tb, rho, t, yk, omega, nullptr);
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
-        rn[l] = rhoY[l] + omega[l] * h;
+        rn[l] = fma(omega[l], h, rhoY[l]);
         ys[l] = rn[l] / rho;
-        imw += ys[l] * tb->imw[l];
+        imw = fma(ys[l], tb->imw[l], imw);
       }
       double ts = reactor_temperature<M>(tb, t, imw, ys, e);
       reactor_source<M>(tb, rho, ts, ys, omega, nullptr);
       imw = 0;
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
-        rn[l] = 0.75 * rhoY[l] + 0.25 * (rn[l] + omega[l] * h);
+        rn[l] = dot2(0.75, rhoY[l], 0.25, fma(omega[l], h, rn[l]));
         ys[l] = rn[l] / rho;
-        imw += ys[l] * tb->imw[l];
+        imw = fma(ys[l], tb->imw[l], imw);
       }
       ts = reactor_temperature<M>(tb, ts, imw, ys, e);
       reactor_source<M>(tb, rho, ts, ys, omega, nullptr);
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
-        rhoY[l] = (rhoY[l] + 2.0 * (rn[l] + omega[l] * h)) / 3.0;
+        rhoY[l] = div_by<3>(fma(2.0, fma(omega[l], h, rn[l]), rhoY[l]));
         if (rhoY[l] < 0) rhoY[l] = 0;
         yk[l] = rhoY[l] / rho;
       }
@@ -1592,12 +1610,12 @@ __global__ __launch_bounds__(kReactorBlock) void k_reactors(ReactorPool P, const
 #pragma unroll
       for (int m = 0; m < NS; ++m) {
         const double jmm = rhoY[m] > 1e-30 ? zz[(m * NS + m) * kReactorBlock] / rhoY[m] * 1e+3 / tb->imw[m] : 0.0;
-        omega[m] /= 1 - h * jmm;
+        omega[m] /= fma(-h, jmm, 1.0);
       }
       double sum = 0;
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
-        rhoY[l] += omega[l] * h;
+        rhoY[l] = fma(omega[l], h, rhoY[l]);
         if (rhoY[l] < 0) rhoY[l] = 0;
         sum += rhoY[l];
       }
@@ -1615,7 +1633,7 @@ __global__ __launch_bounds__(kReactorBlock) void k_reactors(ReactorPool P, const
     if (!accepted) continue;
     double imw = 0;
 #pragma unroll
-    for (int l = 0; l < NS; ++l) imw += yk[l] * tb->imw[l];
+    for (int l = 0; l < NS; ++l) imw = fma(yk[l], tb->imw[l], imw);
     t = reactor_temperature<M>(tb, t, imw, yk, e);
     ++steps;
   }
@@ -1635,394 +1653,547 @@ __global__ __launch_bounds__(kReactorBlock) void k_reactors(ReactorPool P, const
 }
 
 // ---------------------------------------------------------------------------
-// The same reactors with one wave per slot (latency): the state and the step
-// control are held by every lane alike, and the costly parts of a step are
-// spread over the lanes: G/RT, h and cp per species, the rates of progress per
-// reaction, the creation / destruction sums per species and the source
-// Jacobian per matrix element, the LU factorisation per row.  Every sum runs
-// in the order of the one-lane kernel above, so a slot's result is the same
-// bit for bit under either kernel.
+// The same reactors with one wave per slot: species l's partial density, mass
+// fraction, ROK4E stages, h, cp and G/RT live on lane l, reaction r's constants
+// and rates of progress on lane r, row m of the iteration matrix in lane m's
+// registers (no LDS in the factorisation), so an operation over species is one
+// instruction instead of n_spec and nothing about the mechanism is read from
+// memory inside a step.  Values cross lanes by readlane (uniform source) or
+// through LDS where the source differs per lane.  Every sum runs in the order
+// of the one-lane kernel above, so a slot's result is the same bit for bit
+// under either kernel.
+//
+// Bound by the latency of dependent FP64 operations while few waves share a
+// SIMD: a step is four source evaluations (log, three exponentials and the
+// Troe chain in sequence), three temperature solves, the LU factorisation and
+// its four solves.  A step takes 25 us with six reactors in flight against 49
+// with the state replicated in every lane, the tables read from memory and the
+// factors in LDS, and 58 us with 5000 in flight against 212 with a lane each.
 // ---------------------------------------------------------------------------
 constexpr int kWave = 64;
 
-// h and cp of species i at t (the arithmetic of thermo_h_cp)
-template <int M>
-DEV void thermo_h_cp1(const Tab *__restrict__ tb, int i, double t, double &h, double &cp) {
-  if constexpr (kNasa9(M)) {
-    nasa9_h_cp<true, true>(tb, i, nasa9_terms(t), h, cp);
-    h *= tb->gas_const[i];
-    cp *= tb->gas_const[i];
-  } else {
-    const double t2 = t * t, t3 = t2 * t, t4 = t3 * t, t5 = t4 * t;
-    const double tl = tb->t_low[i], th = tb->t_high[i];
-    double vh, vc;
-    if (t < tl || t > th) {
-      const double tt = t < tl ? tl : th;
-      const double *c = t < tl ? tb->low_coeff[i] : tb->high_coeff[i];
-      const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt5 = tt4 * tt;
-      vh = nasa_h(c, tt, tt2, tt3, tt4, tt5);
-      vc = nasa_cp(c, tt, tt2, tt3, tt4);
-      vh += vc * (t - tt);
-    } else {
-      const bool lo = t < tb->t_mid[i];
-      double c[6];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) c[k] = lo ? tb->low_coeff[i][k] : tb->high_coeff[i][k];
-      vh = nasa_h(c, t, t2, t3, t4, t5);
-      vc = nasa_cp(c, t, t2, t3, t4);
-    }
-    h = vh * tb->gas_const[i];
-    cp = vc * tb->gas_const[i];
-  }
+// x / d with rd = 1 / d rounded: the IEEE quotient's bits (see div_by)
+DEV double div_rcp(double x, double d, double rd) {
+  const double q = x * rd;
+  return fma(fma(-d, q, x), rd, q);
+}
+
+// lane src's v in every lane (src uniform)
+DEV double bcast(double v, int src) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), src);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
+  return __hiloint2double(hi, lo);
 }
 
 template <int M>
 struct ReactorWaveLds {
   static constexpr int NS = kNs(M);
-  double c[NS], g[NS], h[NS], cp[NS], cr[NS], od[NS];
-  double q1[COREFL_MAX_REAC], q2[COREFL_MAX_REAC];
-  double a[NS * NS];  // source Jacobian, then the ROK4E iteration matrix and its LU factors
+  double c[NS], g[NS], y[NS], h[NS], cp[NS];
+  double a[NS * NS];  // source Jacobian sums, or the iteration matrix on its way to the row lanes
   // forward / backward stoichiometric coefficients (r, l) of the mechanism, staged once per launch
   double sf[COREFL_MAX_REAC * NS], sb[COREFL_MAX_REAC * NS];
+  double third[COREFL_MAX_REAC * NS];       // third-body efficiencies (r, l)
+  double poly[kNasa9(M) ? 1 : 14 * NS];     // NASA-7 low and high coefficients (k, l)
 };
 
-// Stages the stoichiometry of the mechanism into the wave's LDS (the reaction
-// lists' coefficients; a species takes part in reaction r when either is not 0).
-// Read from LDS the species sums below take less time than walking the
-// reaction lists in global memory.
+// A lane's constants: those of its reaction (lane r) and of its species (lane l).
 template <int M>
-DEV void wave_stage_stoichiometry(const Tab *__restrict__ tb, ReactorWaveLds<M> &L) {
-  constexpr int NS = kNs(M);
-  const int n = tb->n_reac * NS;
-  for (int e = threadIdx.x; e < n; e += kWave) {
-    const int r = e / NS, l = e % NS;
-    L.sf[e] = static_cast<double>(tb->stoi_f[r][l]);
-    L.sb[e] = static_cast<double>(tb->stoi_b[r][l]);
-  }
-  __syncthreads();
-}
+struct ReactorLane {
+  static constexpr int NS = kNs(M);
+  static constexpr int kIn = 4, kNu = 8;  // list entries held in registers; longer lists go on in the tables
+  // reaction
+  int type, rev, nf, nb, nnu;
+  double A, b, Ea, A2, b2, Ea2, alpha, t1, t2, t3, order;
+  unsigned long long f, bk, nu[2];  // 16 bits an entry: species, exponent (or nu)
+  // species
+  double imw, gas, conv, tl, tm, th;
+};
 
-// v[i] of a register array for a lane-dependent i
-template <int N>
-DEV double pick(const double *v, int i) {
-  double x = 0;
+template <int M>
+DEV void load_reactor_lane(const Tab *__restrict__ tb, int lane, ReactorLane<M> &K) {
+  constexpr int NS = kNs(M);
+  const int r = lane < tb->n_reac ? lane : 0, l = lane < NS ? lane : 0;
+  K.type = K.rev = K.nf = K.nb = K.nnu = 0;
+  K.f = K.bk = K.nu[0] = K.nu[1] = 0;
+  if (tb->n_reac > 0) {
+    const Reac &R = tb->reac[r];
+    K.type = tb->reac_type[r];
+    K.rev = tb->rev_type[r];
+    K.nf = R.nf;
+    K.nb = R.nb;
+    K.nnu = R.nnu;
 #pragma unroll
-  for (int l = 0; l < N; ++l) x = l == i ? v[l] : x;
-  return x;
+    for (int k = 0; k < ReactorLane<M>::kIn; ++k)
+      if (k < R.nf) K.f |= static_cast<unsigned long long>((R.f_idx[k] & 255) | (R.f_ord[k] & 255) << 8) << (16 * k);
+#pragma unroll
+    for (int k = 0; k < ReactorLane<M>::kIn; ++k)
+      if (k < R.nb) K.bk |= static_cast<unsigned long long>((R.b_idx[k] & 255) | (R.b_ord[k] & 255) << 8) << (16 * k);
+#pragma unroll
+    for (int k = 0; k < ReactorLane<M>::kNu; ++k)
+      if (k < R.nnu)
+        K.nu[k / 4] |= static_cast<unsigned long long>((R.nu_idx[k] & 255) | (static_cast<int>(R.nu[k]) & 255) << 8)
+                     << (16 * (k % 4));
+  }
+  K.A = tb->A[r];
+  K.b = tb->b[r];
+  K.Ea = tb->Ea[r];
+  K.A2 = tb->A2[r];
+  K.b2 = tb->b2[r];
+  K.Ea2 = tb->Ea2[r];
+  K.alpha = tb->troe_alpha[r];
+  K.t1 = tb->troe_t1[r];
+  K.t2 = tb->troe_t2[r];
+  K.t3 = tb->troe_t3[r];
+  K.order = static_cast<double>(tb->order[r]);
+  K.imw = tb->imw[l];
+  K.gas = tb->gas_const[l];
+  K.conv = tb->mol_conv[l];
+  if constexpr (!kNasa9(M)) {
+    K.tl = tb->t_low[l];
+    K.tm = tb->t_mid[l];
+    K.th = tb->t_high[l];
+  }
 }
 
-// reactor_source over the wave: omega (every lane) and, with JAC, the source
-// Jacobian sums zz in L.a
-template <int M, bool JAC>
-DEV void wave_source(const Tab *__restrict__ tb, ReactorWaveLds<M> &L, double rho, double t, const double *yk,
-                     double *omega) {
+// h and cp of the lane's species at t (the arithmetic of thermo_h_cp)
+template <int M>
+DEV void lane_h_cp(const Tab *__restrict__ tb, const ReactorLane<M> &K, const ReactorWaveLds<M> &L, int l, double t,
+                   double &h, double &cp) {
+  if constexpr (kNasa9(M)) {
+    nasa9_h_cp<true, true>(tb, l, nasa9_terms(t), h, cp);
+    h *= K.gas;
+    cp *= K.gas;
+  } else {
+    const bool low = t < K.tl, out = low || t > K.th;
+    const double x = out ? (low ? K.tl : K.th) : t;
+    const bool lo = out ? low : t < K.tm;
+    const double t2 = x * x, t3 = t2 * x, t4 = t3 * x, t5 = t4 * x;
+    double c[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) c[k] = L.poly[(k + (lo ? 0 : 7)) * kNs(M) + l];
+    double vh = nasa_h(c, x, t2, t3, t4, t5);
+    const double vc = nasa_cp(c, x, t2, t3, t4);
+    if (out) vh = fma(vc, t - x, vh);
+    h = vh * K.gas;
+    cp = vc * K.gas;
+  }
+}
+
+// G/RT of the lane's species at t (the arithmetic of thermo_gibbs; ln_t = log t)
+template <int M>
+DEV double lane_gibbs(const Tab *__restrict__ tb, const ReactorLane<M> &K, const ReactorWaveLds<M> &L, int l, double t,
+                      double ln_t) {
+  if constexpr (kNasa9(M)) {
+    return nasa9_g1(tb, l, nasa9_terms(t));
+  } else {
+    const bool low = t < K.tl, out = low || t > K.th;
+    const double x = out ? (low ? K.tl : K.th) : t;
+    const bool lo = out ? low : t < K.tm;
+    const double t2 = x * x, t3 = t2 * x, t4 = t3 * x;
+    double lx = ln_t;
+    if (out) lx = log(x);
+    double c[7];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) c[k] = L.poly[(k + (lo ? 0 : 7)) * kNs(M) + l];
+    return nasa_g(c, x, t2, t3, t4, 1 / x, lx);
+  }
+}
+
+// Rates of progress of the lane's reaction (the arithmetic of reaction_progress,
+// one temperature) from the concentrations and G/RT in LDS.  The exponentials
+// that do not depend on each other are formed together, ahead of the fall-off
+// branch, so that their chains overlap.
+template <int M>
+DEV void lane_progress(const Tab *__restrict__ tb, const ReactorLane<M> &K, const ReactorWaveLds<M> &L, int r, double T,
+                       double ln_t, double inv_t, double ln_temp_t, double &q1, double &q2) {
   constexpr int NS = kNs(M);
+  constexpr double kLn10 = 2.302585092994046, kInvLn10 = 0.4342944819032518;
+  const int type = K.type;
+  double cc = 0;
+#pragma unroll
+  for (int l = 0; l < NS; ++l) cc = fma(L.c[l], L.third[r * NS + l], cc);
+  double d_gibbs = 0;
+#pragma unroll
+  for (int k = 0; k < ReactorLane<M>::kNu; ++k) {
+    const int e = static_cast<int>(K.nu[k / 4] >> (16 * (k % 4)));
+    if (k < K.nnu) d_gibbs = fma(L.g[e & 255], static_cast<double>(static_cast<signed char>(e >> 8)), d_gibbs);
+  }
+  for (int k = ReactorLane<M>::kNu; k < K.nnu; ++k) d_gibbs = fma(L.g[tb->reac[r].nu_idx[k]], tb->reac[r].nu[k], d_gibbs);
+  double kf = arrhenius_ln(ln_t, inv_t, K.A, K.b, K.Ea);
+  const double k2 = arrhenius_ln(ln_t, inv_t, K.A2, K.b2, K.Ea2);
+  const double ekc = exp(fma(-K.order, ln_temp_t, d_gibbs));
+  double p1 = 1.0, p2 = 1.0;
+#pragma unroll
+  for (int k = 0; k < ReactorLane<M>::kIn; ++k) {
+    const int e = static_cast<int>(K.f >> (16 * k)) & 0xffff, w = static_cast<int>(K.bk >> (16 * k)) & 0xffff;
+    if (k < K.nf) p1 *= ipow(L.c[e & 255], e >> 8);
+    if (k < K.nb) p2 *= ipow(L.c[w & 255], w >> 8);
+  }
+  for (int k = ReactorLane<M>::kIn; k < K.nf; ++k) p1 *= ipow(L.c[tb->reac[r].f_idx[k]], tb->reac[r].f_ord[k]);
+  for (int k = ReactorLane<M>::kIn; k < K.nb; ++k) p2 *= ipow(L.c[tb->reac[r].b_idx[k]], tb->reac[r].b_ord[k]);
+  if (type == 3) {
+    kf += k2;
+  } else if (type == 4) {
+    kf *= cc;
+  } else if (type > 4) {
+    const double kf_low = k2, kf_high = kf;
+    if (kf_high < 1e-25 && kf_low < 1e-25) {
+      kf = 0;
+    } else {
+      const double reduced_pressure = kf_low * cc / kf_high;
+      double F = 1.0;
+      if (type > 5) {
+        double f_cent = dot2(1 - K.alpha, exp(-T / K.t3), K.alpha, exp(-T / K.t1));
+        if (type == 7) f_cent += exp(-K.t2 * inv_t);
+        const double logFc = log(f_cent) * kInvLn10;
+        const double cT = fma(-0.67, logFc, -0.4);
+        const double nn = fma(-1.27, logFc, 0.75);
+        const double lp = fma(log(reduced_pressure), kInvLn10, cT);  // log10 Pr + c
+        const double tempo = lp / fma(-0.14, lp, nn);
+        F = exp(kLn10 * (logFc / fma(tempo, tempo, 1.0)));
+      }
+      kf = kf_high * reduced_pressure / (1.0 + reduced_pressure) * F;
+    }
+  }
+  double kb = 0;
+  if (type != 0) {
+    if (K.rev == 1) {
+      kb = k2;
+      if (type == 4) kb *= cc;
+    }
+    if (type != 2) kb = kf * ekc;
+  }
+  q1 = p1 * kf;
+  q2 = type != 0 ? p2 * kb : 0.0;
+}
+
+// The source Jacobian's elements spread over the lanes: lane -> column lane % NS
+// and the rows lane / NS + k kGroups.
+template <int NS>
+struct JacLanes {
+  static constexpr int kGroups = NS * NS <= kWave ? NS : kWave / NS;
+  static constexpr int kRows = (NS + kGroups - 1) / kGroups;
+};
+
+// omega of the lane's species from t and the lane's y and, with jac (uniform),
+// the source Jacobian sums zz of the lane's elements (reactor_source).
+template <int M>
+DEV double wave_source(const Tab *__restrict__ tb, const ReactorLane<M> &K, ReactorWaveLds<M> &L, double rho, double t,
+                       double y, bool jac, double *zz) {
+  constexpr int NS = kNs(M), G = JacLanes<NS>::kGroups, RP = JacLanes<NS>::kRows;
   const int lane = threadIdx.x, nr = tb->n_reac;
+  const double ln_t = log(t), inv_t = 1.0 / t;
   if (lane < NS) {
-    L.c[lane] = rho * pick<NS>(yk, lane) * tb->imw[lane] * 1e-3;
-    L.g[lane] = gibbs1<M>(tb, lane, t);
+    L.c[lane] = rho * y * K.imw * 1e-3;
+    L.g[lane] = lane_gibbs<M>(tb, K, L, lane, t, ln_t);
   }
   __syncthreads();
-  if (lane < nr) {
-    // concentrations and G/RT read from LDS at the reaction's own species indices
-    const double ln_t = log(t), inv_t = 1.0 / t;
-    double q1, q2;
-    reaction_progress<M>(tb, lane, t, t, false, ln_t, inv_t, ln_std_conc(ln_t), L.c, L.g, q1, q2);
-    L.q1[lane] = q1;
-    L.q2[lane] = q2;
-  }
+  double q1 = 0, q2 = 0;
+  if (lane < nr) lane_progress<M>(tb, K, L, lane, t, ln_t, inv_t, ln_std_conc(ln_t), q1, q2);
   __syncthreads();
-  if (lane < NS) {
-    double cr = 0, od = 0;
-#pragma unroll 4
-    for (int r = 0; r < nr; ++r) {
-      const double sf = L.sf[r * NS + lane], sb = L.sb[r * NS + lane];
-      if (sf != 0.0 || sb != 0.0) {
-        const double q1 = L.q1[r], q2 = L.q2[r];
-        cr += q2 * sf + q1 * sb;
-        od += q1 * sf + q2 * sb;
-      }
-    }
-    L.cr[lane] = cr;
-    L.od[lane] = od;
-  }
-  if constexpr (JAC) {
-    for (int e = lane; e < NS * NS; e += kWave) {
-      const int l = e / NS, l2 = e % NS;
-      double zz = 0;
-#pragma unroll 4
-      for (int r = 0; r < nr; ++r) {
-        const double sf = L.sf[r * NS + l], sb = L.sb[r * NS + l];
-        const double sf2 = L.sf[r * NS + l2], sb2 = L.sb[r * NS + l2];
-        if ((sf != 0.0 || sb != 0.0) && (sf2 != 0.0 || sb2 != 0.0))
-          zz += (sb - sf) * (sf2 * L.q1[r] - sb2 * L.q2[r]);
-      }
-      L.a[e] = zz;
-    }
-  }
-  __syncthreads();
+  const int col = lane % NS, row0 = lane / NS;
+  double cr = 0, od = 0;
 #pragma unroll
-  for (int l = 0; l < NS; ++l) {
-    const double conv = tb->mol_conv[l];
-    omega[l] = L.cr[l] * conv - L.od[l] * conv;
+  for (int k = 0; k < RP; ++k) zz[k] = 0;
+#pragma unroll 4
+  for (int r = 0; r < nr; ++r) {
+    const double q1r = bcast(q1, r), q2r = bcast(q2, r);
+    const double sf = L.sf[r * NS + col], sb = L.sb[r * NS + col];
+    if (sf != 0.0 || sb != 0.0) {
+      cr += dot2(q2r, sf, q1r, sb);
+      od += dot2(q1r, sf, q2r, sb);
+      if (jac) {
+#pragma unroll
+        for (int k = 0; k < RP; ++k) {
+          const int row = min(row0 + k * G, NS - 1);
+          const double sfm = L.sf[r * NS + row], sbm = L.sb[r * NS + row];
+          if (sfm != 0.0 || sbm != 0.0) zz[k] = fma(sbm - sfm, dot2(sf, q1r, -sb, q2r), zz[k]);
+        }
+      }
+    }
   }
+  return dot2(cr, K.conv, -od, K.conv);
+}
+
+// sum over the species of the lanes' v times the table's imw, in species order
+template <int M>
+DEV double wave_imw(const Tab *__restrict__ tb, double v) {
+  constexpr int NS = kNs(M);
+  double s = 0;
+#pragma unroll
+  for (int l = 0; l < NS; ++l) s = fma(bcast(v, l), tb->imw[l], s);
+  return s;
 }
 
 // reactor_temperature over the wave (h and cp per species on its lane)
 template <int M>
-DEV double wave_temperature(const Tab *__restrict__ tb, ReactorWaveLds<M> &L, double t0, double imw, const double *yk,
-                            double e) {
+DEV double wave_temperature(const Tab *__restrict__ tb, const ReactorLane<M> &K, ReactorWaveLds<M> &L, double t0,
+                            double imw, double y, double e) {
   constexpr int NS = kNs(M);
   const int lane = threadIdx.x;
-  double t = t0, err = 1e+6;
+  double t = t0, err = 1e+6, ya[NS];
   const double r = kRu * imw;
+  if (lane < NS) L.y[lane] = y;
+  __syncthreads();
+#pragma unroll
+  for (int l = 0; l < NS; ++l) ya[l] = L.y[l];
   int iter = 0;
   while (err > 1e-8 && iter++ < 100) {
-    if (lane < NS) {
-      double h, cp;
-      thermo_h_cp1<M>(tb, lane, t, h, cp);
-      L.h[lane] = h;
-      L.cp[lane] = cp;
-    }
+    if (lane < NS) lane_h_cp<M>(tb, K, L, lane, t, L.h[lane], L.cp[lane]);
     __syncthreads();
     double cp_tot = 0, hm = 0;
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      cp_tot += L.cp[l] * yk[l];
-      hm += L.h[l] * yk[l];
+      cp_tot = fma(L.cp[l], ya[l], cp_tot);
+      hm = fma(L.h[l], ya[l], hm);
     }
     __syncthreads();  // read before the next iteration writes
-    const double t1 = t - (hm - r * t - e) / (cp_tot - r);
+    const double t1 = t - (fma(-r, t, hm) - e) / (cp_tot - r);
     err = fabs(1 - t1 / t);
     t = t1;
   }
   return t;
 }
 
-// lu_factor over the wave: each step's column, row and scaling spread over the rows / columns
+// The wave's LU factors: row m of the matrix and the reciprocal of its pivot on
+// lane m, the pivots' rows (uniform).
 template <int NS>
-DEV void wave_lu_factor(double *a, int *ipiv) {
+struct WaveLu {
+  double row[NS], rp;
+  int ipiv[NS];
+};
+
+// lu_factor: each column's multipliers and updates row by row on the lanes, the
+// pivot row by readlane; an element takes its terms in the order of lu_factor.
+template <int NS>
+DEV void wave_lu_factor(WaveLu<NS> &F) {
   const int lane = threadIdx.x;
+  F.rp = 0;
 #pragma unroll
   for (int n = 0; n < NS; ++n) {
-    if (lane >= n && lane < NS) {
-      double v = a[lane * NS + n];
-      for (int t = 0; t < n; ++t) v -= a[lane * NS + t] * a[t * NS + n];
-      a[lane * NS + n] = v;
-    }
-    __syncthreads();
+    double piv = bcast(F.row[n], n);
     int ik = n;
-    double best = fabs(a[n * NS + n]);
+    if (__any(lane > n && lane < NS && fabs(F.row[n]) > fabs(piv))) {
+      double best = fabs(piv);
 #pragma unroll
-    for (int m = n + 1; m < NS; ++m) {
-      const double v = fabs(a[m * NS + n]);
-      if (v > best) {
-        best = v;
-        ik = m;
+      for (int m = n + 1; m < NS; ++m) {
+        const double v = fabs(bcast(F.row[n], m));
+        if (v > best) {
+          best = v;
+          ik = m;
+        }
       }
+      ik = __builtin_amdgcn_readfirstlane(ik);
+      const int src = lane == n ? ik : (lane == ik ? n : lane);
+#pragma unroll
+      for (int q = 0; q < NS; ++q) F.row[q] = __shfl(F.row[q], src, kWave);
+      piv = bcast(F.row[n], n);
     }
-    ipiv[n] = ik;
-    __syncthreads();  // every lane has read column n
-    if (ik != n && lane < NS) {
-      const double x = a[n * NS + lane], w = a[ik * NS + lane];
-      a[n * NS + lane] = w;
-      a[ik * NS + lane] = x;
+    F.ipiv[n] = ik;
+    const double rp = 1.0 / piv;
+    if (lane == n) F.rp = rp;
+    double u[NS];
+#pragma unroll
+    for (int q = n + 1; q < NS; ++q) u[q] = bcast(F.row[q], n);
+    if (lane > n) {
+      F.row[n] = div_rcp(F.row[n], piv, rp);
+#pragma unroll
+      for (int q = n + 1; q < NS; ++q) F.row[q] = fma(-F.row[n], u[q], F.row[q]);
     }
-    __syncthreads();
-    if (lane > n && lane < NS) {
-      double v = a[n * NS + lane];
-      for (int t = 0; t < n; ++t) v -= a[n * NS + t] * a[t * NS + lane];
-      a[n * NS + lane] = v;
-      a[lane * NS + n] /= a[n * NS + n];
-    }
-    __syncthreads();
   }
 }
 
+// lu_apply on the lanes' right-hand side
+template <int NS>
+DEV double wave_lu_apply(const WaveLu<NS> &F, double b) {
+  const int lane = threadIdx.x;
+#pragma unroll
+  for (int m = 0; m < NS; ++m)
+    if (F.ipiv[m] != m)
+      b = __shfl(b, lane == m ? F.ipiv[m] : (lane == F.ipiv[m] ? m : lane), kWave);
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t) {
+    const double x = bcast(b, t);
+    if (lane > t) b = fma(-F.row[t], x, b);
+  }
+#pragma unroll
+  for (int m = NS - 1; m >= 0; --m) {
+    if (lane == m) b = div_rcp(b, F.row[m], F.rp);
+    const double x = bcast(b, m);
+    if (lane < m) b = fma(-F.row[m], x, b);
+  }
+  return b;
+}
+
+// reactor_fault with the partial densities on the lanes
+template <int NS>
+DEV int wave_fault(double t, double time, double h, double t_end, double rhoY, long tries, long cap) {
+  const bool finite =
+      isfinite(t) && isfinite(time) && isfinite(h) && !__any(static_cast<int>(threadIdx.x) < NS && !isfinite(rhoY));
+  if (!finite) return COREFL_FAIL_NONFINITE;
+  if (time >= t_end) return 0;
+  const double hs = fmin(h, t_end - time);
+  if (!(hs > 0) || time + hs == time) return COREFL_FAIL_STEP;
+  if (cap > 0 && tries >= cap) return COREFL_FAIL_CAP;
+  return 0;
+}
+
 template <int M>
-__global__ __launch_bounds__(kWave) void k_reactors_wave(ReactorPool P, const Tab *__restrict__ tb, int max_steps,
+__global__ __launch_bounds__(kWave, 2) void k_reactors_wave(ReactorPool P, const Tab *__restrict__ tb, int max_steps,
                                                          int n_slots) {
-  constexpr int NS = kNs(M);
+  constexpr int NS = kNs(M), G = JacLanes<NS>::kGroups, RP = JacLanes<NS>::kRows;
   __shared__ ReactorWaveLds<M> L;
   const int s = blockIdx.x;
   if (s >= n_slots || P.status[s] != 1) return;
-  const int lane = threadIdx.x;
-  wave_stage_stoichiometry<M>(tb, L);
+  const int lane = threadIdx.x, sl = lane < NS ? lane : 0;
+  const int n_stoi = tb->n_reac * NS;
+  for (int e = lane; e < n_stoi; e += kWave) {
+    L.sf[e] = static_cast<double>(tb->stoi_f[e / NS][e % NS]);
+    L.sb[e] = static_cast<double>(tb->stoi_b[e / NS][e % NS]);
+    L.third[e] = tb->third_body[e / NS][e % NS];
+  }
+  if constexpr (!kNasa9(M))
+    for (int e = lane; e < 14 * NS; e += kWave)
+      L.poly[e] = e / NS < 7 ? tb->low_coeff[e % NS][e / NS] : tb->high_coeff[e % NS][e / NS - 7];
+  ReactorLane<M> K;
+  load_reactor_lane<M>(tb, lane, K);
   const long cap = P.cap;
-  double rhoY[NS], yk[NS], omega[NS];
   const double rho = P.rho[s], e = P.e[s], t_end = P.t_end[s], rtol = P.rtol[s], atol = P.atol[s];
+  const double rrho = 1.0 / rho;
   const int scheme = P.scheme[s], adaptive = P.adaptive[s], conserve = P.conserve[s];
   double t = P.t[s], time = P.time[s], h = P.h[s], err_last = P.err_last[s];
   long steps = P.steps[s], rejected = P.rejected[s];
   const long step_cap = P.max_steps[s];
-#pragma unroll
-  for (int l = 0; l < NS; ++l) {
-    rhoY[l] = P.rhoY[l * cap + s];
-    yk[l] = rhoY[l] / rho;
-  }
+  double rhoY = P.rhoY[sl * cap + s];
+  double y = div_rcp(rhoY, rho, rrho);
+  __syncthreads();
   int fail = 0;
+  // The schemes share one source and one temperature evaluation in the code: a step is a source at the
+  // step's start, then for each further stage the stage's mass fractions, their temperature and a source
+  // there, and the temperature of the new state.  The last stage is 2 (ROK4E, SSP-RK3) or 0 (point-implicit).
+  const int last = scheme == 1 || scheme == 3 ? 2 : 0;
+  const int col = lane % NS, row0 = lane / NS;
   for (int it = 0; it < max_steps; ++it) {
-    fail = reactor_fault<NS>(t, time, h, t_end, rhoY, steps + rejected, step_cap);
+    fail = wave_fault<NS>(t, time, h, t_end, rhoY, steps + rejected, step_cap);
     if (fail || time >= t_end) break;
+    const double hs = fmin(h, t_end - time);
     bool accepted = true;
-    if (scheme == 1) {
-      double k1[NS], k2[NS], k3[NS], k4[NS], ys[NS];
-      int ipiv[NS];
-      wave_source<M, true>(tb, L, rho, t, yk, omega);
-      const double hs = fmin(h, t_end - time);
-      for (int el = lane; el < NS * NS; el += kWave) {
-        const int m = el / NS, n = el % NS;
-        const double rn = pick<NS>(rhoY, n);
-        const double jmn = rn > 1e-30 ? L.a[el] / rn * 1e+3 / tb->imw[m] : 0.0;
-        L.a[el] = (m == n ? 1.0 : 0.0) - hs * kRkGamma * jmn;
-      }
-      __syncthreads();
-      wave_lu_factor<NS>(L.a, ipiv);
+    WaveLu<NS> F;
+    double k1 = 0, k2 = 0, rn = rhoY, ts = t;
+#pragma unroll 1
+    for (int stage = 0; stage <= last; ++stage) {
+      double zz[RP];
+      const double o = wave_source<M>(tb, K, L, rho, ts, y, stage == 0 && scheme != 3, zz);
+      if (scheme == 1) {
+        if (stage == 0) {
+          const double rc = __shfl(rhoY, col, kWave), rrc = 1.0 / rc;
 #pragma unroll
-      for (int l = 0; l < NS; ++l) k1[l] = omega[l];
-      lu_apply<NS>(L.a, ipiv, k1);
-      double imw = 0;
-#pragma unroll
-      for (int l = 0; l < NS; ++l) {
-        ys[l] = rhoY[l] + hs * kRkA21 * k1[l];
-        yk[l] = ys[l] / rho;
-        imw += yk[l] * tb->imw[l];
-      }
-      double ts = wave_temperature<M>(tb, L, t, imw, yk, e);
-      wave_source<M, false>(tb, L, rho, ts, yk, omega);
-#pragma unroll
-      for (int l = 0; l < NS; ++l) k2[l] = omega[l] + kRkG21 * k1[l];
-      lu_apply<NS>(L.a, ipiv, k2);
-#pragma unroll
-      for (int l = 0; l < NS; ++l) k2[l] -= kRkG21 * k1[l];
-      imw = 0;
-#pragma unroll
-      for (int l = 0; l < NS; ++l) {
-        ys[l] = rhoY[l] + hs * (kRkA31 * k1[l] + kRkA32 * k2[l]);
-        yk[l] = ys[l] / rho;
-        imw += yk[l] * tb->imw[l];
-      }
-      ts = wave_temperature<M>(tb, L, ts, imw, yk, e);
-      wave_source<M, false>(tb, L, rho, ts, yk, omega);
-#pragma unroll
-      for (int l = 0; l < NS; ++l) k3[l] = omega[l] + kRkG31 * k1[l] + kRkG32 * k2[l];
-      lu_apply<NS>(L.a, ipiv, k3);
-#pragma unroll
-      for (int l = 0; l < NS; ++l) k3[l] -= kRkG31 * k1[l] + kRkG32 * k2[l];
-#pragma unroll
-      for (int l = 0; l < NS; ++l) k4[l] = omega[l] + kRkG41 * k1[l] + kRkG42 * k2[l] + kRkG43 * k3[l];
-      lu_apply<NS>(L.a, ipiv, k4);
-#pragma unroll
-      for (int l = 0; l < NS; ++l) k4[l] -= kRkG41 * k1[l] + kRkG42 * k2[l] + kRkG43 * k3[l];
-      __syncthreads();  // the factors are read before the next step's Jacobian overwrites them
-      if (adaptive) {
-        double rn[NS], err = 0;
-#pragma unroll
-        for (int l = 0; l < NS; ++l) {
-          rn[l] = rhoY[l] + hs * (kRkB1 * k1[l] + kRkB2 * k2[l] + kRkB4 * k4[l]);
-          double dy = hs * (kRkE1 * k1[l] + kRkE2 * k2[l] + kRkE3 * k3[l] + kRkE4 * k4[l]);
-          dy /= rtol * rn[l] + atol;
-          err += dy * dy;
-        }
-        err = sqrt(err / NS);
-        double hstar = hs;
-        if (steps > 0)
-          hstar *= fmin(5.0, fmax(0.2, 0.8 * pow(err_last, 0.1) * pow(err + 1e-20, -0.175)));
-        else if (err > 1)
-          hstar *= 0.2;
-        if (err <= 1) {
-#pragma unroll
-          for (int l = 0; l < NS; ++l) {
-            rhoY[l] = rn[l];
-            yk[l] = rn[l] / rho;
+          for (int k = 0; k < RP; ++k) {
+            const int row = row0 + k * G;
+            if (lane < NS * G && row < NS) {
+              const double jmn =
+                  rc > 1e-30 ? div_rcp(div_rcp(zz[k], rc, rrc) * 1e+3, tb->imw[row], tb->rcp_imw[row]) : 0.0;
+              L.a[row * NS + col] = fma(-(hs * kRkGamma), jmn, row == col ? 1.0 : 0.0);
+            }
           }
-          time += hs;
-          err_last = err;
-        } else {
-          accepted = false;
-          ++rejected;
+          __syncthreads();
 #pragma unroll
-          for (int l = 0; l < NS; ++l) yk[l] = rhoY[l] / rho;
+          for (int n = 0; n < NS; ++n) F.row[n] = L.a[sl * NS + n];
+          __syncthreads();
+          wave_lu_factor<NS>(F);
         }
-        h = hstar;
+        const double g = stage == 0 ? 0.0 : (stage == 1 ? kRkG21 * k1 : dot2(kRkG31, k1, kRkG32, k2));
+        double x = wave_lu_apply<NS>(F, stage == 1 ? fma(kRkG21, k1, o) : (stage == 0 ? o : o + g));
+        if (stage == 0) {
+          k1 = x;
+          y = div_rcp(fma(hs * kRkA21, k1, rhoY), rho, rrho);
+        } else if (stage == 1) {
+          k2 = fma(-kRkG21, k1, x);
+          y = div_rcp(fma(hs, dot2(kRkA31, k1, kRkA32, k2), rhoY), rho, rrho);
+        } else {
+          const double k3 = x - g, g4 = dot3(kRkG41, k1, kRkG42, k2, kRkG43, k3);
+          const double k4 = wave_lu_apply<NS>(F, o + g4) - g4;
+          rn = fma(hs, dot3(kRkB1, k1, kRkB2, k2, kRkB4, k4), rhoY);
+          if (adaptive) {
+            double dy = hs * fma(kRkE4, k4, dot3(kRkE1, k1, kRkE2, k2, kRkE3, k3));
+            dy /= fma(rtol, rn, atol);
+            double err = 0;
+#pragma unroll
+            for (int l = 0; l < NS; ++l) {
+              const double d = bcast(dy, l);
+              err = fma(d, d, err);
+            }
+            err = sqrt(err / NS);
+            double hstar = hs;
+            if (steps > 0)
+              hstar *= fmin(5.0, fmax(0.2, 0.8 * pow(err_last, 0.1) * pow(err + 1e-20, -0.175)));
+            else if (err > 1)
+              hstar *= 0.2;
+            if (err <= 1) {
+              rhoY = rn;
+              time += hs;
+              err_last = err;
+            } else {
+              accepted = false;
+              ++rejected;
+            }
+            h = hstar;
+          } else {
+            rhoY = rn;
+            time += hs;
+          }
+          y = div_rcp(rhoY, rho, rrho);
+        }
+      } else if (scheme == 3) {
+        if (stage == 0) {
+          rn = fma(o, h, rhoY);
+        } else if (stage == 1) {
+          rn = dot2(0.75, rhoY, 0.25, fma(o, h, rn));
+        } else {
+          rhoY = div_by<3>(fma(2.0, fma(o, h, rn), rhoY));
+          if (rhoY < 0) rhoY = 0;
+          rn = rhoY;
+          time += h;
+        }
+        y = div_rcp(rn, rho, rrho);
       } else {
 #pragma unroll
-        for (int l = 0; l < NS; ++l) {
-          rhoY[l] += hs * (kRkB1 * k1[l] + kRkB2 * k2[l] + kRkB4 * k4[l]);
-          yk[l] = rhoY[l] / rho;
+        for (int k = 0; k < RP; ++k) {
+          const int row = row0 + k * G;
+          if (lane < NS * G && row < NS) L.a[row * NS + col] = zz[k];
         }
-        time += hs;
-      }
-    } else if (scheme == 3) {
-      double rn[NS], ys[NS], imw = 0;
-      wave_source<M, false>(tb, L, rho, t, yk, omega);
-#pragma unroll
-      for (int l = 0; l < NS; ++l) {
-        rn[l] = rhoY[l] + omega[l] * h;
-        ys[l] = rn[l] / rho;
-        imw += ys[l] * tb->imw[l];
-      }
-      double ts = wave_temperature<M>(tb, L, t, imw, ys, e);
-      wave_source<M, false>(tb, L, rho, ts, ys, omega);
-      imw = 0;
-#pragma unroll
-      for (int l = 0; l < NS; ++l) {
-        rn[l] = 0.75 * rhoY[l] + 0.25 * (rn[l] + omega[l] * h);
-        ys[l] = rn[l] / rho;
-        imw += ys[l] * tb->imw[l];
-      }
-      ts = wave_temperature<M>(tb, L, ts, imw, ys, e);
-      wave_source<M, false>(tb, L, rho, ts, ys, omega);
-#pragma unroll
-      for (int l = 0; l < NS; ++l) {
-        rhoY[l] = (rhoY[l] + 2.0 * (rn[l] + omega[l] * h)) / 3.0;
-        if (rhoY[l] < 0) rhoY[l] = 0;
-        yk[l] = rhoY[l] / rho;
-      }
-      time += h;
-    } else {
-      wave_source<M, true>(tb, L, rho, t, yk, omega);
-#pragma unroll
-      for (int m = 0; m < NS; ++m) {
-        const double jmm = rhoY[m] > 1e-30 ? L.a[m * NS + m] / rhoY[m] * 1e+3 / tb->imw[m] : 0.0;
-        omega[m] /= 1 - h * jmm;
-      }
-      __syncthreads();  // the diagonal is read before the next step's Jacobian overwrites it
-      double sum = 0;
-#pragma unroll
-      for (int l = 0; l < NS; ++l) {
-        rhoY[l] += omega[l] * h;
-        if (rhoY[l] < 0) rhoY[l] = 0;
-        sum += rhoY[l];
-      }
-#pragma unroll
-      for (int l = 0; l < NS; ++l) {
+        __syncthreads();
+        const double jmm = rhoY > 1e-30 ? L.a[sl * NS + sl] / rhoY * 1e+3 / K.imw : 0.0;
+        __syncthreads();
+        rhoY = fma(o / fma(-h, jmm, 1.0), h, rhoY);
+        if (rhoY < 0) rhoY = 0;
         if (conserve) {
-          yk[l] = rhoY[l] / sum;
-          rhoY[l] = yk[l] * rho;
+          double sum = 0;
+#pragma unroll
+          for (int l = 0; l < NS; ++l) sum += bcast(rhoY, l);
+          y = rhoY / sum;
+          rhoY = y * rho;
         } else {
-          yk[l] = rhoY[l] / rho;
+          y = div_rcp(rhoY, rho, rrho);
         }
+        time += h;
       }
-      time += h;
+      if (!accepted) break;
+      ts = wave_temperature<M>(tb, K, L, stage == last ? t : ts, wave_imw<M>(tb, y), y, e);
     }
     if (!accepted) continue;
-    double imw = 0;
-#pragma unroll
-    for (int l = 0; l < NS; ++l) imw += yk[l] * tb->imw[l];
-    t = wave_temperature<M>(tb, L, t, imw, yk, e);
+    t = ts;
     ++steps;
   }
+  if (!fail) fail = wave_fault<NS>(t, time, h, t_end, rhoY, steps + rejected, step_cap);
+  if (lane < NS) P.rhoY[lane * cap + s] = rhoY;
   if (lane != 0) return;
-#pragma unroll
-  for (int l = 0; l < NS; ++l) P.rhoY[l * cap + s] = rhoY[l];
   P.t[s] = t;
   P.time[s] = time;
   P.h[s] = h;
   P.err_last[s] = err_last;
   P.steps[s] = steps;
   P.rejected[s] = rejected;
-  if (!fail) fail = reactor_fault<NS>(t, time, h, t_end, rhoY, steps + rejected, step_cap);
   if (fail)
     P.status[s] = kSlotFailed + fail;
   else if (time >= t_end)

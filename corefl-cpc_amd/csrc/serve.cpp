@@ -53,6 +53,9 @@ int sfail(corefl_server *s, Status st, const std::string &m) {
     if (e_ != hipSuccess) return sfail(srv, Status::Hip, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
+// a slot's status: done, or failed for a reason
+bool finished(int st) { return st == 2 || st > corefl::kSlotFailed; }
+
 template <class T>
 hipError_t dalloc(corefl_server *s, T *&p, size_t n) {
   void *q = nullptr;
@@ -195,18 +198,24 @@ int corefl_serve_progress(corefl_server *s, int *pending) {
       SHIP(s, corefl::launch_reactors(P, s->model, s->d_tables, s->steps_per_launch, s->stream));
     const size_t n = s->high_water;
     SHIP(s, hipMemcpyAsync(s->h_status, P.status, n * sizeof(int), hipMemcpyDeviceToHost, s->stream));
-    SHIP(s, hipMemcpyAsync(s->h_t, P.t, n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    SHIP(s, hipMemcpyAsync(s->h_time, P.time, n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    SHIP(s, hipMemcpyAsync(s->h_rho, P.rho, n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    SHIP(s, hipMemcpyAsync(s->h_steps, P.steps, n * sizeof(long), hipMemcpyDeviceToHost, s->stream));
-    SHIP(s, hipMemcpyAsync(s->h_rejected, P.rejected, n * sizeof(long), hipMemcpyDeviceToHost, s->stream));
-    for (int l = 0; l < s->ns; ++l)
-      SHIP(s, hipMemcpyAsync(s->h_rhoY + static_cast<size_t>(l) * P.cap, P.rhoY + static_cast<size_t>(l) * P.cap,
-                             n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
     SHIP(s, hipStreamSynchronize(s->stream));
+    // most calls finish no request: the results come over only when a status says that there is one
+    bool any = false;
+    for (int i = 0; i < s->high_water && !any; ++i) any = s->slot_ticket[i] >= 0 && finished(s->h_status[i]);
+    if (any) {
+      SHIP(s, hipMemcpyAsync(s->h_t, P.t, n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+      SHIP(s, hipMemcpyAsync(s->h_time, P.time, n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+      SHIP(s, hipMemcpyAsync(s->h_rho, P.rho, n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+      SHIP(s, hipMemcpyAsync(s->h_steps, P.steps, n * sizeof(long), hipMemcpyDeviceToHost, s->stream));
+      SHIP(s, hipMemcpyAsync(s->h_rejected, P.rejected, n * sizeof(long), hipMemcpyDeviceToHost, s->stream));
+      for (int l = 0; l < s->ns; ++l)
+        SHIP(s, hipMemcpyAsync(s->h_rhoY + static_cast<size_t>(l) * P.cap, P.rhoY + static_cast<size_t>(l) * P.cap,
+                               n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+      SHIP(s, hipStreamSynchronize(s->stream));
+    }
     for (int i = 0; i < s->high_water; ++i) {
       const int st = s->h_status[i];
-      if (s->slot_ticket[i] < 0 || (st != 2 && st <= corefl::kSlotFailed)) continue;
+      if (s->slot_ticket[i] < 0 || !finished(st)) continue;
       corefl_reactor_result r{};
       if (st > corefl::kSlotFailed) {
         r.status = static_cast<int>(Status::State);

@@ -3,7 +3,7 @@ both sides of each rule and at ragged ends of its tiles."""
 import numpy as np
 import pytest
 
-from corefl_amd import Solver, _abi, channel_case, load_tables
+from corefl_amd import ReactorServer, Solver, _abi, channel_case, h2_air_mass_fractions, load_tables
 from oracle import Oracle
 
 pytestmark = pytest.mark.gpu
@@ -43,6 +43,48 @@ def test_viscous_column_splits(tables, h2_oracle_tables, mx, my, mz):
     o.op("zero_dq")
     s.op(_abi.OP_VISCOUS)
     o.op("viscous")
-    err = normwise(s.download(0, _abi.F_DQ), o.a["dq"])
-    assert np.all(err <= STAGE_TOL), err
+    gpu, ref = s.download(0, _abi.F_DQ), o.a["dq"]
     s.close()
+    err = normwise(gpu, ref)
+    # a species whose own gradients are far below Y / dx (fine grids) is dominated by the rounding of Y and of
+    # the other species' fluxes in its correction velocity, two derivatives of J |grad xi| each: bound it by
+    # 64 roundings of that size beside the relative tolerance
+    m, rho_d, y = o.a["metric"], o.a["rhoD"], o.a["sv"]
+    k2 = max((o.a["jac"] * (m[3 * d:3 * d + 3] ** 2).sum(axis=0)).max() for d in range(3))
+    top = [float((rho_d[l] * y[l]).max()) for l in range(9)]
+    for l in range(9):
+        bound = 64 * 2.2e-16 * k2 * (top[l] + y[l].max() * sum(top))
+        worst = np.abs(gpu[5 + l] - ref[5 + l]).max()
+        assert worst <= STAGE_TOL * np.abs(ref[5 + l]).max() + bound, (l, worst, bound)
+    assert np.all(err[:5] <= STAGE_TOL), err
+
+
+def test_reactor_result_across_the_kernel_switch(tables):
+    """Above 16,384 slots in flight a reactor has a lane, below a wave: 16,500 requests start on the first,
+    and once the short ones are done the others finish on the second, bit for bit as they do alone."""
+    mw = np.array(tables.mw[:9])
+    n = 16500
+
+    def request(i):
+        r = np.random.default_rng(i)
+        return dict(temperature=r.uniform(1000.0, 1600.0), pressure=r.uniform(1.0, 10.0) * 101325.0,
+                    y=h2_air_mass_fractions(r.uniform(0.5, 2.0), mw), t_end=2e-5 if i % 16 == 0 else 2e-7, dt=1e-8)
+
+    pick = [0, 16 * 500, 16400]
+    alone = {}
+    for i in pick:
+        srv = ReactorServer(tables, budget_bytes=1 << 20, steps_per_launch=16)
+        t = srv.submit(**request(i))
+        alone[i] = srv.run_until_done([t])[t]
+        srv.close()
+    srv = ReactorServer(tables, budget_bytes=32 << 20, steps_per_launch=16)
+    assert srv.capacity >= n
+    tickets = [srv.submit(**request(i)) for i in range(n)]
+    while srv.progress():
+        pass
+    res = srv.drain(n)
+    srv.close()
+    for i in pick:
+        r = res[tickets[i]]
+        assert r["status"] == 0 and r["steps"] == alone[i]["steps"]
+        assert r["temperature"] == alone[i]["temperature"] and np.array_equal(r["y"], alone[i]["y"])

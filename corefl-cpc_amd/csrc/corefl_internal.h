@@ -182,6 +182,9 @@ hipError_t launch_copy(double *dst, const double *src, long n, hipStream_t s);
 hipError_t launch_scaled_copy(double *dst, const double *src, double a, long n, hipStream_t s);
 hipError_t launch_cv_from_bv(const Zone &z, const Run &r, const Tab *tb, hipStream_t s);
 hipError_t launch_properties(const Zone &z, const Run &r, const Tab *tb, hipStream_t s);
+// the end of a stage on a 2-D block: properties of plane k = 0 and, with planes, the ghost planes' state and
+// properties (launch_k_gradient followed by launch_properties)
+hipError_t launch_close_2d(const Zone &z, const Run &r, const Tab *tb, bool planes, hipStream_t s);
 // save_qn: the first stage of a recorded step, whose cv is the step's start state, saves qn itself
 hipError_t launch_update_rk(const Zone &z, const Run &r, const Tab *tb, double dt, int rk, hipStream_t s,
                             const double *dtp = nullptr, const double *dtc = nullptr, bool save_qn = false);
@@ -214,9 +217,11 @@ hipError_t launch_viscous_flux(const Zone &z, const Run &r, const Tab *tb, hipSt
 // store: replace dq instead of adding to it (the stage's first contribution, dq not cleared before)
 hipError_t launch_viscous_derivative(const Zone &z, const Run &r, hipStream_t s, bool store = false);
 // 2nd-order face scheme, all directions (flux faces in fFlux, then the difference)
-hipError_t launch_viscous2(const Zone &z, const Run &r, const Tab *tb, hipStream_t s);
+// (flat: stages after the first of a 2-D step whose ghost planes follow at its end)
+hipError_t launch_viscous2(const Zone &z, const Run &r, const Tab *tb, hipStream_t s, bool flat = false);
 hipError_t launch_periodic_flux(const Zone &z, const Run &r, const corefl_boundary &b, hipStream_t s);
-hipError_t launch_bc_outflow(const Zone &z, const Run &r, const Tab *tb, const corefl_boundary &b, hipStream_t s);
+hipError_t launch_bc_outflow(const Zone &z, const Run &r, const Tab *tb, const corefl_boundary *b, int n_faces,
+                             hipStream_t s);
 hipError_t launch_bc_periodic(const Zone &z, const Run &r, const Tab *tb, const corefl_boundary &b, hipStream_t s);
 // both periodic faces of one axis in one launch (lo: the face at index 0 of the axis); the same result as the
 // two faces' launches in sequence when the block holds at least 2 ngg + 1 nodes along the axis

@@ -37,6 +37,7 @@ struct corefl_ctx {
   struct Block {
     corefl::Zone z{};
     std::vector<Face> faces;
+    std::vector<corefl_boundary> outflow;  // the outflow faces, launched together
     std::vector<corefl::InnerDev> inner;
     std::vector<void *> allocs;
     int shape[3] = {0, 0, 0};  // tile shape of each direction's characteristic WENO sweep
@@ -275,8 +276,8 @@ int op_block(corefl_ctx *c, int op, corefl_ctx::Block &b, int rk, double dt) {
     case COREFL_OP_BC:
       // apply_boundary_conditions in its priority order (src/BoundCond.cu:3846-3997):
       // outflow, inflow, symmetry, wall, periodic; within a kind, faces in block order
-      for (const auto &f : b.faces)
-        if (f.kind == COREFL_BC_OUTFLOW) HIP_TRY(c, launch_bc_outflow(z, r, c->d_tables, f.b, s));
+      if (!b.outflow.empty())
+        HIP_TRY(c, launch_bc_outflow(z, r, c->d_tables, b.outflow.data(), static_cast<int>(b.outflow.size()), s));
       for (const auto &f : b.faces)
         if (f.kind == COREFL_BC_INFLOW) HIP_TRY(c, launch_bc_inflow(z, r, c->d_tables, f.b, f.cond, s));
       for (const auto &f : b.faces)
@@ -373,6 +374,19 @@ int check_inner(corefl_ctx *c) {
   return 0;
 }
 
+// The end of a stage on one block: eliminate_k_gradient (2-D) and the properties.  planes: also a 2-D
+// block's ghost planes (else they keep the step's start until its last stage).
+int close_block(corefl_ctx *c, corefl_ctx::Block &b, bool planes) {
+  if (b.z.mz != 1) return op_block(c, COREFL_OP_PROPERTIES, b, 0, 0);
+  OpTimer timer(c, COREFL_OP_PROPERTIES);
+  HIP_TRY(c, launch_close_2d(b.z, c->run, c->d_tables, planes, c->cur ? c->cur : c->stream));
+  return 0;
+}
+
+// Whether a stage inside a step leaves a 2-D block's ghost planes complete: the last one does; the 8th-order
+// viscous terms read them in every stage (the 2nd-order ones only as differences that are 0).
+bool stage_fills_planes(const Run &r, int rk) { return rk == 2 || r.viscous_order == 8; }
+
 // data_communication: inner faces of every block in block and face order,
 // src/DataCommunication.cu:6-35
 int halo_all(corefl_ctx *c) {
@@ -388,12 +402,12 @@ int halo_all(corefl_ctx *c) {
 // fluxes on every block, exchange_value(task 1) over inner faces of every
 // block then periodic faces of every block (src/DataCommunication.cu:437-485),
 // then the derivative on every block.
-int viscous_all(corefl_ctx *c) {
+int viscous_all(corefl_ctx *c, bool flat = false) {
   OpTimer timer(c, COREFL_OP_VISCOUS);
   const Run &r = c->run;
   hipStream_t s = c->stream;
   if (r.viscous_order == 2) {
-    for (auto &b : c->blocks) HIP_TRY(c, launch_viscous2(b.z, r, c->d_tables, s));
+    for (auto &b : c->blocks) HIP_TRY(c, launch_viscous2(b.z, r, c->d_tables, s, flat && b.z.mz == 1));
     return 0;
   }
   if (r.viscous_order != 8) return 0;
@@ -482,7 +496,7 @@ int record_stage(corefl_ctx *c, int rk) {
   };
   auto viscous_head = [&](corefl_ctx::Block &b) -> int {
     hipStream_t s = c->cur;
-    if (r.viscous_order == 2) HIP_TRY(c, launch_viscous2(b.z, r, c->d_tables, s));
+    if (r.viscous_order == 2) HIP_TRY(c, launch_viscous2(b.z, r, c->d_tables, s, rk > 0 && b.z.mz == 1));
     if (visc8) HIP_TRY(c, launch_viscous_flux(b.z, r, c->d_tables, s));
     return 0;
   };
@@ -501,7 +515,7 @@ int record_stage(corefl_ctx *c, int rk) {
     return ops(b, {COREFL_OP_CHEMISTRY, COREFL_OP_INVISCID_X, COREFL_OP_INVISCID_Y, COREFL_OP_INVISCID_Z,
                    COREFL_OP_UPDATE_RK, COREFL_OP_LIMIT_FLOW, COREFL_OP_BC});
   };
-  auto closing = [&](corefl_ctx::Block &b) -> int { return ops(b, {COREFL_OP_K_GRADIENT, COREFL_OP_PROPERTIES}); };
+  auto closing = [&](corefl_ctx::Block &b) -> int { return close_block(c, b, stage_fills_planes(r, rk)); };
   if (inner && c->batched) {
     // the same stage with the block-local pointwise operators and the outflow faces of all blocks in one
     // launch each (blocks are independent between the flux exchange and the halo, so this is the
@@ -631,7 +645,7 @@ int upload_block_tables(corefl_ctx *c) {
       out.push_back(it);
       long n = 1;
       for (int d = 0; d < 3; ++d) n *= f.b.range_end[d] - f.b.range_start[d] + 1;
-      c->mb_face = std::max(c->mb_face, n);
+      c->mb_face = std::max(c->mb_face, n * z.ngg);
     }
   }
   HIP_TRY(c, hipMalloc(&c->d_zones, nb * sizeof(Zone)));
@@ -725,7 +739,7 @@ int clear_state_flag(corefl_ctx *c) {
   return 0;
 }
 
-int run_stage(corefl_ctx *c, int rk, double dt);
+int run_stage(corefl_ctx *c, int rk, double dt, bool in_step = false);
 int run_step(corefl_ctx *c, double *dt_inout);
 
 }  // namespace
@@ -1136,6 +1150,7 @@ int corefl_block_add(corefl_ctx *c, const corefl_block_desc *d, int *block_id) {
     if (bf.range_start[bf.face] != at || bf.range_end[bf.face] != at)
       return fail(c, Status::Arg, "boundary face does not lie on the block face");
     b.faces.push_back(face);
+    if (face.kind == COREFL_BC_OUTFLOW) b.outflow.push_back(bf);
   }
   if (d->n_inner < 0 || (d->n_inner > 0 && !d->inner)) return fail(c, Status::Arg, "bad inner face list");
   for (int f = 0; f < d->n_inner; ++f) {
@@ -1428,10 +1443,11 @@ int wu_step(corefl_ctx *c, double *dt_inout) {
   return 0;
 }
 
-int run_stage(corefl_ctx *c, int rk, double dt) {
+// in_step: a stage of corefl_step, whose state is seen after the last one only
+int run_stage(corefl_ctx *c, int rk, double dt, bool in_step) {
   int st;
   if ((st = op_all(c, COREFL_OP_ZERO_DQ, rk, dt))) return st;
-  if ((st = op_all(c, COREFL_OP_VISCOUS, rk, dt))) return st;
+  if ((st = viscous_all(c, in_step && rk > 0))) return st;
   for (auto &b : c->blocks) {
     if ((st = op_block(c, COREFL_OP_CHEMISTRY, b, rk, dt))) return st;
     if ((st = op_block(c, COREFL_OP_INVISCID_X, b, rk, dt))) return st;
@@ -1442,8 +1458,8 @@ int run_stage(corefl_ctx *c, int rk, double dt) {
     if ((st = op_block(c, COREFL_OP_BC, b, rk, dt))) return st;
   }
   if ((st = op_all(c, COREFL_OP_HALO, rk, dt))) return st;
-  if ((st = op_all(c, COREFL_OP_K_GRADIENT, rk, dt))) return st;
-  if ((st = op_all(c, COREFL_OP_PROPERTIES, rk, dt))) return st;
+  for (auto &b : c->blocks)
+    if ((st = close_block(c, b, !in_step || stage_fills_planes(c->run, rk)))) return st;
   return 0;
 }
 
@@ -1475,7 +1491,7 @@ int run_step(corefl_ctx *c, double *dt_inout) {
     if (!(dt > 0) || !std::isfinite(dt)) return fail(c, Status::State, "non-positive or non-finite CFL time step");
   }
   for (int rk = 0; rk < 3; ++rk)
-    if ((st = run_stage(c, rk, dt))) return st;
+    if ((st = run_stage(c, rk, dt, true))) return st;
   *dt_inout = dt;
   return 0;
 }

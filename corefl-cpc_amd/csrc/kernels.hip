@@ -775,62 +775,143 @@ DEV void transport(const Tab *__restrict__ tb, double temperature, double mw_tot
 
 // update_physical_properties (1T) over the padded extent, src/FieldOperation.cuh:183-247
 template <int M>
-DEV void properties_point(const Zone &z, const Tab *__restrict__ tb, int transport_ghosts, long t) {
+struct PointProps {
+  static constexpr int NS = kNs(M) > 0 ? kNs(M) : 1;
+  double gam, c, mach, mul, kap, kappa_ve, cpt, y[NS], rd[NS];
+};
+
+template <int M>
+DEV void properties_eval(const Zone &z, const Tab *__restrict__ tb, long p, bool with_transport, PointProps<M> &P) {
   [[maybe_unused]] constexpr int NS = kNs(M);
-  int i, j, k;
-  padded_ijk(z, t, i, j, k);
-  const long p = z.ix(i, j, k), sz = z.sz;
+  const long sz = z.sz;
   const double T = z.bv[p + 5 * sz];
   const double V = norm3(z.bv[p + sz], z.bv[p + 2 * sz], z.bv[p + 3 * sz]);
   if constexpr (NS > 0) {
-    double cp[NS], y[NS];
+    double cp[NS];
     thermo_cp<M>(tb, T, cp);
     double imw = 0, cpt = 0;
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      y[l] = z.sv[p + l * sz];
-      imw = fma(y[l], tb->imw[l], imw);
-      cpt = fma(y[l], cp[l], cpt);
+      P.y[l] = z.sv[p + l * sz];
+      imw = fma(P.y[l], tb->imw[l], imw);
+      cpt = fma(P.y[l], cp[l], cpt);
     }
+    P.cpt = cpt;
     const double mw = 1 / fmax(imw, 1e-12);
     const double R = kRu * imw;
     if constexpr (kTT(M)) {
       // translational-rotational gamma and sound speed, src/FieldOperation.cuh:207-229
       double cv_tr, cpm, rm;
-      mix_tr_energy<M>(tb, T, y, cv_tr, cpm, rm);
-      const double gam = cpm / fmax(cv_tr, 1e-8);
-      z.gam[p] = gam;
-      const double c = sqrt(fmax(gam * rm * T, 1e-12));
-      z.acoustic[p] = c;
-      z.mach[p] = V / c;
+      mix_tr_energy<M>(tb, T, P.y, cv_tr, cpm, rm);
+      P.gam = cpm / fmax(cv_tr, 1e-8);
+      P.c = sqrt(fmax(P.gam * rm * T, 1e-12));
+      P.mach = V / P.c;
       if (z.tve[p] <= 0) z.tve[p] = T;
     } else {
-      const double gam = cpt / (cpt - R);
-      z.gam[p] = gam;
-      const double c = sqrt(gam * R * T);
-      z.acoustic[p] = c;
-      z.mach[p] = V / c;
+      P.gam = cpt / (cpt - R);
+      P.c = sqrt(P.gam * R * T);
+      P.mach = V / P.c;
     }
-    // The 8th-order viscous fluxes and the time-step bound read mu, kappa
-    // and rho*D at interior nodes only; the 2nd-order face scheme also reads
-    // them one node outside, so there the padded extent is covered.
-    if (transport_ghosts || (i >= 0 && i < z.mx && j >= 0 && j < z.my && k >= 0 && k < z.mz)) {
-      double rd[NS], mul, kap;
-      transport<M>(tb, T, mw, y, cp, mul, kap, rd);
-      z.mul[p] = mul;
-      z.kappa[p] = kap;
+    if (with_transport) {
+      transport<M>(tb, T, mw, P.y, cp, P.mul, P.kap, P.rd);
       if constexpr (kTT(M)) {
         double cv_ve = 0.0;
-        mix_ve_energy<M>(tb, z.tve[p], y, &cv_ve);
-        z.kappa_ve[p] = kap * cv_ve / fmax(cpt, 1e-8);
+        mix_ve_energy<M>(tb, z.tve[p], P.y, &cv_ve);
+        P.kappa_ve = P.kap * cv_ve / fmax(cpt, 1e-8);
       }
-#pragma unroll
-      for (int l = 0; l < NS; ++l) z.rhoD[p + l * sz] = rd[l];
     }
   } else {
     constexpr double c_temp = kGammaAir * kRu / kMwAir;
-    z.mul[p] = sutherland(T);
-    z.mach[p] = V / sqrt(c_temp * T);
+    P.mul = sutherland(T);
+    P.mach = V / sqrt(c_temp * T);
+  }
+}
+
+template <int M>
+DEV void properties_store(const Zone &z, long p, bool with_transport, const PointProps<M> &P) {
+  [[maybe_unused]] constexpr int NS = kNs(M);
+  z.mach[p] = P.mach;
+  if constexpr (NS > 0) {
+    z.gam[p] = P.gam;
+    z.acoustic[p] = P.c;
+    if (with_transport) {
+      z.mul[p] = P.mul;
+      z.kappa[p] = P.kap;
+      if constexpr (kTT(M)) z.kappa_ve[p] = P.kappa_ve;
+#pragma unroll
+      for (int l = 0; l < NS; ++l) z.rhoD[p + l * z.sz] = P.rd[l];
+    }
+  } else {
+    z.mul[p] = P.mul;
+  }
+}
+
+// The 8th-order viscous fluxes and the time-step bound read mu, kappa and
+// rho*D at interior nodes only; the 2nd-order face scheme also reads them one
+// node outside, so there (transport_ghosts) the padded extent is covered.
+template <int M>
+DEV void properties_point(const Zone &z, const Tab *__restrict__ tb, int transport_ghosts, long t) {
+  int i, j, k;
+  padded_ijk(z, t, i, j, k);
+  const long p = z.ix(i, j, k);
+  const bool tr = transport_ghosts || (i >= 0 && i < z.mx && j >= 0 && j < z.my && k >= 0 && k < z.mz);
+  PointProps<M> P;
+  properties_eval<M>(z, tb, p, tr, P);
+  properties_store<M>(z, p, tr, P);
+}
+
+// A 2-D block's plane k = 0 closes a stage for its ghost planes too: the
+// elimination of the k gradient (k_k_gradient) gives them the plane's state, so
+// their properties are the plane's and are stored, not evaluated, for all of
+// them (with ngg = 3 that is six of seven planes; 1024x512 two-temperature air:
+// 920 + 182 us a stage -> 145 us, 395 us in the stage that fills the planes).  Tve is the one input that stays the ghost planes' own.
+// planes 0: plane 0 only (the ghost planes follow at the step's end).
+template <int M>
+__global__ __launch_bounds__(kBlock) void k_close_2d(Zone z, const Tab *__restrict__ tb, int transport_ghosts,
+                                                     int planes, long n) {
+  const long t = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
+  if (t >= n) return;
+  const int nxp = z.mx + 2 * z.ngg;
+  const int i = static_cast<int>(t % nxp) - z.ngg, j = static_cast<int>(t / nxp) - z.ngg;
+  const long p = z.ix(i, j, 0), sz = z.sz;
+  const bool tr = transport_ghosts || (i >= 0 && i < z.mx && j >= 0 && j < z.my);
+  PointProps<M> P;
+  properties_eval<M>(z, tb, p, tr, P);
+  properties_store<M>(z, p, tr, P);
+  if (!planes) return;
+  double b6[6], cv[kNv(M)], sc[kNsc(M) > 0 ? kNsc(M) : 1];
+#pragma unroll
+  for (int l = 0; l < 6; ++l) b6[l] = z.bv[p + l * sz];
+#pragma unroll
+  for (int l = 0; l < kNsc(M); ++l) sc[l] = z.sv[p + l * sz];
+#pragma unroll
+  for (int l = 0; l < kNv(M); ++l) cv[l] = z.cv[p + l * sz];
+  [[maybe_unused]] double tve = kTT(M) ? z.tve[p] : 0.0;
+  // Air stores its viscosity on every plane; a mixture's transport reaches the ghost planes only where
+  // transport_ghosts asks for it
+  for (int m = 0; m < 2 * z.ngg; ++m) {
+    const int k = m < z.ngg ? m - z.ngg : m - z.ngg + 1;
+    const long pg = z.ix(i, j, k);
+#pragma unroll
+    for (int l = 0; l < 6; ++l) z.bv[pg + l * sz] = b6[l];
+#pragma unroll
+    for (int l = 0; l < kNsc(M); ++l) z.sv[pg + l * sz] = sc[l];
+#pragma unroll
+    for (int l = 0; l < kNv(M); ++l) z.cv[pg + l * sz] = cv[l];
+    if constexpr (kTT(M)) {
+      double tg = z.tve[pg];
+      if (tg <= 0) {
+        tg = b6[5];
+        z.tve[pg] = tg;
+      }
+      if (transport_ghosts && tg != tve) {
+        double cv_ve = 0.0;
+        mix_ve_energy<M>(tb, tg, P.y, &cv_ve);
+        P.kappa_ve = P.kap * cv_ve / fmax(P.cpt, 1e-8);
+        tve = tg;
+      }
+    }
+    properties_store<M>(z, pg, transport_ghosts != 0, P);
   }
 }
 
@@ -4002,9 +4083,11 @@ __global__ __launch_bounds__(kBlock) void k_viscous_derivative(Zone z, int nv, i
 // differences across the face and four-point central differences along the
 // other axes, with face-averaged mu, kappa, rho*D, metrics and J grad(DIR).
 // One thread per face (faces -1 .. n-1 along DIR); fFlux holds the faces.
+// flat: a later stage of a 2-D step, whose ghost planes are refreshed at its end;
+// the two planes beside k = 0 hold equal states, so the k differences are 0.
 template <int M, int DIR>
 __global__ __launch_bounds__(kBlock) void k_visc2_flux(Zone z, const Tab *__restrict__ tb, double prandtl, int gradp,
-                                                      long n) {
+                                                      int flat, long n) {
   [[maybe_unused]] constexpr int NS = kNs(M);
   const long t = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
   if (t >= n) return;
@@ -4026,6 +4109,7 @@ __global__ __launch_bounds__(kBlock) void k_visc2_flux(Zone z, const Tab *__rest
   auto dd = [&](const double *arr, int l, int a) {
     const long o = static_cast<long>(l) * sz;
     if (a == DIR) return arr[pe + o] - arr[p + o];
+    if (a == 2 && flat && arr != z.tve) return 0.0;
     return 0.25 * (arr[p + st[a] + o] - arr[p - st[a] + o] + arr[pe + st[a] + o] - arr[pe - st[a] + o]);
   };
   auto grad = [&](const double *arr, int l, double &gx, double &gy, double &gz) {
@@ -4141,20 +4225,20 @@ __global__ __launch_bounds__(kBlock) void k_visc2_diff(Zone z, long n) {
 }
 
 // One thread per (face point, layer) of a boundary face; layer 0 is the face
-// node itself, layers 1..g its ghosts.  On i-faces the layer index runs
+// node itself, layers 1..g its ghosts (first: the first layer taken, 0 or 1).  On i-faces the layer index runs
 // fastest so that neighbouring lanes touch neighbouring addresses; on j/k
 // faces i runs fastest.
 struct FaceSite {
   int i, j, k, layer;
 };
-DEV bool face_site(const Zone &z, const corefl_boundary &b, long t, FaceSite &f) {
+DEV bool face_site(const Zone &z, const corefl_boundary &b, long t, FaceSite &f, int first = 0) {
   const int n0 = b.range_end[0] - b.range_start[0] + 1, n1 = b.range_end[1] - b.range_start[1] + 1;
   const int n2 = b.range_end[2] - b.range_start[2] + 1;
-  const int nl = z.ngg + 1;
+  const int nl = z.ngg + 1 - first;
   if (t >= static_cast<long>(n0) * n1 * n2 * nl) return false;
   int a0, a1, a2;
   if (b.face == 0) {
-    f.layer = static_cast<int>(t % nl);
+    f.layer = first + static_cast<int>(t % nl);
     const long r = t / nl;
     a0 = 0;
     a1 = static_cast<int>(r % n1);
@@ -4164,7 +4248,7 @@ DEV bool face_site(const Zone &z, const corefl_boundary &b, long t, FaceSite &f)
     const long r = t / n0;
     const int nm = b.face == 1 ? n2 : n1;  // the other tangential extent
     const int o = static_cast<int>(r % nm);
-    f.layer = static_cast<int>(r / nm);
+    f.layer = first + static_cast<int>(r / nm);
     a1 = b.face == 1 ? 0 : o;
     a2 = b.face == 1 ? o : 0;
   }
@@ -4312,34 +4396,20 @@ DEV void bc_outflow_layer(const Zone &z, const Tab *__restrict__ tb, int i, int 
   cv_from_bv_point<M>(z, tb, pg);
 }
 
+// The outflow faces of a block in one launch (blockIdx.y = face): a face writes
+// only ghost nodes beyond itself and reads only its own nodes.
+constexpr int kFaceSet = 8;
+struct FaceSet {
+  corefl_boundary b[kFaceSet];
+};
 template <int M>
-DEV void bc_outflow_point(const Zone &z, const Tab *__restrict__ tb, int i, int j, int k, const int *d) {
-  for (int g = 1; g <= z.ngg; ++g) bc_outflow_layer<M>(z, tb, i, j, k, d, g);
-}
-
-template <int M>
-__global__ void k_bc_outflow(Zone z, const Tab *__restrict__ tb, corefl_boundary b) {
-  const int n0 = b.range_end[0] - b.range_start[0] + 1, n1 = b.range_end[1] - b.range_start[1] + 1;
-  const int n2 = b.range_end[2] - b.range_start[2] + 1;
-  const long t = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-  if (t >= static_cast<long>(n0) * n1 * n2) return;
-  const int i = b.range_start[0] + static_cast<int>(t % n0);
-  const int j = b.range_start[1] + static_cast<int>((t / n0) % n1);
-  const int k = b.range_start[2] + static_cast<int>(t / (static_cast<long>(n0) * n1));
+__global__ __launch_bounds__(kFaceBlock) void k_bc_outflow(Zone z, const Tab *__restrict__ tb, FaceSet faces) {
+  const corefl_boundary &b = faces.b[blockIdx.y];
+  FaceSite f;
+  if (!face_site(z, b, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, f, 1)) return;
   int d[3] = {0, 0, 0};
   d[b.face] = b.direction;
-  bc_outflow_point<M>(z, tb, i, j, k, d);
-}
-
-// Face point t of a boundary face (i fastest).
-DEV bool face_point(const corefl_boundary &b, long t, int &i, int &j, int &k) {
-  const int n0 = b.range_end[0] - b.range_start[0] + 1, n1 = b.range_end[1] - b.range_start[1] + 1;
-  const int n2 = b.range_end[2] - b.range_start[2] + 1;
-  if (t >= static_cast<long>(n0) * n1 * n2) return false;
-  i = b.range_start[0] + static_cast<int>(t % n0);
-  j = b.range_start[1] + static_cast<int>((t / n0) % n1);
-  k = b.range_start[2] + static_cast<int>(t / (static_cast<long>(n0) * n1));
-  return true;
+  bc_outflow_layer<M>(z, tb, f.i, f.j, f.k, d, f.layer);
 }
 
 template <int M>
@@ -4406,17 +4476,12 @@ DEV void bc_symmetry_layer(const Zone &z, const Tab *__restrict__ tb, int i, int
 }
 
 // The face node (layer 0) and the ghost layers read only interior nodes, so
-// they are independent of each other.
+// they are independent of each other: a thread per site and layer.
 template <int M>
-DEV void bc_symmetry_point(const Zone &z, const Tab *__restrict__ tb, int i, int j, int k, int face, int direction) {
-  for (int layer = 0; layer <= z.ngg; ++layer) bc_symmetry_layer<M>(z, tb, i, j, k, face, direction, layer);
-}
-
-template <int M>
-__global__ void k_bc_symmetry(Zone z, const Tab *__restrict__ tb, corefl_boundary b) {
-  int i, j, k;
-  if (!face_point(b, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, i, j, k)) return;
-  bc_symmetry_point<M>(z, tb, i, j, k, b.face, b.direction);
+__global__ __launch_bounds__(kFaceBlock) void k_bc_symmetry(Zone z, const Tab *__restrict__ tb, corefl_boundary b) {
+  FaceSite f;
+  if (!face_site(z, b, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, f)) return;
+  bc_symmetry_layer<M>(z, tb, f.i, f.j, f.k, b.face, b.direction, f.layer);
 }
 
 // apply_inflow, constant inflow without fluctuations, src/BoundCond.cu:2810-2997:
@@ -4425,10 +4490,15 @@ __global__ void k_bc_symmetry(Zone z, const Tab *__restrict__ tb, corefl_boundar
 // combination of the inflow state with the interior neighbour; ghosts take
 // the face state, or with inflow_sub its reflection about the face.
 template <int M>
-__global__ void k_bc_inflow(Zone z, const Tab *__restrict__ tb, corefl_boundary b, corefl_bc_condition c) {
+__global__ __launch_bounds__(kFaceBlock) void k_bc_inflow(Zone z, const Tab *__restrict__ tb, corefl_boundary b, corefl_bc_condition c) {
   [[maybe_unused]] constexpr int NS = kNs(M);
-  int i, j, k;
-  if (!face_point(b, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, i, j, k)) return;
+  FaceSite f;
+  if (!face_site(z, b, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, f)) return;
+  // the characteristic treatment reads the face node before replacing it, so one thread takes the site's
+  // layers in turn; the imposed state needs no other node and takes a thread per layer
+  if (c.inflow_sub && f.layer > 0) return;
+  const int i = f.i, j = f.j, k = f.k;
+  const int g_first = c.inflow_sub ? 1 : f.layer, g_last = c.inflow_sub ? z.ngg : f.layer;
   int d[3] = {0, 0, 0};
   d[b.face] = b.direction;
   const long sz = z.sz, p = z.ix(i, j, k);
@@ -4456,16 +4526,18 @@ __global__ void k_bc_inflow(Zone z, const Tab *__restrict__ tb, corefl_boundary 
       T = NS > 0 ? pr * c.mw / (density * kRu) : pr / (density * kRair);
     }
   }
-  z.bv[p] = density;
-  z.bv[p + sz] = u;
-  z.bv[p + 2 * sz] = v;
-  z.bv[p + 3 * sz] = w;
-  z.bv[p + 4 * sz] = pr;
-  z.bv[p + 5 * sz] = T;
+  if (f.layer == 0) {
+    z.bv[p] = density;
+    z.bv[p + sz] = u;
+    z.bv[p + 2 * sz] = v;
+    z.bv[p + 3 * sz] = w;
+    z.bv[p + 4 * sz] = pr;
+    z.bv[p + 5 * sz] = T;
 #pragma unroll
-  for (int l = 0; l < kNsc(M); ++l) z.sv[p + l * sz] = c.sv[l];
-  cv_from_bv_point<M>(z, tb, p);
-  for (int g = 1; g <= z.ngg; ++g) {
+    for (int l = 0; l < kNsc(M); ++l) z.sv[p + l * sz] = c.sv[l];
+    cv_from_bv_point<M>(z, tb, p);
+  }
+  for (int g = max(g_first, 1); g <= g_last; ++g) {
     const long pg = z.ix(i + g * d[0], j + g * d[1], k + g * d[2]);
 #pragma unroll
     for (int l = 0; l < kNsc(M); ++l) z.sv[pg + l * sz] = c.sv[l];
@@ -4517,10 +4589,11 @@ DEV void project_to_interior(const Zone &z, int *ix) {
 // reflects the velocity of interior layer g and takes T_g = 2 T_w - T_i
 // (isothermal; T_w where that falls to 0.1 T_w or below) or T_i.
 template <int M>
-__global__ void k_bc_wall(Zone z, const Tab *__restrict__ tb, corefl_boundary b, corefl_bc_condition c) {
+__global__ __launch_bounds__(kFaceBlock) void k_bc_wall(Zone z, const Tab *__restrict__ tb, corefl_boundary b, corefl_bc_condition c) {
   [[maybe_unused]] constexpr int NS = kNs(M);
-  int i, j, k;
-  if (!face_point(b, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, i, j, k)) return;
+  FaceSite f;
+  if (!face_site(z, b, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, f)) return;
+  const int i = f.i, j = f.j, k = f.k;
   int d[3] = {0, 0, 0};
   d[b.face] = b.direction;
   const long sz = z.sz, p = z.ix(i, j, k);
@@ -4534,59 +4607,62 @@ __global__ void k_bc_wall(Zone z, const Tab *__restrict__ tb, corefl_boundary b,
     const double tve_in = z.tve[pin] > 0.0 ? z.tve[pin] : z.bv[pin + 5 * sz];
     tve_wall = c.thermal_type == 1 ? tve_in : (c.temperature_ve > 0.0 ? c.temperature_ve : t_wall);
   }
-  const double pr = z.bv[pin + 4 * sz];
+  // the face node and each ghost layer read interior nodes only: a thread per site and layer
+  if (f.layer == 0) {
+    const double pr = z.bv[pin + 4 * sz];
 #pragma unroll
-  for (int l = 0; l < NS; ++l) z.sv[p + l * sz] = z.sv[pin + l * sz];
-  z.bv[p] = pr / (t_wall * gas_constant_at<M>(z, tb, p));
-  z.bv[p + sz] = 0;
-  z.bv[p + 2 * sz] = 0;
-  z.bv[p + 3 * sz] = 0;
-  z.bv[p + 4 * sz] = pr;
-  z.bv[p + 5 * sz] = t_wall;
-  if constexpr (kTT(M)) {
-    double y[NS];
-#pragma unroll
-    for (int l = 0; l < NS; ++l) y[l] = z.sv[p + l * sz];
-    z.tve[p] = tve_wall;
-    z.sv[p + NS * sz] = mix_ve_energy<M>(tb, tve_wall, y, nullptr);
-  }
-  cv_from_bv_point<M>(z, tb, p);
-  for (int g = 1; g <= z.ngg; ++g) {
-    int in[3] = {i - g * d[0], j - g * d[1], k - g * d[2]};
-    project_to_interior(z, in);
-    const long pi = z.ix(in[0], in[1], in[2]);
-    const long pg = z.ix(i + g * d[0], j + g * d[1], k + g * d[2]);
-    const double p_i = z.bv[pi + 4 * sz], t_i = z.bv[pi + 5 * sz];
-    double t_g = t_i;
-    if (c.thermal_type == 0) {
-      t_g = 2 * t_wall - t_i;
-      // the floor is 0.1 T_w in the two-temperature build and T_w otherwise
-      if (t_g <= 0.1 * t_wall) t_g = kTT(M) ? 0.1 * t_wall : t_wall;
-    }
-#pragma unroll
-    for (int l = 0; l < NS; ++l) z.sv[pg + l * sz] = z.sv[pi + l * sz];
+    for (int l = 0; l < NS; ++l) z.sv[p + l * sz] = z.sv[pin + l * sz];
+    z.bv[p] = pr / (t_wall * gas_constant_at<M>(z, tb, p));
+    z.bv[p + sz] = 0;
+    z.bv[p + 2 * sz] = 0;
+    z.bv[p + 3 * sz] = 0;
+    z.bv[p + 4 * sz] = pr;
+    z.bv[p + 5 * sz] = t_wall;
     if constexpr (kTT(M)) {
-      const double tve_i = z.tve[pi] > 0.0 ? z.tve[pi] : t_i;
-      double tve_g = tve_i;
-      if (c.thermal_type == 0) {
-        tve_g = 2 * tve_wall - tve_i;
-        const double floor_ve = 0.1 * fmax(tve_wall, 1.0);
-        if (tve_g <= floor_ve) tve_g = floor_ve;
-      }
       double y[NS];
 #pragma unroll
-      for (int l = 0; l < NS; ++l) y[l] = z.sv[pg + l * sz];
-      z.tve[pg] = tve_g;
-      z.sv[pg + NS * sz] = mix_ve_energy<M>(tb, tve_g, y, nullptr);
+      for (int l = 0; l < NS; ++l) y[l] = z.sv[p + l * sz];
+      z.tve[p] = tve_wall;
+      z.sv[p + NS * sz] = mix_ve_energy<M>(tb, tve_wall, y, nullptr);
     }
-    z.bv[pg] = p_i / (t_g * gas_constant_at<M>(z, tb, pi));
-    z.bv[pg + sz] = -z.bv[pi + sz];
-    z.bv[pg + 2 * sz] = -z.bv[pi + 2 * sz];
-    z.bv[pg + 3 * sz] = -z.bv[pi + 3 * sz];
-    z.bv[pg + 4 * sz] = p_i;
-    z.bv[pg + 5 * sz] = t_g;
-    cv_from_bv_point<M>(z, tb, pg);
+    cv_from_bv_point<M>(z, tb, p);
+    return;
   }
+  const int g = f.layer;
+  int in[3] = {i - g * d[0], j - g * d[1], k - g * d[2]};
+  project_to_interior(z, in);
+  const long pi = z.ix(in[0], in[1], in[2]);
+  const long pg = z.ix(i + g * d[0], j + g * d[1], k + g * d[2]);
+  const double p_i = z.bv[pi + 4 * sz], t_i = z.bv[pi + 5 * sz];
+  double t_g = t_i;
+  if (c.thermal_type == 0) {
+    t_g = 2 * t_wall - t_i;
+    // the floor is 0.1 T_w in the two-temperature build and T_w otherwise
+    if (t_g <= 0.1 * t_wall) t_g = kTT(M) ? 0.1 * t_wall : t_wall;
+  }
+#pragma unroll
+  for (int l = 0; l < NS; ++l) z.sv[pg + l * sz] = z.sv[pi + l * sz];
+  if constexpr (kTT(M)) {
+    const double tve_i = z.tve[pi] > 0.0 ? z.tve[pi] : t_i;
+    double tve_g = tve_i;
+    if (c.thermal_type == 0) {
+      tve_g = 2 * tve_wall - tve_i;
+      const double floor_ve = 0.1 * fmax(tve_wall, 1.0);
+      if (tve_g <= floor_ve) tve_g = floor_ve;
+    }
+    double y[NS];
+#pragma unroll
+    for (int l = 0; l < NS; ++l) y[l] = z.sv[pg + l * sz];
+    z.tve[pg] = tve_g;
+    z.sv[pg + NS * sz] = mix_ve_energy<M>(tb, tve_g, y, nullptr);
+  }
+  z.bv[pg] = p_i / (t_g * gas_constant_at<M>(z, tb, pi));
+  z.bv[pg + sz] = -z.bv[pi + sz];
+  z.bv[pg + 2 * sz] = -z.bv[pi + 2 * sz];
+  z.bv[pg + 3 * sz] = -z.bv[pi + 3 * sz];
+  z.bv[pg + 4 * sz] = p_i;
+  z.bv[pg + 5 * sz] = t_g;
+  cv_from_bv_point<M>(z, tb, pg);
 }
 
 // limit_flow, src/TimeAdvanceFunc.cuh:129-232.  A point with a NaN or an
@@ -5189,6 +5265,13 @@ hipError_t launch_cv_from_bv(const Zone &z, const Run &r, const Tab *tb, hipStre
   return hipGetLastError();
 }
 
+hipError_t launch_close_2d(const Zone &z, const Run &r, const Tab *tb, bool planes, hipStream_t s) {
+  const long n = static_cast<long>(z.mx + 2 * z.ngg) * (z.my + 2 * z.ngg);
+  COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_close_2d<MV>), dim3(blocks_for(n, 64)), dim3(64), 0, s, z, tb,
+                                              r.viscous_order == 2 ? 1 : 0, planes ? 1 : 0, n));
+  return hipGetLastError();
+}
+
 hipError_t launch_properties(const Zone &z, const Run &r, const Tab *tb, hipStream_t s) {
   const long n = padded_points(z);
   COREFL_DISPATCH(r.model,
@@ -5334,27 +5417,27 @@ hipError_t launch_viscous_flux(const Zone &z, const Run &r, const Tab *tb, hipSt
 }
 
 template <int M, int DIR>
-hipError_t launch_visc2_dir(const Zone &z, const Run &r, const Tab *tb, hipStream_t s) {
+hipError_t launch_visc2_dir(const Zone &z, const Run &r, const Tab *tb, hipStream_t s, int flat) {
   [[maybe_unused]] constexpr int NS = kNs(M);
   const long nf = static_cast<long>(z.mx + (DIR == 0)) * (z.my + (DIR == 1)) * (z.mz + (DIR == 2));
   hipLaunchKernelGGL((k_visc2_flux<M, DIR>), dim3(blocks_for(nf)), dim3(kBlock), 0, s, z, tb, r.prandtl, r.gradp,
-                     nf);
+                     flat, nf);
   const long n = interior_points(z);
   hipLaunchKernelGGL((k_visc2_diff<kNv(M), DIR>), dim3(blocks_for(n)), dim3(kBlock), 0, s, z, n);
   return hipGetLastError();
 }
 
 template <int M>
-hipError_t launch_visc2_t(const Zone &z, const Run &r, const Tab *tb, hipStream_t s) {
+hipError_t launch_visc2_t(const Zone &z, const Run &r, const Tab *tb, hipStream_t s, int flat) {
   [[maybe_unused]] constexpr int NS = kNs(M);
-  hipError_t e = launch_visc2_dir<M, 0>(z, r, tb, s);
-  if (e == hipSuccess) e = launch_visc2_dir<M, 1>(z, r, tb, s);
-  if (e == hipSuccess && z.mz > 1) e = launch_visc2_dir<M, 2>(z, r, tb, s);
+  hipError_t e = launch_visc2_dir<M, 0>(z, r, tb, s, flat);
+  if (e == hipSuccess) e = launch_visc2_dir<M, 1>(z, r, tb, s, flat);
+  if (e == hipSuccess && z.mz > 1) e = launch_visc2_dir<M, 2>(z, r, tb, s, 0);
   return e;
 }
 
-hipError_t launch_viscous2(const Zone &z, const Run &r, const Tab *tb, hipStream_t s) {
-  COREFL_DISPATCH(r.model, return launch_visc2_t<MV>(z, r, tb, s));
+hipError_t launch_viscous2(const Zone &z, const Run &r, const Tab *tb, hipStream_t s, bool flat) {
+  COREFL_DISPATCH(r.model, return launch_visc2_t<MV>(z, r, tb, s, flat ? 1 : 0));
   return hipSuccess;
 }
 
@@ -5381,33 +5464,42 @@ hipError_t launch_periodic_flux(const Zone &z, const Run &r, const corefl_bounda
   return hipGetLastError();
 }
 
-hipError_t launch_bc_outflow(const Zone &z, const Run &r, const Tab *tb, const corefl_boundary &b, hipStream_t s) {
-  const long n = face_points(b);
-  COREFL_DISPATCH(r.model,
-                     hipLaunchKernelGGL((k_bc_outflow<MV>), dim3(blocks_for(n)), dim3(kBlock), 0, s, z, tb, b));
+hipError_t launch_bc_outflow(const Zone &z, const Run &r, const Tab *tb, const corefl_boundary *b, int n_faces,
+                             hipStream_t s) {
+  for (int first = 0; first < n_faces; first += kFaceSet) {
+    FaceSet set{};
+    const int n = std::min(kFaceSet, n_faces - first);
+    long most = 0;
+    for (int q = 0; q < n; ++q) {
+      set.b[q] = b[first + q];
+      most = std::max(most, face_points(set.b[q]) * z.ngg);
+    }
+    COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_bc_outflow<MV>), dim3(blocks_for(most, kFaceBlock), n),
+                                                dim3(kFaceBlock), 0, s, z, tb, set));
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_bc_symmetry(const Zone &z, const Run &r, const Tab *tb, const corefl_boundary &b, hipStream_t s) {
-  const long n = face_points(b);
+  const long n = face_points(b) * (z.ngg + 1);
   COREFL_DISPATCH(r.model,
-                     hipLaunchKernelGGL((k_bc_symmetry<MV>), dim3(blocks_for(n)), dim3(kBlock), 0, s, z, tb, b));
+                     hipLaunchKernelGGL((k_bc_symmetry<MV>), dim3(blocks_for(n, kFaceBlock)), dim3(kFaceBlock), 0, s, z, tb, b));
   return hipGetLastError();
 }
 
 hipError_t launch_bc_inflow(const Zone &z, const Run &r, const Tab *tb, const corefl_boundary &b,
                             const corefl_bc_condition &c, hipStream_t s) {
-  const long n = face_points(b);
+  const long n = face_points(b) * (z.ngg + 1);
   COREFL_DISPATCH(r.model,
-                     hipLaunchKernelGGL((k_bc_inflow<MV>), dim3(blocks_for(n)), dim3(kBlock), 0, s, z, tb, b, c));
+                     hipLaunchKernelGGL((k_bc_inflow<MV>), dim3(blocks_for(n, kFaceBlock)), dim3(kFaceBlock), 0, s, z, tb, b, c));
   return hipGetLastError();
 }
 
 hipError_t launch_bc_wall(const Zone &z, const Run &r, const Tab *tb, const corefl_boundary &b,
                           const corefl_bc_condition &c, hipStream_t s) {
-  const long n = face_points(b);
+  const long n = face_points(b) * (z.ngg + 1);
   COREFL_DISPATCH(r.model,
-                     hipLaunchKernelGGL((k_bc_wall<MV>), dim3(blocks_for(n)), dim3(kBlock), 0, s, z, tb, b, c));
+                     hipLaunchKernelGGL((k_bc_wall<MV>), dim3(blocks_for(n, kFaceBlock)), dim3(kFaceBlock), 0, s, z, tb, b, c));
   return hipGetLastError();
 }
 
@@ -5491,21 +5583,16 @@ __global__ __launch_bounds__(kBlock) void k_zero_dq_multi(const Zone *__restrict
 }
 
 template <int M>
-__global__ __launch_bounds__(kBlock) void k_bc_outflow_multi(const Zone *__restrict__ zs,
-                                                             const BcItem *__restrict__ items,
-                                                             const Tab *__restrict__ tb) {
+__global__ __launch_bounds__(kFaceBlock) void k_bc_outflow_multi(const Zone *__restrict__ zs,
+                                                                 const BcItem *__restrict__ items,
+                                                                 const Tab *__restrict__ tb) {
   const BcItem &it = items[blockIdx.y];
-  const corefl_boundary &b = it.b;
-  const int n0 = b.range_end[0] - b.range_start[0] + 1, n1 = b.range_end[1] - b.range_start[1] + 1;
-  const int n2 = b.range_end[2] - b.range_start[2] + 1;
-  const long t = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-  if (t >= static_cast<long>(n0) * n1 * n2) return;
-  const int i = b.range_start[0] + static_cast<int>(t % n0);
-  const int j = b.range_start[1] + static_cast<int>((t / n0) % n1);
-  const int k = b.range_start[2] + static_cast<int>(t / (static_cast<long>(n0) * n1));
+  const Zone &z = zs[it.blk];
+  FaceSite f;
+  if (!face_site(z, it.b, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, f, 1)) return;
   int d[3] = {0, 0, 0};
-  d[b.face] = b.direction;
-  bc_outflow_point<M>(zs[it.blk], tb, i, j, k, d);
+  d[it.b.face] = it.b.direction;
+  bc_outflow_layer<M>(z, tb, f.i, f.j, f.k, d, f.layer);
 }
 
 hipError_t launch_zero_dq_multi(const Zone *zs, int nb, long max_n, int nv, hipStream_t s) {
@@ -5538,8 +5625,8 @@ hipError_t launch_properties_multi(const Zone *zs, int nb, long max_padded, cons
 hipError_t launch_bc_outflow_multi(const Zone *zs, const BcItem *items, int n_items, long max_face, const Run &r,
                                    const Tab *tb, hipStream_t s) {
   if (n_items <= 0) return hipSuccess;
-  COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_bc_outflow_multi<MV>), dim3(blocks_for(max_face), n_items),
-                                              dim3(kBlock), 0, s, zs, items, tb));
+  COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_bc_outflow_multi<MV>), dim3(blocks_for(max_face, kFaceBlock), n_items),
+                                              dim3(kFaceBlock), 0, s, zs, items, tb));
   return hipGetLastError();
 }
 

@@ -134,6 +134,15 @@ struct Tab : corefl_chem_tables {
   double pw_kbe[COREFL_MAX_SPEC][COREFL_MAX_SPEC];  // 1.0548 kb_over_eps_jk^-0.15504
   double inv_bdc[COREFL_MAX_SPEC][COREFL_MAX_SPEC]; // 1 / binary_diffusivity_coeff
   double rcp_imw[COREFL_MAX_SPEC], mol_conv[COREFL_MAX_SPEC];  // 1 / imw, 1e3 / imw
+  double vt_mw[COREFL_MAX_SPEC];  // molar mass of the V-T relaxation times, 1 / max(imw, 1e-20)
+  // electronic levels in groups of four, padded with levels of weight 0; a level more than elec_stop
+  // temperatures above elec_first (the first excited one) cannot change the Boltzmann sums (infinite when the
+  // levels are not in rising order)
+  static_assert(COREFL_MAX_ELEC % 4 == 0, "whole groups of levels");
+  double elec_th4[COREFL_MAX_SPEC][COREFL_MAX_ELEC], elec_g4[COREFL_MAX_SPEC][COREFL_MAX_ELEC];
+  double elec_first[COREFL_MAX_SPEC], elec_stop[COREFL_MAX_SPEC];
+  // which of the usual control temperatures a reaction's rates take: 0 T, 1 sqrt(T Tve), 2 Tve, -1 another
+  int tcf_set[COREFL_MAX_REAC], tcb_set[COREFL_MAX_REAC];
   Reac reac[COREFL_MAX_REAC];
 };
 void derive_tables(const corefl_chem_tables &in, Tab &out);

@@ -751,13 +751,42 @@ void derive_tables(const corefl_chem_tables &in, Tab &out) {
     out.pw_lj[l] = std::exp(-0.145 * ln_lj);
     out.rcp_imw[l] = 1.0 / in.imw[l];
     out.mol_conv[l] = 1e+3 / in.imw[l];
+    out.vt_mw[l] = 1.0 / std::fmax(in.imw[l], 1e-20);
+    const int ne = in.two_temperature ? in.n_elec[l] : 0;
+    for (int j = 0; j < COREFL_MAX_ELEC; ++j) {
+      out.elec_th4[l][j] = j < ne ? in.elec_theta[l][j] : 0.0;
+      out.elec_g4[l][j] = j < ne ? in.elec_g[l][j] : 0.0;
+    }
+    // the first excited level (theta > 0, weight > 0) and how far above it a level's term is below 2^-54 of its
+    // term in sum g e^-x, sum g theta e^-x and sum g theta^2 e^-x: ln of the largest ratio of weights and
+    // squared energies, plus 38 > 54 ln 2
+    out.elec_first[l] = 0.0;
+    out.elec_stop[l] = INFINITY;
+    int first = 0;
+    bool rising = true;
+    while (first < ne && !(in.elec_theta[l][first] > 0.0 && in.elec_g[l][first] > 0.0)) ++first;
+    for (int j = 1; j < ne; ++j) rising = rising && in.elec_theta[l][j] >= in.elec_theta[l][j - 1];
+    if (rising && first < ne) {
+      double most = 1.0;
+      for (int j = first; j < ne; ++j) {
+        const double e = in.elec_theta[l][j] / in.elec_theta[l][first], w = in.elec_g[l][j] / in.elec_g[l][first];
+        most = std::fmax(most, std::fabs(w) * e * e);
+      }
+      out.elec_first[l] = in.elec_theta[l][first];
+      out.elec_stop[l] = std::log(most) + 38.0;
+    }
     for (int k = 0; k < in.n_spec; ++k) {
       const double ln_kbe = in.kb_over_eps_jk[l][k] > 0 ? std::log(in.kb_over_eps_jk[l][k]) : 0.0;
       out.pw_kbe[l][k] = 1.0548 * std::exp(-0.15504 * ln_kbe);
       out.inv_bdc[l][k] = in.binary_diffusivity_coeff[l][k] != 0 ? 1.0 / in.binary_diffusivity_coeff[l][k] : 0.0;
     }
   }
+  auto ctrl_set = [](double a, double b) {
+    return a == 1.0 && b == 0.0 ? 0 : (a == 0.5 && b == 0.5 ? 1 : (a == 0.0 && b == 1.0 ? 2 : -1));
+  };
   for (int r = 0; r < in.n_reac; ++r) {
+    out.tcf_set[r] = ctrl_set(in.tcf_a[r], in.tcf_b[r]);
+    out.tcb_set[r] = ctrl_set(in.tcb_a[r], in.tcb_b[r]);
     Reac &R = out.reac[r];
     R = Reac{};
     for (int l = 0; l < in.n_spec; ++l) {

@@ -56,6 +56,12 @@ DEV double div_by(double x) {
   return fma(fma(-d, q, x), y, q);
 }
 
+// the same for a divisor d whose rounded reciprocal rd serves several quotients
+DEV double div_rcp(double x, double d, double rd) {
+  const double q = x * rd;
+  return fma(fma(-d, q, x), rd, q);
+}
+
 // a x + b y and a x + b y + c z with the fused operations written out: where two
 // products meet, which one the compiler fuses depends on the code around them,
 // and the two reactor kernels have to agree in every bit.
@@ -314,22 +320,24 @@ DEV void thermo_gibbs(const Tab *__restrict__ tb, double t, double *g) {
 // unit mass; temperatures clamped at 1 K).  Only the two-temperature models
 // call these.
 // ---------------------------------------------------------------------------
-DEV double vib_energy1(const Tab *__restrict__ tb, int i, double t) {
+// (it: 1 / max(t, 1), shared by the species and levels at one temperature)
+DEV double ve_inverse(double t) { return 1.0 / fmax(t, 1.0); }
+DEV double vib_energy1(const Tab *__restrict__ tb, int i, double t, double it) {
   const double temp = fmax(t, 1.0);
   double e = 0.0;
   const double th = tb->theta_v[i];
   if (th > 0) {
-    const double x = th / temp;
+    const double x = div_rcp(th, temp, it);
     if (x < 200) e += tb->gas_const[i] * th / expm1(x);
   }
   return e;
 }
-DEV double vib_cv1(const Tab *__restrict__ tb, int i, double t) {
+DEV double vib_cv1(const Tab *__restrict__ tb, int i, double t, double it) {
   const double temp = fmax(t, 1.0);
   double c = 0.0;
   const double th = tb->theta_v[i];
   if (th > 0) {
-    const double x = th / temp;
+    const double x = div_rcp(th, temp, it);
     if (x < 200) {
       const double ex = exp(x), d = ex - 1.0;
       c += tb->gas_const[i] * x * x * ex / (d * d);
@@ -337,20 +345,36 @@ DEV double vib_cv1(const Tab *__restrict__ tb, int i, double t) {
   }
   return c;
 }
-// E_ve of species i (compute_ve_energy) and, when WANT_CV, its c_v (compute_ve_cv)
+// E_ve of species i (compute_ve_energy) and, when WANT_CV, its c_v (compute_ve_cv).
+// The electronic levels go four at a time (the exponentials overlap, the table
+// reads come together; the tables are padded with levels of weight 0), and stop
+// where the remaining levels cannot change the sums: with the levels in rising
+// order, a level elec_stop temperatures above the first excited one is below
+// 2^-54 of that one's term in each of them.  Cold gas needs one or two groups of
+// the 46 levels of five-species air.
 template <bool WANT_CV>
-DEV double ve_energy1(const Tab *__restrict__ tb, int i, double t, double *cv) {
+DEV double ve_energy1(const Tab *__restrict__ tb, int i, double t, double it, double *cv) {
   const double temp = fmax(t, 1.0);
-  double e = vib_energy1(tb, i, temp);
-  double c = WANT_CV ? vib_cv1(tb, i, temp) : 0.0;
+  double e = vib_energy1(tb, i, temp, it);
+  double c = WANT_CV ? vib_cv1(tb, i, temp, it) : 0.0;
   const int n = tb->n_elec[i];
   if (n > 0) {
     double zz = 0.0, b = 0.0, cc = 0.0;
-    for (int j = 0; j < n; ++j) {
-      const double th = tb->elec_theta[i][j], boltz = tb->elec_g[i][j] * exp(-th / temp);
-      zz += boltz;
-      b += boltz * th;
-      if (WANT_CV) cc += boltz * th * th;
+    const double top = fma(tb->elec_stop[i], temp, tb->elec_first[i]);
+    for (int j = 0; j < n; j += 4) {
+      if (tb->elec_th4[i][j] > top) break;
+      double th[4], boltz[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        th[m] = tb->elec_th4[i][j + m];
+        boltz[m] = tb->elec_g4[i][j + m] * exp(div_rcp(-th[m], temp, it));
+      }
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        zz += boltz[m];
+        b += boltz[m] * th[m];
+        if (WANT_CV) cc += boltz[m] * th[m] * th[m];
+      }
     }
     if (zz > 0) {
       e += tb->gas_const[i] * b / zz;
@@ -368,10 +392,11 @@ template <int M>
 DEV double mix_ve_energy(const Tab *__restrict__ tb, double t, const double *y, double *cv_ve) {
   constexpr int NS = kNs(M);
   double e = 0.0, c = 0.0;
+  const double it = ve_inverse(t);
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
     double ci = 0.0;
-    const double ei = cv_ve ? ve_energy1<true>(tb, i, t, &ci) : ve_energy1<false>(tb, i, t, nullptr);
+    const double ei = cv_ve ? ve_energy1<true>(tb, i, t, it, &ci) : ve_energy1<false>(tb, i, t, it, nullptr);
     e += y[i] * ei;
     c += y[i] * ci;
   }
@@ -383,7 +408,7 @@ DEV double mix_vib_energy(const Tab *__restrict__ tb, double t, const double *y)
   constexpr int NS = kNs(M);
   double e = 0.0;
 #pragma unroll
-  for (int i = 0; i < NS; ++i) e += y[i] * vib_energy1(tb, i, t);
+  for (int i = 0; i < NS; ++i) e += y[i] * vib_energy1(tb, i, t, ve_inverse(t));
   return e;
 }
 // compute_mixture_tr_energy, src/Thermo.cu:746-770: E_tr with the
@@ -430,35 +455,37 @@ DEV double invert_tve(const Tab *__restrict__ tb, double eve_target, const doubl
   return tve;
 }
 // Millikan-White pair time with Park's correction, src/Thermo.cu:805-854
-DEV double mw_pair_tau(const Tab *__restrict__ tb, int iv, int ip, double t, double p) {
+// (t_m3 = t^(-1/3), once per point)
+DEV double mw_pair_tau(const Tab *__restrict__ tb, int iv, int ip, double t, double t_m3, double p) {
   if (p <= 1e-16 || t <= 1.0) return 1e30;
-  const double mv = 1.0 / fmax(tb->imw[iv], 1e-20), mp = 1.0 / fmax(tb->imw[ip], 1e-20);
-  const double mu = mv * mp / fmax(mv + mp, 1e-20);
   double a = tb->lt_a[iv][ip], b = tb->lt_b[iv][ip];
   if (a <= 0.0 || b <= 0.0) {
+    const double mv = 1.0 / fmax(tb->imw[iv], 1e-20), mp = 1.0 / fmax(tb->imw[ip], 1e-20);
+    const double mu = mv * mp / fmax(mv + mp, 1e-20);
     a = 1.16e-3 * sqrt(fmax(mu, 1e-20)) * pow(fmax(tb->theta_v[iv], 0.0), 4.0 / 3.0);
     b = 0.015 * pow(fmax(mu, 1e-20), 0.25);
   }
-  const double ex = a * (pow(t, -1.0 / 3.0) - b) - 18.421;
+  const double ex = a * (t_m3 - b) - 18.421;
   return fmax(exp(ex) * kPatm / p, 1e-30);
 }
 template <int M>
-DEV double species_vt_tau(const Tab *__restrict__ tb, int iv, double rho, double t, double p, const double *y) {
+DEV double species_vt_tau(const Tab *__restrict__ tb, int iv, double rho, double t, double t_m3, double p,
+                          const double *y) {
   constexpr int NS = kNs(M);
   double conc = 0.0, den = 0.0;
 #pragma unroll
   for (int j = 0; j < NS; ++j) {
     const double yj = fmax(y[j], 0.0);
     if (yj <= 0.0) continue;
-    const double mole = yj / (1.0 / fmax(tb->imw[j], 1e-20));
+    const double mole = yj / tb->vt_mw[j];
     conc += mole;
-    den += mole / mw_pair_tau(tb, iv, j, t, p);
+    den += mole / mw_pair_tau(tb, iv, j, t, t_m3, p);
   }
   if (conc <= 0.0 || den <= 0.0) return 1e30;
   const double tau_mw = conc / den;
   const double sigma = fmax(tb->park_sigma[iv], 1e-30) * (2.5e9 / fmax(t * t, 1.0));
   const double n_total = rho * conc * 6.02214076e26;
-  const double mv = 1.0 / fmax(tb->imw[iv], 1e-20);
+  const double mv = tb->vt_mw[iv];
   const double cs = sqrt(fmax(8.0 * kRu * t / (kPi * mv), 1e-30));
   const double tau_park = 1.0 / fmax(sigma * cs * n_total, 1e-30);
   return fmax(tau_mw + tau_park, 1e-30);
@@ -474,15 +501,16 @@ DEV void vt_relaxation_time(const Tab *__restrict__ tb, double rho, double t, do
   for (int i = 0; i < NS; ++i) rm += fmax(y[i], 0.0) * tb->gas_const[i];
   const double p = rho * rm * fmax(t, 1.0);
   double eq = 0.0, em = 0.0, src = 0.0;
+  const double it = ve_inverse(t), itve = ve_inverse(tve), t_m3 = pow(t, -1.0 / 3.0);
   for (int i = 0; i < NS; ++i) {
     if (tb->theta_v[i] <= 0.0) continue;
     const double yi = fmax(y[i], 0.0);
     if (yi <= 0.0) continue;
-    const double e_eq = vib_energy1(tb, i, t), e_i = vib_energy1(tb, i, tve), d = e_eq - e_i;
+    const double e_eq = vib_energy1(tb, i, t, it), e_i = vib_energy1(tb, i, tve, itve), d = e_eq - e_i;
     eq += yi * e_eq;
     em += yi * e_i;
     if (fabs(d) <= 1e-16) continue;
-    const double tau = species_vt_tau<M>(tb, i, rho, t, p, y);
+    const double tau = species_vt_tau<M>(tb, i, rho, t, t_m3, p, y);
     if (tau < 1e29) src += rho * yi * d / tau;
   }
   eve_eq = eq;
@@ -1136,26 +1164,38 @@ __global__ __launch_bounds__(kBlock) void k_vt_relax(Zone z, const Tab *__restri
 // for 1 and 2).
 // ---------------------------------------------------------------------------
 // reaction_temperature with smooth_reaction_temperature, src/FiniteRateChem.cu:1490-1503
-DEV double reaction_temperature(double t, double tve, double a, double b) {
-  const double trx = pow(fmax(t, 1.0), a) * pow(fmax(tve, 1.0), b);
-  return 0.5 * (trx + 800.0 + sqrt((trx - 800.0) * (trx - 800.0) + 80.0 * 80.0));
-}
-// G/RT of one species (same arithmetic as thermo_gibbs)
+// One control temperature T^a Tve^b (smoothed) with what a reaction needs there.
+// Mechanisms use a few exponent pairs for all their reactions, so chem_rates
+// evaluates the three usual ones once per point: (1, 0), (1/2, 1/2) and (0, 1).
 template <int M>
-DEV double gibbs1(const Tab *__restrict__ tb, int i, double t) {
-  if constexpr (kNasa9(M)) {
-    return nasa9_g1(tb, i, nasa9_terms(t));
-  } else {
-    const double tl = tb->t_low[i], th = tb->t_high[i];
-    const bool out = t < tl || t > th;
-    const double tt = out ? (t < tl ? tl : th) : t;
-    const double *c = out ? (t < tl ? tb->low_coeff[i] : tb->high_coeff[i])
-                          : (t < tb->t_mid[i] ? tb->low_coeff[i] : tb->high_coeff[i]);
-    const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt_inv = 1 / tt, log_tt = log(tt);
-    return nasa_g(c, tt, tt2, tt3, tt4, tt_inv, log_tt);
-  }
+struct CtrlTemp {
+  double th, lt, it, g[kNs(M) > 0 ? kNs(M) : 1];
+};
+template <int M>
+DEV void thermo_gibbs(const Tab *__restrict__ tb, double t, double *g);
+template <int M>
+DEV void ctrl_at(const Tab *__restrict__ tb, double trx, bool want_g, CtrlTemp<M> &c) {
+  c.th = 0.5 * (trx + 800.0 + sqrt((trx - 800.0) * (trx - 800.0) + 80.0 * 80.0));
+  c.lt = log(c.th);
+  c.it = 1.0 / c.th;
+  if (want_g) thermo_gibbs<M>(tb, c.th, c.g);
 }
-
+template <int M>
+struct CtrlSets {
+  CtrlTemp<M> s[3];
+};
+template <int M>
+DEV void ctrl_pick(const Tab *__restrict__ tb, const CtrlSets<M> &sets, int set, double a, double b, double t,
+                   double tve, bool want_g, CtrlTemp<M> &c) {
+  if (set == 0)
+    c = sets.s[0];
+  else if (set == 1)
+    c = sets.s[1];
+  else if (set == 2)
+    c = sets.s[2];
+  else
+    ctrl_at<M>(tb, pow(fmax(t, 1.0), a) * pow(fmax(tve, 1.0), b), want_g, c);
+}
 DEV double ipow(double c, int e) {
   if (e == 0) return 1.0;
   double p = c;
@@ -1182,19 +1222,20 @@ DEV double ln_std_conc(double ln_t) {
 }
 
 template <int M>
-DEV void reaction_progress(const Tab *__restrict__ tb, int r, double T, double tve, bool trx, double ln_t,
-                           double inv_t, double ln_temp_t, const double *c, const double *g, double &q1,
+DEV void reaction_progress(const Tab *__restrict__ tb, int r, double T, double tve, bool trx, const CtrlSets<M> *sets,
+                           double ln_t, double inv_t, double ln_temp_t, const double *c, const double *g, double &q1,
                            double &q2) {
   [[maybe_unused]] constexpr int NS = kNs(M);
   constexpr double temp_p = kPatm / kRu * 1e-3;
   constexpr double kLn10 = 2.302585092994046, kInvLn10 = 0.4342944819032518;
-  const Reac &R = tb->reac[r];
   const int type = tb->reac_type[r];
   double thf = T, lt = ln_t, it = inv_t;
   if (kTT(M) && trx) {
-    thf = reaction_temperature(T, tve, tb->tcf_a[r], tb->tcf_b[r]);
-    lt = log(thf);
-    it = 1.0 / thf;
+    CtrlTemp<M> f;
+    ctrl_pick<M>(tb, *sets, tb->tcf_set[r], tb->tcf_a[r], tb->tcf_b[r], T, tve, false, f);
+    thf = f.th;
+    lt = f.lt;
+    it = f.it;
   }
   double kf = arrhenius_ln(lt, it, tb->A[r], tb->b[r], tb->Ea[r]);
   if (type == 3) {
@@ -1236,10 +1277,11 @@ DEV void reaction_progress(const Tab *__restrict__ tb, int r, double T, double t
   if (kTT(M) && trx && type != 0) {
     // per-reaction backward temperature; REV keeps its rate, otherwise
     // kf / Kc with G/RT at that temperature (src/FiniteRateChem.cu:1560-1589)
-    const double thb = reaction_temperature(T, tve, tb->tcb_a[r], tb->tcb_b[r]);
-    const double lb = log(thb);
+    CtrlTemp<M> b;
+    ctrl_pick<M>(tb, *sets, tb->tcb_set[r], tb->tcb_a[r], tb->tcb_b[r], T, tve, true, b);
+    const double lb = b.lt;
     if (tb->rev_type[r] == 1) {
-      kb = arrhenius_ln(lb, 1.0 / thb, tb->A2[r], tb->b2[r], tb->Ea2[r]);
+      kb = arrhenius_ln(lb, b.it, tb->A2[r], tb->b2[r], tb->Ea2[r]);
       if (type == 4) {
         double cc = 0;
 #pragma unroll
@@ -1247,8 +1289,11 @@ DEV void reaction_progress(const Tab *__restrict__ tb, int r, double T, double t
         kb *= cc;
       }
     } else {
+      const int *sf = tb->stoi_f[r], *sb = tb->stoi_b[r];
       double d_gibbs = 0;
-      for (int m = 0; m < R.nnu; ++m) d_gibbs += gibbs1<M>(tb, R.nu_idx[m], thb) * R.nu[m];
+#pragma unroll
+      for (int l = 0; l < NS; ++l)
+        if (sb[l] != sf[l]) d_gibbs = fma(b.g[l], static_cast<double>(sb[l] - sf[l]), d_gibbs);
       kb = kf * exp(d_gibbs - static_cast<double>(tb->order[r]) * (log(temp_p) - lb));
     }
   } else if (type != 0) {
@@ -1326,10 +1371,19 @@ DEV void chem_rates(const Tab *__restrict__ tb, double density, double T, double
     tve = fmax(tve_in, 1.0);
     trx = tb->trx_model != 0;
   }
+  CtrlSets<M> sets;
+  if constexpr (kTT(M)) {
+    if (trx) {
+      const double t1 = fmax(T, 1.0), v1 = fmax(tve, 1.0);
+      ctrl_at<M>(tb, t1, true, sets.s[0]);
+      ctrl_at<M>(tb, sqrt(t1) * sqrt(v1), true, sets.s[1]);
+      ctrl_at<M>(tb, v1, true, sets.s[2]);
+    }
+  }
   const int nr = tb->n_reac;
   for (int r = 0; r < nr; ++r) {
     double q1, q2;
-    reaction_progress<M>(tb, r, T, tve, kTT(M) && trx, ln_t, inv_t, ln_temp_t, c, g, q1, q2);
+    reaction_progress<M>(tb, r, T, tve, kTT(M) && trx, &sets, ln_t, inv_t, ln_temp_t, c, g, q1, q2);
     // chemical_source accumulation, src/FiniteRateChem.cu:1665-1681, over the species taking part (either
     // coefficient not 0), looped over every species with tests the wave takes together
     const int *sfi = tb->stoi_f[r], *sbi = tb->stoi_b[r];
@@ -1386,7 +1440,7 @@ __global__ __launch_bounds__(kBlock) void k_chemistry(Zone z, const Tab *__restr
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
       const double conv = tb->mol_conv[l];
-      src += (creation[l] * conv - omega_d[l] * conv) * ve_energy1<false>(tb, l, tv, nullptr);
+      src += (creation[l] * conv - omega_d[l] * conv) * ve_energy1<false>(tb, l, tv, ve_inverse(tv), nullptr);
     }
     z.dq[t + (5 + NS) * dsz] += jac * src;
   }
@@ -1752,12 +1806,6 @@ __global__ __launch_bounds__(kReactorBlock) void k_reactors(ReactorPool P, const
 // factors in LDS, and 58 us with 5000 in flight against 212 with a lane each.
 // ---------------------------------------------------------------------------
 constexpr int kWave = 64;
-
-// x / d with rd = 1 / d rounded: the IEEE quotient's bits (see div_by)
-DEV double div_rcp(double x, double d, double rd) {
-  const double q = x * rd;
-  return fma(fma(-d, q, x), rd, q);
-}
 
 // lane src's v in every lane (src uniform)
 DEV double bcast(double v, int src) {
@@ -2774,7 +2822,7 @@ __global__ __launch_bounds__(TX *TS) void k_weno(Zone z, const Tab *__restrict__
 #pragma unroll
         for (int l = 0; l < NS; ++l) {
           double cv_ve;
-          h[l] -= ve_energy1<true>(tb, l, t_eval, &cv_ve);
+          h[l] -= ve_energy1<true>(tb, l, t_eval, ve_inverse(t_eval), &cv_ve);
           cp[l] -= cv_ve;
         }
       }
@@ -3299,7 +3347,7 @@ DEV void mix_e_gamma(const Tab *__restrict__ tb, double t, const double *y, doub
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
       double cv_ve;
-      h[l] -= ve_energy1<true>(tb, l, t_eval, &cv_ve);
+      h[l] -= ve_energy1<true>(tb, l, t_eval, ve_inverse(t_eval), &cv_ve);
       cp[l] -= cv_ve;
     }
   }
@@ -3701,7 +3749,7 @@ __global__ __launch_bounds__(TX *TS) void k_pv(Zone z, const Tab *__restrict__ t
 #pragma unroll
         for (int l = 0; l < NS; ++l) {
           h_s[l] = thermo_h1<M>(tb, l, t_roe, te2, te3, te4, te5);
-          if constexpr (kTT(M)) h_s[l] -= ve_energy1<false>(tb, l, t_roe, nullptr);
+          if constexpr (kTT(M)) h_s[l] -= ve_energy1<false>(tb, l, t_roe, ve_inverse(t_roe), nullptr);
           const double alpha = (gamma * tb->gas_const[l] * t_roe - (gamma - 1.0) * h_s[l]) / c2s;
           c1 += alpha * dq[l + 5];
         }
@@ -3981,8 +4029,8 @@ __global__ __launch_bounds__(kBlock) void k_viscous_flux(Zone z, const Tab *__re
       double h_diff = h[l];
       [[maybe_unused]] double eve_l = 0;
       if constexpr (kTT(M)) {
-        eve_l = ve_energy1<false>(tb, l, tve_m, nullptr);
-        h_diff = h[l] - ve_energy1<false>(tb, l, tm, nullptr) + eve_l;
+        eve_l = ve_energy1<false>(tb, l, tve_m, ve_inverse(tve_m), nullptr);
+        h_diff = h[l] - ve_energy1<false>(tb, l, tm, ve_inverse(tm), nullptr) + eve_l;
       }
       double dflux = diffusivity[l] * (dfx[l] - mw_tot * yk[l] * sGx) - yk[l] * CVx;
       fv[p + (5 + l) * sz] = dflux;
@@ -4184,7 +4232,7 @@ __global__ __launch_bounds__(kBlock) void k_visc2_flux(Zone z, const Tab *__rest
     if constexpr (kTT(M)) {
       tve_m = 0.5 * (z.tve[p] + z.tve[pe]);
 #pragma unroll
-      for (int l = 0; l < NS; ++l) eve_m[l] = ve_energy1<false>(tb, l, tve_m, nullptr);
+      for (int l = 0; l < NS; ++l) eve_m[l] = ve_energy1<false>(tb, l, tve_m, ve_inverse(tve_m), nullptr);
     }
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
@@ -4192,7 +4240,7 @@ __global__ __launch_bounds__(kBlock) void k_visc2_flux(Zone z, const Tab *__rest
       fv[p + (4 + l) * sz] = dflux;
       double h_diff = h[l];
       // compute_nonequilibrium_diffusion_enthalpy, src/Thermo.cuh:43-47
-      if constexpr (kTT(M)) h_diff = h[l] - ve_energy1<false>(tb, l, tm, nullptr) + eve_m[l];
+      if constexpr (kTT(M)) h_diff = h[l] - ve_energy1<false>(tb, l, tm, ve_inverse(tm), nullptr) + eve_m[l];
       f3 += h_diff * dflux;
     }
     if constexpr (kTT(M)) {

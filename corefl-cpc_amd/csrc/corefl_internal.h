@@ -188,7 +188,6 @@ void register_inner(const corefl_inner_face &in, int dim, int ngg, InnerDev &f);
 // ---- kernel launchers (kernels.hip) ----
 hipError_t launch_fill(double *p, long n, double v, hipStream_t s);
 hipError_t launch_copy(double *dst, const double *src, long n, hipStream_t s);
-hipError_t launch_scaled_copy(double *dst, const double *src, double a, long n, hipStream_t s);
 hipError_t launch_cv_from_bv(const Zone &z, const Run &r, const Tab *tb, hipStream_t s);
 hipError_t launch_properties(const Zone &z, const Run &r, const Tab *tb, hipStream_t s);
 // the end of a stage on a 2-D block: properties of plane k = 0 and, with planes, the ghost planes' state and
@@ -208,7 +207,9 @@ hipError_t launch_vt_relaxation(const Zone &z, const Run &r, const Tab *tb, doub
 hipError_t launch_min_combine(const double *v, int n, double *out, hipStream_t s);
 // shape: tile shape of the characteristic WENO sweep (0 or 1, kWenoShapes of them; same results)
 constexpr int kWenoShapes = 2;
-hipError_t launch_inviscid(const Zone &z, const Run &r, const Tab *tb, int dir, hipStream_t s, int shape = 0);
+// store (WENO schemes): replace dq instead of adding to it (the stage's first contribution, dq not cleared before)
+hipError_t launch_inviscid(const Zone &z, const Run &r, const Tab *tb, int dir, hipStream_t s, int shape = 0,
+                           bool store = false);
 hipError_t launch_shock_sensor(const Zone &z, const Run &r, hipStream_t s);
 hipError_t launch_reactors(const ReactorPool &p, int model, const Tab *tb, int max_steps, hipStream_t s);
 // the same step with one wave per slot, over slots [0, n_slots).  The servers take it while at most
@@ -249,7 +250,7 @@ hipError_t launch_limit_flow(const Zone &z, const Run &r, const Tab *tb, hipStre
 hipError_t launch_inner_comm(const Zone &z, const Zone &tz, const Run &r, const Tab *tb, const InnerDev &f,
                              hipStream_t s);
 hipError_t launch_inner_flux(const Zone &z, const Zone &tz, const Run &r, const InnerDev &f, hipStream_t s);
-// Writes dt_local and the block minimum into *dmin (device scalar, reduced with min).
+// Writes dt_local and, unless dmin is null, the block minimum into *dmin (device scalar).
 hipError_t launch_local_dt(const Zone &z, const Run &r, const Tab *tb, double *dmin, hipStream_t s);
 // one boundary face of one block of a multi-block launch
 struct BcItem {
@@ -271,7 +272,9 @@ hipError_t launch_tube_admit(const Zone &z, const TubePool &P, int model, const 
 hipError_t launch_tube_cv(const Zone &z, int model, const Tab *tb, const double *rec, int n_rec, hipStream_t s);
 hipError_t launch_tube_bc(const Zone &z, const TubePool &P, int model, const Tab *tb, int n_slots, hipStream_t s);
 hipError_t launch_tube_dt(const Zone &z, const TubePool &P, int n_slots, hipStream_t s, double fixed_dt = 0.0);
-hipError_t launch_tube_dtc(const Zone &z, const TubePool &P, const int *map, double *dtc, hipStream_t s);
+// dth (may be null): half of each point's step
+hipError_t launch_tube_dtc(const Zone &z, const TubePool &P, const int *map, double *dtc, hipStream_t s,
+                           double *dth = nullptr);
 hipError_t launch_tube_finish(const TubePool &P, int n_slots, hipStream_t s);
 // properties over one padded row (my = mz = 1 zones with zero y/z strides)
 hipError_t launch_properties_row(const Zone &z, const Run &r, const Tab *tb, hipStream_t s);

@@ -59,6 +59,7 @@ struct corefl_ctx {
   std::vector<hipEvent_t> join_ev;
   hipEvent_t fork_ev = nullptr;
   hipStream_t cur = nullptr;  // stream op_block launches on (nullptr: `stream`)
+  bool in_stage = false;      // issuing a whole stage: its x sweep may store dq
   bool qn_in_update = false;  // recording a step whose first-stage update saves qn (no separate copy)
   // multi-block launches of a recorded multi-block step: the zones and the outflow faces in device memory
   bool batched = false;
@@ -232,6 +233,17 @@ hipError_t periodic_launches(const corefl_ctx::Block &b, bool pairs, One one, Pa
   return hipSuccess;
 }
 
+// Whether a stage's x sweep is its first contribution to dq, which it then stores (dq is not cleared first):
+// the WENO sweeps without viscous terms and chemistry.
+bool sweep_stores(const Run &r) { return r.viscous_order == 0 && !(r.mixture && r.reaction) && r.scheme >= 51; }
+
+// marks the operators issued while it lives as a stage's (see sweep_stores)
+struct StageScope {
+  corefl_ctx *c;
+  explicit StageScope(corefl_ctx *ctx) : c(ctx) { c->in_stage = true; }
+  ~StageScope() { c->in_stage = false; }
+};
+
 // ---- operators on one block ----
 int op_block(corefl_ctx *c, int op, corefl_ctx::Block &b, int rk, double dt) {
   const Zone &z = b.z;
@@ -261,7 +273,7 @@ int op_block(corefl_ctx *c, int op, corefl_ctx::Block &b, int rk, double dt) {
       const int dir = op - COREFL_OP_INVISCID_X;
       if (dir == 2 && z.mz == 1) break;
       if (r.scheme == 51 || r.scheme == 52 || r.scheme == 71 || r.scheme == 72)
-        HIP_TRY(c, launch_inviscid(z, r, c->d_tables, dir, s, b.shape[dir]));
+        HIP_TRY(c, launch_inviscid(z, r, c->d_tables, dir, s, b.shape[dir], c->in_stage && sweep_stores(r) && dir == 0));
       else
         HIP_TRY(c, launch_inviscid_pv(z, r, c->d_tables, dir, s));
       break;
@@ -483,9 +495,10 @@ int per_block(corefl_ctx *c, F &&f) {
 // (inner-face halo); without inner faces a stage is one chain per block.
 int record_stage(corefl_ctx *c, int rk) {
   const Run &r = c->run;
+  StageScope scope(c);
   bool inner = false;
   for (const auto &b : c->blocks) inner = inner || !b.inner.empty();
-  const bool visc8 = r.viscous_order == 8;
+  const bool visc8 = r.viscous_order == 8, clear = !visc8 && !sweep_stores(r);
   int st;
   auto ops = [&](corefl_ctx::Block &b, std::initializer_list<int> list) -> int {
     for (int op : list) {
@@ -522,7 +535,7 @@ int record_stage(corefl_ctx *c, int rk) {
     // per-block order); the sweeps stay per block on the block streams
     if ((st = check_inner(c))) return st;
     const int nb = static_cast<int>(c->blocks.size());
-    if (!visc8) HIP_TRY(c, launch_zero_dq_multi(c->d_zones, nb, c->mb_interior, r.nv, c->stream));
+    if (clear) HIP_TRY(c, launch_zero_dq_multi(c->d_zones, nb, c->mb_interior, r.nv, c->stream));
     if (r.viscous_order && (st = per_block(c, viscous_head))) return st;
     if (visc8)
       for (auto &b : c->blocks)
@@ -563,13 +576,13 @@ int record_stage(corefl_ctx *c, int rk) {
   }
   if (!inner) {
     return per_block(c, [&](corefl_ctx::Block &b) -> int {
-      if ((!visc8 && (st = ops(b, {COREFL_OP_ZERO_DQ}))) || (st = viscous_head(b)) || (st = rhs_update(b))) return st;
+      if ((clear && (st = ops(b, {COREFL_OP_ZERO_DQ}))) || (st = viscous_head(b)) || (st = rhs_update(b))) return st;
       return closing(b);
     });
   }
   if ((st = check_inner(c))) return st;
   if ((st = per_block(c, [&](corefl_ctx::Block &b) -> int {
-         if (!visc8 && (st = ops(b, {COREFL_OP_ZERO_DQ}))) return st;
+         if (clear && (st = ops(b, {COREFL_OP_ZERO_DQ}))) return st;
          return viscous_head(b);
        })))
     return st;
@@ -1475,7 +1488,8 @@ int wu_step(corefl_ctx *c, double *dt_inout) {
 // in_step: a stage of corefl_step, whose state is seen after the last one only
 int run_stage(corefl_ctx *c, int rk, double dt, bool in_step) {
   int st;
-  if ((st = op_all(c, COREFL_OP_ZERO_DQ, rk, dt))) return st;
+  StageScope scope(c);
+  if (!sweep_stores(c->run) && (st = op_all(c, COREFL_OP_ZERO_DQ, rk, dt))) return st;
   if ((st = viscous_all(c, in_step && rk > 0))) return st;
   for (auto &b : c->blocks) {
     if ((st = op_block(c, COREFL_OP_CHEMISTRY, b, rk, dt))) return st;

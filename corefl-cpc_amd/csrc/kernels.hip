@@ -588,6 +588,35 @@ __device__ __noinline__ bool tt_temperature_pressure(const Zone &z, const Tab *_
 // total energy from primitives, compute_cv_from_bv_1_point + compute_total_energy
 // (1T), src/FieldOperation.cuh:90-161
 // ---------------------------------------------------------------------------
+// the conservative variables of one temperature at node p from its primitives b
+// (rho, u, v, w, p, T) and mass fractions y
+template <int M>
+DEV void cv_store(const Zone &z, const Tab *__restrict__ tb, long p, const double *b, const double *y) {
+  [[maybe_unused]] constexpr int NS = kNs(M);
+  const long sz = z.sz;
+  const double rho = b[0], u = b[1], v = b[2], w = b[3], pres = b[4], T = b[5];
+  z.cv[p] = rho;
+  z.cv[p + sz] = rho * u;
+  z.cv[p + 2 * sz] = rho * v;
+  z.cv[p + 3 * sz] = rho * w;
+#pragma unroll
+  for (int l = 0; l < NS; ++l) z.cv[p + (5 + l) * sz] = rho * y[l];
+  const double V2 = u * u + v * v + w * w;
+  double E = 0.5 * V2;
+  if constexpr (NS > 0) {
+    double h[NS];
+    thermo_h<M>(tb, T, h);
+#pragma unroll
+    for (int l = 0; l < NS; ++l) E += h[l] * y[l];
+    E *= rho;
+    E -= pres;
+  } else {
+    E *= rho;
+    E += pres / (kGammaAir - 1);
+  }
+  z.cv[p + 4 * sz] = E;
+}
+
 template <int M>
 DEV void cv_from_bv_point(const Zone &z, const Tab *__restrict__ tb, long p) {
   [[maybe_unused]] constexpr int NS = kNs(M);
@@ -633,6 +662,38 @@ DEV void cv_from_bv_point(const Zone &z, const Tab *__restrict__ tb, long p) {
   z.cv[p + 4 * sz] = E;
 }
 
+// the mean of two nodes' values, rounded by itself whatever consumes it
+DEV double mean2(double a, double b) {
+#pragma clang fp contract(off)
+  return 0.5 * (a + b);
+}
+
+// A boundary node's new state: bv, sv and the conservative variables.  With
+// FROM_REGS one temperature forms them from the values at hand: a boundary
+// kernel is a chain of memory latencies, and reading the node back doubles it.
+template <int M, bool FROM_REGS>
+DEV void node_store(const Zone &z, const Tab *__restrict__ tb, long p, const double *b, const double *sc) {
+  const long sz = z.sz;
+#pragma unroll
+  for (int l = 0; l < 6; ++l) z.bv[p + l * sz] = b[l];
+#pragma unroll
+  for (int l = 0; l < kNsc(M); ++l) z.sv[p + l * sz] = sc[l];
+  if constexpr (kTT(M) || !FROM_REGS)
+    cv_from_bv_point<M>(z, tb, p);
+  else
+    cv_store<M>(z, tb, p, b, sc);
+}
+template <int M>
+DEV void node_load(const Zone &z, long p, double *b, double *sc) {
+  const long sz = z.sz;
+#pragma unroll
+  for (int l = 0; l < 6; ++l) b[l] = z.bv[p + l * sz];
+#pragma unroll
+  for (int l = 0; l < kNsc(M); ++l) sc[l] = z.sv[p + l * sz];
+}
+template <int M>
+constexpr int kScArr = kNsc(M) > 0 ? kNsc(M) : 1;
+
 DEV void padded_ijk(const Zone &z, long t, int &i, int &j, int &k) {
   const long nxp = z.mx + 2 * z.ngg, nyp = z.my + 2 * z.ngg;
   i = static_cast<int>(t % nxp) - z.ngg;
@@ -654,10 +715,6 @@ __global__ void k_fill(double *p, long n, double v) {
 __global__ void k_copy(double *__restrict__ d, const double *__restrict__ s, long n) {
   const long t = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
   if (t < n) d[t] = s[t];
-}
-__global__ void k_scaled_copy(double *__restrict__ d, const double *__restrict__ s, double a, long n) {
-  const long t = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-  if (t < n) d[t] = a * s[t];
 }
 
 template <int M>
@@ -803,6 +860,69 @@ DEV void transport(const Tab *__restrict__ tb, double temperature, double mw_tot
 
 // update_physical_properties (1T) over the padded extent, src/FieldOperation.cuh:183-247
 template <int M>
+DEV void properties_point(const Zone &z, const Tab *__restrict__ tb, int transport_ghosts, long t) {
+  [[maybe_unused]] constexpr int NS = kNs(M);
+  int i, j, k;
+  padded_ijk(z, t, i, j, k);
+  const long p = z.ix(i, j, k), sz = z.sz;
+  const double T = z.bv[p + 5 * sz];
+  const double V = norm3(z.bv[p + sz], z.bv[p + 2 * sz], z.bv[p + 3 * sz]);
+  if constexpr (NS > 0) {
+    double cp[NS], y[NS];
+    thermo_cp<M>(tb, T, cp);
+    double imw = 0, cpt = 0;
+#pragma unroll
+    for (int l = 0; l < NS; ++l) {
+      y[l] = z.sv[p + l * sz];
+      imw = fma(y[l], tb->imw[l], imw);
+      cpt = fma(y[l], cp[l], cpt);
+    }
+    const double mw = 1 / fmax(imw, 1e-12);
+    const double R = kRu * imw;
+    if constexpr (kTT(M)) {
+      // translational-rotational gamma and sound speed, src/FieldOperation.cuh:207-229
+      double cv_tr, cpm, rm;
+      mix_tr_energy<M>(tb, T, y, cv_tr, cpm, rm);
+      const double gam = cpm / fmax(cv_tr, 1e-8);
+      z.gam[p] = gam;
+      const double c = sqrt(fmax(gam * rm * T, 1e-12));
+      z.acoustic[p] = c;
+      z.mach[p] = V / c;
+      if (z.tve[p] <= 0) z.tve[p] = T;
+    } else {
+      const double gam = cpt / (cpt - R);
+      z.gam[p] = gam;
+      const double c = sqrt(gam * R * T);
+      z.acoustic[p] = c;
+      z.mach[p] = V / c;
+    }
+    // The 8th-order viscous fluxes and the time-step bound read mu, kappa
+    // and rho*D at interior nodes only; the 2nd-order face scheme also reads
+    // them one node outside, so there the padded extent is covered.
+    if (transport_ghosts || (i >= 0 && i < z.mx && j >= 0 && j < z.my && k >= 0 && k < z.mz)) {
+      double rd[NS], mul, kap;
+      transport<M>(tb, T, mw, y, cp, mul, kap, rd);
+      z.mul[p] = mul;
+      z.kappa[p] = kap;
+      if constexpr (kTT(M)) {
+        double cv_ve = 0.0;
+        mix_ve_energy<M>(tb, z.tve[p], y, &cv_ve);
+        z.kappa_ve[p] = kap * cv_ve / fmax(cpt, 1e-8);
+      }
+#pragma unroll
+      for (int l = 0; l < NS; ++l) z.rhoD[p + l * sz] = rd[l];
+    }
+  } else {
+    constexpr double c_temp = kGammaAir * kRu / kMwAir;
+    z.mul[p] = sutherland(T);
+    z.mach[p] = V / sqrt(c_temp * T);
+  }
+}
+
+// The same at one node with the results held, for the 2-D closing kernel, which stores them on several planes
+// (holding them costs registers: the general kernel stores each as it is formed, 0.75 ms against 0.96 ms at
+// 256x128x128 with nine species).
+template <int M>
 struct PointProps {
   static constexpr int NS = kNs(M) > 0 ? kNs(M) : 1;
   double gam, c, mach, mul, kap, kappa_ve, cpt, y[NS], rd[NS];
@@ -872,20 +992,6 @@ DEV void properties_store(const Zone &z, long p, bool with_transport, const Poin
   } else {
     z.mul[p] = P.mul;
   }
-}
-
-// The 8th-order viscous fluxes and the time-step bound read mu, kappa and
-// rho*D at interior nodes only; the 2nd-order face scheme also reads them one
-// node outside, so there (transport_ghosts) the padded extent is covered.
-template <int M>
-DEV void properties_point(const Zone &z, const Tab *__restrict__ tb, int transport_ghosts, long t) {
-  int i, j, k;
-  padded_ijk(z, t, i, j, k);
-  const long p = z.ix(i, j, k);
-  const bool tr = transport_ghosts || (i >= 0 && i < z.mx && j >= 0 && j < z.my && k >= 0 && k < z.mz);
-  PointProps<M> P;
-  properties_eval<M>(z, tb, p, tr, P);
-  properties_store<M>(z, p, tr, P);
 }
 
 // A 2-D block's plane k = 0 closes a stage for its ghost planes too: the
@@ -2547,6 +2653,7 @@ struct WenoOpt {
   double pp_dt;          // DParameter::dt (fixed step) or 0: then dt_local of the face's left node
   double alpha;          // 1/3 in 3-D, 1/2 in 2-D
   double rho_ref, v_ref;
+  int store;             // the sweep is the stage's first contribution: dq is replaced, not read
 };
 
 // if_shock of the face whose left node is pf: a sensor value above the
@@ -3050,7 +3157,12 @@ __global__ __launch_bounds__(TX *TS) void k_weno(Zone z, const Tab *__restrict__
 #pragma unroll
     for (int l = 0; l < NV; ++l) {
       const double *fl = s + flux_plane(l) * PL;
-      z.dq[q + l * dsz] -= fl[me] - fl[left];
+      if constexpr (DIR == 0) {
+        const double old = o.store ? 0.0 : z.dq[q + l * dsz];
+        z.dq[q + l * dsz] = old - (fl[me] - fl[left]);
+      } else {
+        z.dq[q + l * dsz] -= fl[me] - fl[left];
+      }
     }
   }
 #undef SQ
@@ -3245,7 +3357,10 @@ __global__ __launch_bounds__(TX *TS) void k_weno_cp(Zone z, double eps_ref, Weno
     const long dsz = z.dsz;
     const int left = (ts - 1) * TX + tx;
 #pragma unroll
-    for (int l = 0; l < NV; ++l) z.dq[q + l * dsz] -= s[l * NT + me] - s[l * NT + left];
+    for (int l = 0; l < NV; ++l) {
+      const double old = o.store ? 0.0 : z.dq[q + l * dsz];
+      z.dq[q + l * dsz] = old - (s[l * NT + me] - s[l * NT + left]);
+    }
   }
 #undef FP
 #undef FM
@@ -4427,21 +4542,14 @@ __global__ __launch_bounds__(kFaceBlock) void k_periodic_flux_pair(Zone z, coref
 // (ghost layer g of a face node: the layers are independent of each other)
 template <int M>
 DEV void bc_outflow_layer(const Zone &z, const Tab *__restrict__ tb, int i, int j, int k, const int *d, int g) {
-  [[maybe_unused]] constexpr int NS = kNs(M);
-  const long p = z.ix(i, j, k), sz = z.sz;
-  const long pg = z.ix(i + g * d[0], j + g * d[1], k + g * d[2]);
-  double b6[6], sc[kNsc(M) > 0 ? kNsc(M) : 1];
-#pragma unroll
-  for (int l = 0; l < 6; ++l) b6[l] = z.bv[p + l * sz];
-#pragma unroll
-  for (int l = 0; l < kNsc(M); ++l) sc[l] = z.sv[p + l * sz];
-  [[maybe_unused]] const double tve = kTT(M) ? z.tve[p] : 0.0;
-#pragma unroll
-  for (int l = 0; l < 6; ++l) z.bv[pg + l * sz] = b6[l];
-#pragma unroll
-  for (int l = 0; l < kNsc(M); ++l) z.sv[pg + l * sz] = sc[l];
-  if constexpr (kTT(M)) z.tve[pg] = tve > 0.0 ? tve : b6[5];
-  cv_from_bv_point<M>(z, tb, pg);
+  const long p = z.ix(i, j, k), pg = z.ix(i + g * d[0], j + g * d[1], k + g * d[2]);
+  double b6[6], sc[kScArr<M>];
+  node_load<M>(z, p, b6, sc);
+  if constexpr (kTT(M)) {
+    const double tve = z.tve[p];
+    z.tve[pg] = tve > 0.0 ? tve : b6[5];
+  }
+  node_store<M, true>(z, tb, pg, b6, sc);
 }
 
 // The outflow faces of a block in one launch (blockIdx.y = face): a face writes
@@ -4490,37 +4598,25 @@ DEV void bc_symmetry_layer(const Zone &z, const Tab *__restrict__ tb, int i, int
   kx /= km;
   ky /= km;
   kz /= km;
-  if (layer == 0) {
-    const long pin = z.ix(i - d[0], j - d[1], k - d[2]);
-    const double u1 = z.bv[pin + sz], v1 = z.bv[pin + 2 * sz], w1 = z.bv[pin + 3 * sz];
-    const double u_k = kx * u1 + ky * v1 + kz * w1;
-    z.bv[p + sz] = u1 - kx * u_k;
-    z.bv[p + 2 * sz] = v1 - ky * u_k;
-    z.bv[p + 3 * sz] = w1 - kz * u_k;
-    z.bv[p] = z.bv[pin];
-    z.bv[p + 4 * sz] = z.bv[pin + 4 * sz];
-    z.bv[p + 5 * sz] = z.bv[pin + 5 * sz];
-#pragma unroll
-    for (int l = 0; l < kNsc(M); ++l) z.sv[p + l * sz] = z.sv[pin + l * sz];
-    if constexpr (kTT(M)) z.tve[p] = z.tve[pin];
-    cv_from_bv_point<M>(z, tb, p);
-    return;
-  }
-  const int g = layer;
-  const long pg = z.ix(i + g * d[0], j + g * d[1], k + g * d[2]);
-  const long pi = z.ix(i - g * d[0], j - g * d[1], k - g * d[2]);
-  z.bv[pg] = z.bv[pi];
-  const double u = z.bv[pi + sz], v = z.bv[pi + 2 * sz], w = z.bv[pi + 3 * sz];
+  // the face node takes its neighbour without the normal velocity, ghost g mirrors interior layer g
+  const int from = layer == 0 ? 1 : layer;
+  const long to = z.ix(i + layer * d[0], j + layer * d[1], k + layer * d[2]);
+  const long pi = z.ix(i - from * d[0], j - from * d[1], k - from * d[2]);
+  double b6[6], sc[kScArr<M>];
+  node_load<M>(z, pi, b6, sc);
+  const double u = b6[1], v = b6[2], w = b6[3];
   const double u_k = kx * u + ky * v + kz * w;
-  z.bv[pg + sz] = u - 2 * u_k * kx;
-  z.bv[pg + 2 * sz] = v - 2 * u_k * ky;
-  z.bv[pg + 3 * sz] = w - 2 * u_k * kz;
-  z.bv[pg + 4 * sz] = z.bv[pi + 4 * sz];
-  z.bv[pg + 5 * sz] = z.bv[pi + 5 * sz];
-#pragma unroll
-  for (int l = 0; l < kNsc(M); ++l) z.sv[pg + l * sz] = z.sv[pi + l * sz];
-  if constexpr (kTT(M)) z.tve[pg] = z.tve[pi];
-  cv_from_bv_point<M>(z, tb, pg);
+  if (layer == 0) {
+    b6[1] = u - kx * u_k;
+    b6[2] = v - ky * u_k;
+    b6[3] = w - kz * u_k;
+  } else {
+    b6[1] = u - 2 * u_k * kx;
+    b6[2] = v - 2 * u_k * ky;
+    b6[3] = w - 2 * u_k * kz;
+  }
+  if constexpr (kTT(M)) z.tve[to] = z.tve[pi];
+  node_store<M, true>(z, tb, to, b6, sc);
 }
 
 // The face node (layer 0) and the ghost layers read only interior nodes, so
@@ -4806,48 +4902,46 @@ DEV void inner_nodes(const InnerDev &f, long t, int *idx, int *it) {
 // Coincident-node threads write the target only on its face nodes, ghost
 // threads read it only inside, so the threads of one launch are independent.
 template <int M>
-__global__ void k_inner_comm(Zone z, Zone tz, const Tab *__restrict__ tb, InnerDev f, int n_scalar, long n) {
-  [[maybe_unused]] constexpr int NS = kNs(M);
+__global__ __launch_bounds__(kFaceBlock) void k_inner_comm(Zone z, Zone tz, const Tab *__restrict__ tb, InnerDev f,
+                                                           long n) {
   const long t = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
   if (t >= n) return;
   int idx[3], it[3];
   inner_nodes(f, t, idx, it);
   const long p = z.ix(idx[0], idx[1], idx[2]), q = tz.ix(it[0], it[1], it[2]);
-  const long sz = z.sz, tsz = tz.sz;
   const int face_dir = f.direction > 0 ? f.range_start[f.face] : f.range_end[f.face];
-  if (idx[f.face] == face_dir) {
-    const double u_this = norm3(z.bv[p + sz], z.bv[p + 2 * sz], z.bv[p + 3 * sz]);
-    if (fabs(u_this) > 1e-15) {
-      const double u_that = norm3(tz.bv[q + tsz], tz.bv[q + 2 * tsz], tz.bv[q + 3 * tsz]);
-      if (fabs(u_that) < 1e-15) {
-        for (int l = 0; l < 6; ++l) z.bv[p + l * sz] = tz.bv[q + l * tsz];
-        for (int l = 0; l < n_scalar; ++l) z.sv[p + l * sz] = tz.sv[q + l * tsz];
-        if constexpr (kTT(M)) z.tve[p] = tz.tve[q];
-      } else {
-        for (int l = 0; l < 6; ++l) {
-          const double ave = 0.5 * (tz.bv[q + l * tsz] + z.bv[p + l * sz]);
-          z.bv[p + l * sz] = ave;
-          tz.bv[q + l * tsz] = ave;
-        }
-        for (int l = 0; l < n_scalar; ++l) {
-          const double ave = 0.5 * (tz.sv[q + l * tsz] + z.sv[p + l * sz]);
-          z.sv[p + l * sz] = ave;
-          tz.sv[q + l * tsz] = ave;
-        }
-        if constexpr (kTT(M)) {
-          const double ave = 0.5 * (tz.tve[q] + z.tve[p]);
-          z.tve[p] = ave;
-          tz.tve[q] = ave;
-        }
-        cv_from_bv_point<M>(tz, tb, q);
-      }
-    }
-  } else {
-    for (int l = 0; l < 6; ++l) z.bv[p + l * sz] = tz.bv[q + l * tsz];
-    for (int l = 0; l < n_scalar; ++l) z.sv[p + l * sz] = tz.sv[q + l * tsz];
+  // both nodes' values are read before any is written (see cv_from_bv_point)
+  double a[6], b[6], sa[kScArr<M>], sb[kScArr<M>];
+  node_load<M>(tz, q, b, sb);
+  if (idx[f.face] != face_dir) {
     if constexpr (kTT(M)) z.tve[p] = tz.tve[q];
+    node_store<M, kNs(M) == 0>(z, tb, p, b, sb);
+    return;
   }
-  cv_from_bv_point<M>(z, tb, p);
+  node_load<M>(z, p, a, sa);
+  const double u_this = norm3(a[1], a[2], a[3]);
+  if (fabs(u_this) > 1e-15) {
+    const double u_that = norm3(b[1], b[2], b[3]);
+    if (fabs(u_that) < 1e-15) {
+#pragma unroll
+      for (int l = 0; l < 6; ++l) a[l] = b[l];
+#pragma unroll
+      for (int l = 0; l < kNsc(M); ++l) sa[l] = sb[l];
+      if constexpr (kTT(M)) z.tve[p] = tz.tve[q];
+    } else {
+#pragma unroll
+      for (int l = 0; l < 6; ++l) a[l] = mean2(b[l], a[l]);
+#pragma unroll
+      for (int l = 0; l < kNsc(M); ++l) sa[l] = mean2(sb[l], sa[l]);
+      if constexpr (kTT(M)) {
+        const double ave = 0.5 * (tz.tve[q] + z.tve[p]);
+        z.tve[p] = ave;
+        tz.tve[q] = ave;
+      }
+      node_store<M, kNs(M) == 0>(tz, tb, q, a, sa);
+    }
+  }
+  node_store<M, kNs(M) == 0>(z, tb, p, a, sa);
 }
 
 // inner_exchange(task 1), src/DataCommunication.cu:489-527: coincident nodes
@@ -4881,8 +4975,7 @@ __global__ void k_inner_flux(Zone z, Zone tz, InnerDev f, int nv, long n) {
 // nodes (bv, sv) and recompute cv there; ghosts copy the nodes beyond the
 // opposite face.  Ghost sources are interior nodes no thread of the launch writes.
 template <int M>
-__global__ void k_bc_periodic(Zone z, const Tab *__restrict__ tb, corefl_boundary b) {
-  [[maybe_unused]] constexpr int NS = kNs(M);
+__global__ __launch_bounds__(kFaceBlock) void k_bc_periodic(Zone z, const Tab *__restrict__ tb, corefl_boundary b) {
   FaceSite f;
   if (!face_site(z, b, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, f)) return;
   int o[3] = {f.i, f.j, f.k};
@@ -4892,47 +4985,28 @@ __global__ void k_bc_periodic(Zone z, const Tab *__restrict__ tb, corefl_boundar
   d[b.face] = b.direction;
   const long sz = z.sz;
   // all loads before the stores (see k_periodic_flux)
-  constexpr int NSC = kNsc(M) > 0 ? kNsc(M) : 1;
-  double a6[6], asc[NSC];
+  double a6[6], asc[kScArr<M>];
   if (f.layer == 0) {
     const long p = z.ix(f.i, f.j, f.k), po = z.ix(o[0], o[1], o[2]);
-    double b6[6], bsc[NSC];
+    double b6[6], bsc[kScArr<M>];
+    node_load<M>(z, p, a6, asc);
+    node_load<M>(z, po, b6, bsc);
 #pragma unroll
     for (int l = 0; l < 6; ++l) {
-      a6[l] = z.bv[p + l * sz];
-      b6[l] = z.bv[po + l * sz];
+      a6[l] = mean2(a6[l], b6[l]);
+      z.bv[po + l * sz] = a6[l];
     }
 #pragma unroll
     for (int l = 0; l < kNsc(M); ++l) {
-      asc[l] = z.sv[p + l * sz];
-      bsc[l] = z.sv[po + l * sz];
+      asc[l] = mean2(asc[l], bsc[l]);
+      z.sv[po + l * sz] = asc[l];
     }
-#pragma unroll
-    for (int l = 0; l < 6; ++l) {
-      const double ave = 0.5 * (a6[l] + b6[l]);
-      z.bv[p + l * sz] = ave;
-      z.bv[po + l * sz] = ave;
-    }
-#pragma unroll
-    for (int l = 0; l < kNsc(M); ++l) {
-      const double ave = 0.5 * (asc[l] + bsc[l]);
-      z.sv[p + l * sz] = ave;
-      z.sv[po + l * sz] = ave;
-    }
-    cv_from_bv_point<M>(z, tb, p);
+    node_store<M, kNs(M) == 0>(z, tb, p, a6, asc);
   } else {
     const int g = f.layer;
     const long pg = z.ix(f.i + g * d[0], f.j + g * d[1], f.k + g * d[2]);
-    const long pi = z.ix(o[0] + g * d[0], o[1] + g * d[1], o[2] + g * d[2]);
-#pragma unroll
-    for (int l = 0; l < 6; ++l) a6[l] = z.bv[pi + l * sz];
-#pragma unroll
-    for (int l = 0; l < kNsc(M); ++l) asc[l] = z.sv[pi + l * sz];
-#pragma unroll
-    for (int l = 0; l < 6; ++l) z.bv[pg + l * sz] = a6[l];
-#pragma unroll
-    for (int l = 0; l < kNsc(M); ++l) z.sv[pg + l * sz] = asc[l];
-    cv_from_bv_point<M>(z, tb, pg);
+    node_load<M>(z, z.ix(o[0] + g * d[0], o[1] + g * d[1], o[2] + g * d[2]), a6, asc);
+    node_store<M, kNs(M) == 0>(z, tb, pg, a6, asc);
   }
 }
 
@@ -4945,37 +5019,19 @@ __global__ __launch_bounds__(kFaceBlock) void k_bc_periodic_pair(Zone z, const T
   if (!face_site(z, lo, blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x, f)) return;
   const int a = lo.face;
   const int n = a == 0 ? z.mx : (a == 1 ? z.my : z.mz);
-  const long sz = z.sz;
-  constexpr int NSC = kNsc(M) > 0 ? kNsc(M) : 1;
-  double a6[6], asc[NSC], b6[6], bsc[NSC];
+  double a6[6], asc[kScArr<M>], b6[6], bsc[kScArr<M>];
   if (f.layer == 0) {
     int o[3] = {f.i, f.j, f.k};
     o[a] = n - 1;
     const long p = z.ix(f.i, f.j, f.k), po = z.ix(o[0], o[1], o[2]);
+    node_load<M>(z, p, a6, asc);
+    node_load<M>(z, po, b6, bsc);
 #pragma unroll
-    for (int l = 0; l < 6; ++l) {
-      a6[l] = z.bv[p + l * sz];
-      b6[l] = z.bv[po + l * sz];
-    }
+    for (int l = 0; l < 6; ++l) a6[l] = mean2(a6[l], b6[l]);
 #pragma unroll
-    for (int l = 0; l < kNsc(M); ++l) {
-      asc[l] = z.sv[p + l * sz];
-      bsc[l] = z.sv[po + l * sz];
-    }
-#pragma unroll
-    for (int l = 0; l < 6; ++l) {
-      const double ave = 0.5 * (a6[l] + b6[l]);
-      z.bv[p + l * sz] = ave;
-      z.bv[po + l * sz] = ave;
-    }
-#pragma unroll
-    for (int l = 0; l < kNsc(M); ++l) {
-      const double ave = 0.5 * (asc[l] + bsc[l]);
-      z.sv[p + l * sz] = ave;
-      z.sv[po + l * sz] = ave;
-    }
-    cv_from_bv_point<M>(z, tb, p);
-    cv_from_bv_point<M>(z, tb, po);
+    for (int l = 0; l < kNsc(M); ++l) asc[l] = mean2(asc[l], bsc[l]);
+    node_store<M, kNs(M) == 0>(z, tb, p, a6, asc);
+    node_store<M, kNs(M) == 0>(z, tb, po, a6, asc);
   } else {
     const int g = f.layer;
     int lg[3] = {f.i, f.j, f.k}, li[3] = {f.i, f.j, f.k}, hg[3] = {f.i, f.j, f.k}, hi[3] = {f.i, f.j, f.k};
@@ -4983,30 +5039,10 @@ __global__ __launch_bounds__(kFaceBlock) void k_bc_periodic_pair(Zone z, const T
     li[a] = n - 1 - g;
     hg[a] = n - 1 + g;
     hi[a] = g;
-    const long plg = z.ix(lg[0], lg[1], lg[2]), pli = z.ix(li[0], li[1], li[2]);
-    const long phg = z.ix(hg[0], hg[1], hg[2]), phi = z.ix(hi[0], hi[1], hi[2]);
-#pragma unroll
-    for (int l = 0; l < 6; ++l) {
-      a6[l] = z.bv[pli + l * sz];
-      b6[l] = z.bv[phi + l * sz];
-    }
-#pragma unroll
-    for (int l = 0; l < kNsc(M); ++l) {
-      asc[l] = z.sv[pli + l * sz];
-      bsc[l] = z.sv[phi + l * sz];
-    }
-#pragma unroll
-    for (int l = 0; l < 6; ++l) {
-      z.bv[plg + l * sz] = a6[l];
-      z.bv[phg + l * sz] = b6[l];
-    }
-#pragma unroll
-    for (int l = 0; l < kNsc(M); ++l) {
-      z.sv[plg + l * sz] = asc[l];
-      z.sv[phg + l * sz] = bsc[l];
-    }
-    cv_from_bv_point<M>(z, tb, plg);
-    cv_from_bv_point<M>(z, tb, phg);
+    node_load<M>(z, z.ix(li[0], li[1], li[2]), a6, asc);
+    node_load<M>(z, z.ix(hi[0], hi[1], hi[2]), b6, bsc);
+    node_store<M, kNs(M) == 0>(z, tb, z.ix(lg[0], lg[1], lg[2]), a6, asc);
+    node_store<M, kNs(M) == 0>(z, tb, z.ix(hg[0], hg[1], hg[2]), b6, bsc);
   }
 }
 
@@ -5294,12 +5330,6 @@ hipError_t launch_fill(double *p, long n, double v, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_scaled_copy(double *dst, const double *src, double a, long n, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_scaled_copy, dim3(blocks_for(n)), dim3(kBlock), 0, s, dst, src, a, n);
-  return hipGetLastError();
-}
-
 hipError_t launch_copy(double *dst, const double *src, long n, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_copy, dim3(blocks_for(n)), dim3(kBlock), 0, s, dst, src, n);
@@ -5362,7 +5392,7 @@ hipError_t launch_vt_relaxation(const Zone &z, const Run &r, const Tab *tb, doub
   return hipGetLastError();
 }
 
-hipError_t launch_inviscid(const Zone &z, const Run &r, const Tab *tb, int dir, hipStream_t s, int shape) {
+hipError_t launch_inviscid(const Zone &z, const Run &r, const Tab *tb, int dir, hipStream_t s, int shape, bool store) {
   const bool w7 = r.scheme == 72 || r.scheme == 71, charw = r.scheme == 52 || r.scheme == 72;
   if (!charw && r.scheme != 51 && r.scheme != 71) return hipErrorInvalidValue;
   if (r.hybrid && !z.sensor) return hipErrorInvalidValue;
@@ -5374,6 +5404,7 @@ hipError_t launch_inviscid(const Zone &z, const Run &r, const Tab *tb, int dir, 
   o.alpha = z.mz == 1 ? 0.5 : 1.0 / 3.0;
   o.rho_ref = r.rho_ref;
   o.v_ref = r.v_ref;
+  o.store = store ? 1 : 0;
   if (charw) {
     if (w7) {
       COREFL_DISPATCH(r.model, return (launch_weno_t<MV, true>(z, tb, dir, r.eps_ref, o, s, shape)));
@@ -5554,7 +5585,7 @@ hipError_t launch_bc_wall(const Zone &z, const Run &r, const Tab *tb, const core
 hipError_t launch_bc_periodic(const Zone &z, const Run &r, const Tab *tb, const corefl_boundary &b, hipStream_t s) {
   const long n = face_points(b) * (z.ngg + 1);
   COREFL_DISPATCH(r.model,
-                     hipLaunchKernelGGL((k_bc_periodic<MV>), dim3(blocks_for(n)), dim3(kBlock), 0, s, z, tb, b));
+                     hipLaunchKernelGGL((k_bc_periodic<MV>), dim3(blocks_for(n, kFaceBlock)), dim3(kFaceBlock), 0, s, z, tb, b));
   return hipGetLastError();
 }
 
@@ -5576,8 +5607,8 @@ hipError_t launch_periodic_flux_pair(const Zone &z, const Run &r, const corefl_b
 hipError_t launch_inner_comm(const Zone &z, const Zone &tz, const Run &r, const Tab *tb, const InnerDev &f,
                              hipStream_t s) {
   const long n = static_cast<long>(f.n_point[0]) * f.n_point[1] * f.n_point[2];
-  COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_inner_comm<MV>), dim3(blocks_for(n)), dim3(kBlock),
-                                                             0, s, z, tz, tb, f, r.n_scalar, n));
+  COREFL_DISPATCH(r.model, hipLaunchKernelGGL((k_inner_comm<MV>), dim3(blocks_for(n, kFaceBlock)), dim3(kFaceBlock),
+                                                             0, s, z, tz, tb, f, n));
   return hipGetLastError();
 }
 
@@ -5614,7 +5645,7 @@ hipError_t launch_local_dt(const Zone &z, const Run &r, const Tab *tb, double *d
   COREFL_DISPATCH(r.model,
                      hipLaunchKernelGGL((k_local_dt<MV>), dim3(nb), dim3(kBlock), 0, s, z, tb, r.cfl, r.prandtl,
                                         r.viscous_order, r.reaction, scratch, n));
-  hipLaunchKernelGGL(k_min_reduce, dim3(1), dim3(kBlock), 0, s, scratch, static_cast<long>(nb), dmin);
+  if (dmin) hipLaunchKernelGGL(k_min_reduce, dim3(1), dim3(kBlock), 0, s, scratch, static_cast<long>(nb), dmin);
   return hipGetLastError();
 }
 
@@ -5844,11 +5875,14 @@ __global__ __launch_bounds__(kBlock) void k_tube_dt(Zone z, TubePool P, double f
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_tube_dtc(TubePool P, const int *__restrict__ map, double *dtc, long n) {
+__global__ __launch_bounds__(kBlock) void k_tube_dtc(TubePool P, const int *__restrict__ map, double *dtc,
+                                                      double *dth, long n) {
   const long t = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
   if (t >= n) return;
   const int s = map[t];
-  dtc[t] = (s >= 0 && P.status[s] == 1) ? P.dt[s] : 0.0;
+  const double dt = (s >= 0 && P.status[s] == 1) ? P.dt[s] : 0.0;
+  dtc[t] = dt;
+  if (dth) dth[t] = 0.5 * dt;
 }
 
 __global__ void k_tube_finish(TubePool P, int n_slots) {
@@ -5906,9 +5940,9 @@ hipError_t launch_tube_dt(const Zone &z, const TubePool &P, int n_slots, hipStre
   return hipGetLastError();
 }
 
-hipError_t launch_tube_dtc(const Zone &z, const TubePool &P, const int *map, double *dtc, hipStream_t s) {
+hipError_t launch_tube_dtc(const Zone &z, const TubePool &P, const int *map, double *dtc, hipStream_t s, double *dth) {
   const long n = z.mx;
-  hipLaunchKernelGGL(k_tube_dtc, dim3(blocks_for(n)), dim3(kBlock), 0, s, P, map, dtc, n);
+  hipLaunchKernelGGL(k_tube_dtc, dim3(blocks_for(n)), dim3(kBlock), 0, s, P, map, dtc, dth, n);
   return hipGetLastError();
 }
 

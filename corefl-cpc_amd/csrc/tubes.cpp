@@ -143,13 +143,13 @@ int step_all_wu(corefl_tube_server *s, const corefl::Zone &z) {
   const long len = z.mx + 2L * z.ngg;
   Run rr = r;
   rr.reaction = 0;
-  THIP(s, launch_local_dt(z, rr, s->d_tables, s->d_dtc + s->cap, st));
+  THIP(s, launch_local_dt(z, rr, s->d_tables, nullptr, st));
   THIP(s, launch_tube_dt(z, s->pool, s->slot_high, st, s->fixed_dt));
-  THIP(s, launch_tube_dtc(z, s->pool, s->d_map, s->d_dtc, st));
-  THIP(s, launch_scaled_copy(s->d_dth, s->d_dtc, 0.5, z.mx, st));
-  THIP(s, launch_fill(z.dq, z.dsz * r.nv, 0.0, st));
-  THIP(s, launch_inviscid(z, r, s->d_tables, 0, st));
-  THIP(s, launch_copy(z.cn, z.dq, z.dsz * r.nv, st));
+  THIP(s, launch_tube_dtc(z, s->pool, s->d_map, s->d_dtc, st, s->d_dth));
+  // the x sweep is the whole transport part: stored, and the first one straight into Cn
+  Zone zc = z;
+  zc.dq = z.cn;
+  THIP(s, launch_inviscid(zc, r, s->d_tables, 0, st, 0, true));
   if (r.reaction) {
     if (s->jit.wu && r.chem_advance == 0)
       THIP(s, chem_jit_launch_wu(s->jit, z, 0.0, s->d_dtc, st));
@@ -160,8 +160,7 @@ int step_all_wu(corefl_tube_server *s, const corefl::Zone &z) {
   THIP(s, launch_properties_row(z, r, s->d_tables, st));
   THIP(s, launch_copy_planes(z.qn, z.cv, r.nv, z.sz, len, st));
   for (int rk = 0; rk < 3; ++rk) {
-    THIP(s, launch_fill(z.dq, z.dsz * r.nv, 0.0, st));
-    THIP(s, launch_inviscid(z, r, s->d_tables, 0, st));
+    THIP(s, launch_inviscid(z, r, s->d_tables, 0, st, 0, true));
     THIP(s, launch_update_rk_wu(z, r, s->d_tables, 0.0, rk, st, s->d_dth));
     THIP(s, launch_tube_bc(z, s->pool, r.model, s->d_tables, s->slot_high, st));
   }
@@ -176,19 +175,19 @@ int step_all(corefl_tube_server *s, const corefl::Zone &z) {
   hipStream_t st = s->stream;
   const long len = z.mx + 2L * z.ngg;
   THIP(s, launch_copy_planes(z.qn, z.cv, r.nv, z.sz, len, st));
-  // dt_local of every point; the row's minimum goes to a spare word (each tube takes its own)
-  THIP(s, launch_local_dt(z, r, s->d_tables, s->d_dtc + s->cap, st));
+  // dt_local of every point (each tube takes its own minimum)
+  THIP(s, launch_local_dt(z, r, s->d_tables, nullptr, st));
   THIP(s, launch_tube_dt(z, s->pool, s->slot_high, st, s->fixed_dt));
   THIP(s, launch_tube_dtc(z, s->pool, s->d_map, s->d_dtc, st));
   for (int rk = 0; rk < 3; ++rk) {
-    THIP(s, launch_fill(z.dq, z.dsz * r.nv, 0.0, st));
     if (r.reaction) {
+      THIP(s, launch_fill(z.dq, z.dsz * r.nv, 0.0, st));
       if (s->jit.fn)
         THIP(s, chem_jit_launch(s->jit, z, st));
       else
         THIP(s, launch_chemistry(z, r, s->d_tables, st));
     }
-    THIP(s, launch_inviscid(z, r, s->d_tables, 0, st));
+    THIP(s, launch_inviscid(z, r, s->d_tables, 0, st, 0, !r.reaction));
     THIP(s, launch_update_rk(z, r, s->d_tables, 0.0, rk, st, nullptr, s->d_dtc));
     THIP(s, launch_tube_bc(z, s->pool, r.model, s->d_tables, s->slot_high, st));
     THIP(s, launch_properties_row(z, r, s->d_tables, st));

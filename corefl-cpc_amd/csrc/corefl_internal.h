@@ -250,6 +250,21 @@ hipError_t launch_limit_flow(const Zone &z, const Run &r, const Tab *tb, hipStre
 hipError_t launch_inner_comm(const Zone &z, const Zone &tz, const Run &r, const Tab *tb, const InnerDev &f,
                              hipStream_t s);
 hipError_t launch_inner_flux(const Zone &z, const Zone &tz, const Run &r, const InnerDev &f, hipStream_t s);
+// one inner face of a multi-face launch: its block (the target block is in f) and its loop positions
+struct InnerItem {
+  int blk;
+  InnerDev f;
+  long n;
+};
+// faces that share no node, in one launch (zones in device memory, indexed by block)
+hipError_t launch_inner_comm_multi(const Zone *zs, const InnerItem *items, int n_items, long max_n, const Run &r,
+                                   const Tab *tb, hipStream_t s);
+hipError_t launch_inner_flux_multi(const Zone *zs, const InnerItem *items, int n_items, long max_n, const Run &r,
+                                   hipStream_t s);
+// The levels of an exchange: level[i] of face i (faces in exchange order, blk[i] its block) is one more than
+// that of every earlier face it shares a written node with.  Faces of one level are independent, and running
+// the levels in turn gives the results of the faces in turn.
+std::vector<int> inner_levels(const std::vector<InnerDev> &faces, const std::vector<int> &blk);
 // Writes dt_local and, unless dmin is null, the block minimum into *dmin (device scalar).
 hipError_t launch_local_dt(const Zone &z, const Run &r, const Tab *tb, double *dmin, hipStream_t s);
 // one boundary face of one block of a multi-block launch

@@ -67,6 +67,13 @@ struct corefl_ctx {
   corefl::BcItem *d_outflow = nullptr;
   int n_outflow = 0;
   long mb_interior = 0, mb_padded = 0, mb_face = 0;  // largest block / face
+  // the recorded exchange: the inner faces in device memory level by level (see inner_levels)
+  struct Level {
+    int first, n;
+    long most;
+  };
+  corefl::InnerItem *d_inner = nullptr;
+  std::vector<Level> levels;
   double *d_bmin = nullptr;   // [n_block] block dt minima
   hipGraphExec_t graph_exec = nullptr;
   double graph_dt = 0.0;      // fixed dt recorded in the graph
@@ -507,6 +514,26 @@ int record_stage(corefl_ctx *c, int rk) {
     }
     return 0;
   };
+  // the inner-face exchanges, one launch per level; a single block (periodic through an inner face onto
+  // itself) keeps a launch per face
+  auto exchange_state = [&]() -> int {
+    for (const auto &l : c->levels)
+      HIP_TRY(c, launch_inner_comm_multi(c->d_zones, c->d_inner + l.first, l.n, l.most, r, c->d_tables, c->stream));
+    if (c->levels.empty())
+      for (auto &b : c->blocks)
+        for (const InnerDev &f : b.inner)
+          HIP_TRY(c, launch_inner_comm(b.z, c->blocks[f.target_block].z, r, c->d_tables, f, c->stream));
+    return 0;
+  };
+  auto exchange_flux = [&]() -> int {
+    for (const auto &l : c->levels)
+      HIP_TRY(c, launch_inner_flux_multi(c->d_zones, c->d_inner + l.first, l.n, l.most, r, c->stream));
+    if (c->levels.empty())
+      for (auto &b : c->blocks)
+        for (const InnerDev &f : b.inner)
+          HIP_TRY(c, launch_inner_flux(b.z, c->blocks[f.target_block].z, r, f, c->stream));
+    return 0;
+  };
   auto viscous_head = [&](corefl_ctx::Block &b) -> int {
     hipStream_t s = c->cur;
     if (r.viscous_order == 2) HIP_TRY(c, launch_viscous2(b.z, r, c->d_tables, s, rk > 0 && b.z.mz == 1));
@@ -537,10 +564,7 @@ int record_stage(corefl_ctx *c, int rk) {
     const int nb = static_cast<int>(c->blocks.size());
     if (clear) HIP_TRY(c, launch_zero_dq_multi(c->d_zones, nb, c->mb_interior, r.nv, c->stream));
     if (r.viscous_order && (st = per_block(c, viscous_head))) return st;
-    if (visc8)
-      for (auto &b : c->blocks)
-        for (const InnerDev &f : b.inner)
-          HIP_TRY(c, launch_inner_flux(b.z, c->blocks[f.target_block].z, r, f, c->stream));
+    if (visc8 && (st = exchange_flux())) return st;
     if ((st = per_block(c, [&](corefl_ctx::Block &b) -> int {
            if ((st = viscous_tail(b))) return st;
            return ops(b, {COREFL_OP_CHEMISTRY, COREFL_OP_INVISCID_X, COREFL_OP_INVISCID_Y, COREFL_OP_INVISCID_Z});
@@ -566,9 +590,7 @@ int record_stage(corefl_ctx *c, int rk) {
                        return launch_bc_periodic_pair(b.z, r, c->d_tables, lo, c->stream);
                      }));
     }
-    for (auto &b : c->blocks)
-      for (const InnerDev &f : b.inner)
-        HIP_TRY(c, launch_inner_comm(b.z, c->blocks[f.target_block].z, r, c->d_tables, f, c->stream));
+    if ((st = exchange_state())) return st;
     for (auto &b : c->blocks)
       if ((st = ops(b, {COREFL_OP_K_GRADIENT}))) return st;
     HIP_TRY(c, launch_properties_multi(c->d_zones, nb, c->mb_padded, r, c->d_tables, c->stream));
@@ -586,14 +608,9 @@ int record_stage(corefl_ctx *c, int rk) {
          return viscous_head(b);
        })))
     return st;
-  if (visc8)
-    for (auto &b : c->blocks)
-      for (const InnerDev &f : b.inner)
-        HIP_TRY(c, launch_inner_flux(b.z, c->blocks[f.target_block].z, r, f, c->stream));
+  if (visc8 && (st = exchange_flux())) return st;
   if ((st = per_block(c, rhs_update))) return st;
-  for (auto &b : c->blocks)
-    for (const InnerDev &f : b.inner)
-      HIP_TRY(c, launch_inner_comm(b.z, c->blocks[f.target_block].z, r, c->d_tables, f, c->stream));
+  if ((st = exchange_state())) return st;
   return per_block(c, closing);
 }
 
@@ -626,43 +643,69 @@ void drop_graph(corefl_ctx *c) {
   c->graph_exec = nullptr;
   if (c->d_zones) (void)hipFree(c->d_zones);
   if (c->d_outflow) (void)hipFree(c->d_outflow);
+  if (c->d_inner) (void)hipFree(c->d_inner);
+  c->d_inner = nullptr;
+  c->levels.clear();
   c->d_zones = nullptr;
   c->d_outflow = nullptr;
   c->batched = false;
 }
 
-// Device tables for the multi-block launches (one-temperature runs with several blocks, none above
-// kBatchPoints interior points: larger blocks fill the GPU alone and gain more from running their
-// chains side by side on the block streams).
+// Device tables for the launches over several blocks: the zones and the inner faces in level order for every
+// run with several blocks, the outflow faces and the extents for the pointwise kernels (one-temperature runs,
+// no block above kBatchPoints interior points: larger blocks fill the GPU alone and gain more from running
+// their chains side by side on the block streams).
 constexpr long kBatchPoints = 1L << 20;
 
 int upload_block_tables(corefl_ctx *c) {
   const size_t nb = c->blocks.size();
-  if (nb < 2 || c->run.tt) return 0;
+  if (nb < 2) return 0;
+  std::vector<Zone> zs;
+  for (const auto &b : c->blocks) zs.push_back(b.z);
+  HIP_TRY(c, hipMalloc(&c->d_zones, nb * sizeof(Zone)));
+  HIP_TRY(c, hipMemcpy(c->d_zones, zs.data(), nb * sizeof(Zone), hipMemcpyHostToDevice));
+  // the inner faces in level order
+  std::vector<InnerDev> faces;
+  std::vector<int> blk;
+  for (size_t i = 0; i < nb; ++i)
+    for (const InnerDev &f : c->blocks[i].inner) {
+      faces.push_back(f);
+      blk.push_back(static_cast<int>(i));
+    }
+  if (!faces.empty()) {
+    const std::vector<int> level = inner_levels(faces, blk);
+    std::vector<InnerItem> items;
+    for (int l = 1; items.size() < faces.size(); ++l) {
+      corefl_ctx::Level lv{static_cast<int>(items.size()), 0, 0};
+      for (size_t i = 0; i < faces.size(); ++i) {
+        if (level[i] != l) continue;
+        const InnerDev &f = faces[i];
+        items.push_back({blk[i], f, static_cast<long>(f.n_point[0]) * f.n_point[1] * f.n_point[2]});
+        ++lv.n;
+        lv.most = std::max(lv.most, items.back().n);
+      }
+      c->levels.push_back(lv);
+    }
+    HIP_TRY(c, hipMalloc(&c->d_inner, items.size() * sizeof(InnerItem)));
+    HIP_TRY(c, hipMemcpy(c->d_inner, items.data(), items.size() * sizeof(InnerItem), hipMemcpyHostToDevice));
+  }
+  if (c->run.tt) return 0;
   for (const auto &b : c->blocks)
     if (static_cast<long>(b.z.mx) * b.z.my * b.z.mz > kBatchPoints) return 0;
-  std::vector<Zone> zs;
   std::vector<BcItem> out;
   c->mb_interior = c->mb_padded = c->mb_face = 0;
   for (size_t i = 0; i < nb; ++i) {
     const Zone &z = c->blocks[i].z;
-    zs.push_back(z);
     c->mb_interior = std::max<long>(c->mb_interior, static_cast<long>(z.mx) * z.my * z.mz);
     c->mb_padded = std::max<long>(c->mb_padded, static_cast<long>(z.mx + 2 * z.ngg) * (z.my + 2 * z.ngg) *
                                                     (z.mz + 2 * z.ngg));
-    for (const auto &f : c->blocks[i].faces) {
-      if (f.kind != COREFL_BC_OUTFLOW) continue;
-      BcItem it;
-      it.blk = static_cast<int>(i);
-      it.b = f.b;
-      out.push_back(it);
+    for (const auto &b : c->blocks[i].outflow) {
+      out.push_back({static_cast<int>(i), b});
       long n = 1;
-      for (int d = 0; d < 3; ++d) n *= f.b.range_end[d] - f.b.range_start[d] + 1;
+      for (int d = 0; d < 3; ++d) n *= b.range_end[d] - b.range_start[d] + 1;
       c->mb_face = std::max(c->mb_face, n * z.ngg);
     }
   }
-  HIP_TRY(c, hipMalloc(&c->d_zones, nb * sizeof(Zone)));
-  HIP_TRY(c, hipMemcpy(c->d_zones, zs.data(), nb * sizeof(Zone), hipMemcpyHostToDevice));
   c->n_outflow = static_cast<int>(out.size());
   HIP_TRY(c, hipMalloc(&c->d_outflow, std::max<size_t>(out.size(), 1) * sizeof(BcItem)));
   if (!out.empty())
@@ -823,6 +866,67 @@ void derive_tables(const corefl_chem_tables &in, Tab &out) {
       }
     }
   }
+}
+
+namespace {
+
+// an index box of one block
+struct Box {
+  int blk, lo[3], hi[3];
+};
+bool meet(const Box &a, const Box &b) {
+  if (a.blk != b.blk) return false;
+  for (int d = 0; d < 3; ++d)
+    if (a.hi[d] < b.lo[d] || b.hi[d] < a.lo[d]) return false;
+  return true;
+}
+
+// The nodes an inner face touches: it writes its own loop box (face node and ghosts) and the target's
+// coincident nodes, and reads the target's image of the loop box (inner_comm_point, inner_flux_point).
+struct FaceBoxes {
+  Box own, target_face, target;
+};
+FaceBoxes face_boxes(const InnerDev &f, int blk) {
+  FaceBoxes b{};
+  b.own.blk = blk;
+  b.target.blk = b.target_face.blk = f.target_block;
+  const int face_dir = f.direction > 0 ? f.range_start[f.face] : f.range_end[f.face];
+  for (int a = 0; a < 3; ++a) {
+    b.own.lo[a] = std::min(f.range_start[a], f.range_end[a]);
+    b.own.hi[a] = std::max(f.range_start[a], f.range_end[a]);
+    // target coordinate a follows the loop along source axis x
+    const int x = f.src_tar[a];
+    const int first = f.target_start[a];
+    const int last = first + f.target_loop_dir[a] * f.loop_dir[x] * (f.n_point[x] - 1);
+    b.target.lo[a] = b.target_face.lo[a] = std::min(first, last);
+    b.target.hi[a] = b.target_face.hi[a] = std::max(first, last);
+    if (x == f.face)
+      b.target_face.lo[a] = b.target_face.hi[a] =
+          first + f.target_loop_dir[a] * (face_dir - f.range_start[f.face]);
+  }
+  return b;
+}
+
+}  // namespace
+
+std::vector<int> inner_levels(const std::vector<InnerDev> &faces, const std::vector<int> &blk) {
+  std::vector<FaceBoxes> box;
+  std::vector<int> level;
+  for (size_t i = 0; i < faces.size(); ++i) {
+    box.push_back(face_boxes(faces[i], blk[i]));
+    const FaceBoxes &x = box[i];
+    int l = 1;
+    for (size_t j = 0; j < i; ++j) {
+      const FaceBoxes &y = box[j];
+      bool shared = false;
+      for (const Box *w : {&x.own, &x.target_face})
+        for (const Box *o : {&y.own, &y.target_face, &y.target}) shared = shared || meet(*w, *o);
+      for (const Box *w : {&y.own, &y.target_face}) shared = shared || meet(*w, x.target);
+      if (shared) l = std::max(l, level[j] + 1);
+    }
+    level.push_back(l);
+  }
+  return level;
 }
 
 static int sgn_of(int a) { return a < 0 ? -1 : 1; }  // gxl::sgn, src/gxl_lib/Math.hpp:10-12

@@ -1,0 +1,154 @@
+"""What a step does differently from its operators one by one, against those operators bit for bit: on a 2-D
+block the ghost planes are completed only where a stage reads them, the x sweep stores dq instead of adding to a
+cleared one, the recorded step exchanges independent inner faces in one launch; then outflow faces in numbers
+above one launch's list, and two-temperature tables outside the usual ones against the oracle."""
+import numpy as np
+import pytest
+
+from corefl_amd import (Solver, _abi, air5_box_case, load_air5_tables, load_tables, multiblock_case, sod_case,
+                        square_ogrid_case)
+from oracle import Oracle, air5_tables
+
+pytestmark = pytest.mark.gpu
+
+# one operator, FP64 sums of at most 27 terms against the same sums in another order
+STAGE_TOL = 1e-11
+STATE = (_abi.F_CV, _abi.F_BV, _abi.F_SV)
+OPS = [_abi.OP_ZERO_DQ, _abi.OP_VISCOUS, _abi.OP_CHEMISTRY, _abi.OP_INVISCID_X, _abi.OP_INVISCID_Y,
+       _abi.OP_INVISCID_Z, _abi.OP_UPDATE_RK, _abi.OP_LIMIT_FLOW, _abi.OP_BC, _abi.OP_HALO, _abi.OP_K_GRADIENT,
+       _abi.OP_PROPERTIES]
+
+
+def body_2d(mx, my):
+    t = load_air5_tables(True)
+    return [square_ogrid_case(mx, my, tables=t)], t, STATE + (_abi.F_TVE, _abi.F_GAMMA, _abi.F_KAPPA_VE)
+
+
+def plane_8th(mx, my):
+    t = load_air5_tables(True)
+    c = air5_box_case(mx, my, 1, seed=3, tables=t, two_temperature=True, ngg=4)
+    c.run.update(viscous_order=8, inviscid_scheme=72)
+    return [c], t, STATE + (_abi.F_TVE,)
+
+
+def plane_one_temperature(mx, my):
+    t = load_air5_tables(False)
+    return [air5_box_case(mx, my, 1, seed=4, tables=t)], t, STATE + (_abi.F_GAMMA, _abi.F_ACOUSTIC)
+
+
+def air_sod(mx, my):
+    return [sod_case(mx, my)], None, STATE[:2]
+
+
+def blocks(physics, visc):
+    def make(_mx, _my):
+        t = load_tables() if physics == "h2" else None
+        bl = multiblock_case(split=(3, 2, 2) if physics == "air" else (2, 2, 2), seed=5, physics=physics, rotate=True)
+        for c in bl:
+            c.run.update(viscous_order=visc)
+        return bl, t, STATE if physics == "h2" else STATE[:2]
+    return make
+
+
+@pytest.mark.parametrize("make,mx,my", [
+    (body_2d, 97, 33), (plane_8th, 33, 21), (plane_one_temperature, 65, 18), (air_sod, 101, 9),
+    (blocks("air", 0), 0, 0), (blocks("h2", 0), 0, 0), (blocks("h2", 8), 0, 0),
+], ids=["body", "plane8", "plane1t", "sod", "blocks_air", "blocks_h2", "blocks_h2_visc8"])
+def test_step_is_its_operators(make, mx, my):
+    bl, tb, fields = make(mx, my)
+    run = dict(bl[0].run, fixed_time_step=1)
+    s = {}
+    for way in ("ops", "step", "recorded"):
+        s[way] = Solver(dict(run, step_graph=int(way == "recorded")), tb)
+        for c in bl:
+            s[way].add_block(c)
+        s[way].initialize()
+    dt = 0.3 * s["ops"].cfl_dt()
+    for _ in range(3):
+        s["ops"].op(_abi.OP_COPY_QN)
+        for rk in range(3):
+            for op in OPS:
+                if op != _abi.OP_LIMIT_FLOW or run.get("limit_flow"):
+                    s["ops"].op(op, -1, rk, dt)
+        s["step"].step(dt)
+        s["recorded"].step(dt)
+        for b in range(len(bl)):
+            for f in fields:
+                ref = s["ops"].download(b, f)
+                for way in ("step", "recorded"):
+                    got = s[way].download(b, f)
+                    assert np.array_equal(got, ref), (way, b, f, np.abs(got - ref).max() / np.abs(ref).max())
+    for v in s.values():
+        v.close()
+
+
+@pytest.mark.parametrize("pieces", [8, 9, 19])
+def test_outflow_face_in_many_ranges(pieces):
+    """One outflow face and the same face cut into ranges give the same ghosts."""
+    t = load_air5_tables(True)
+    out = []
+    for n in (1, pieces):
+        c = square_ogrid_case(97, 25, tables=t)
+        kept, cut = [], []
+        for f in c.boundaries:
+            (cut if f[2] == 6 else kept).append(f)
+        for face, direction, label, a, b in cut:
+            edges = np.unique(np.linspace(a[0], b[0] + 1, n + 1).astype(int))
+            for lo, hi in zip(edges[:-1], edges[1:]):
+                kept.append((face, direction, label, (int(lo), a[1], a[2]), (int(hi) - 1, b[1], b[2])))
+        c.boundaries = kept
+        s = Solver(c.run, t)
+        s.add_block(c)
+        s.initialize()
+        rng = np.random.default_rng(1)
+        bv = s.download(0, _abi.F_BV)
+        s.upload(0, bv * rng.uniform(0.9, 1.1, bv.shape), s.download(0, _abi.F_SV))
+        s.op(_abi.OP_BC)
+        out.append([s.download(0, f) for f in STATE + (_abi.F_TVE,)])
+        s.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("change", ["exponents", "order"])
+def test_two_temperature_tables_outside_the_usual(change):
+    """Reaction-temperature exponents other than the three usual pairs, and electronic levels in falling order
+    with one of weight 0 (no early end of the sums)."""
+    tables, ref = load_air5_tables(True), air5_tables(two_temperature=True)
+    for t in (tables, ref):
+        if change == "exponents":
+            t.trx_model = 1
+            for r in range(0, t.n_reac, 2):
+                t.tcf_a[r], t.tcf_b[r] = 0.65, 0.35
+                t.tcb_a[r], t.tcb_b[r] = 0.25, 0.75
+        else:
+            for l in range(t.n_spec):
+                n = t.n_elec[l]
+                th, g = list(t.elec_theta[l][:n])[::-1], list(t.elec_g[l][:n])[::-1]
+                for j in range(n):
+                    t.elec_theta[l][j], t.elec_g[l][j] = th[j], g[j]
+                if n > 3:
+                    t.elec_g[l][1] = 0.0
+    case = air5_box_case(17, 11, 9, seed=12, tables=tables, two_temperature=True)
+    s = Solver(case.run, tables)
+    s.add_block(case)
+    o = Oracle(case, ref)
+    s.initialize()
+    o.initialize()
+
+    def close(a, b):
+        a, b = a.reshape(a.shape[0], -1), b.reshape(b.shape[0], -1)
+        den = np.abs(b).max(axis=1)
+        if len(den) > 4:
+            den[1:4] = den[1:4].max()
+        err = np.abs(a - b).max(axis=1) / np.maximum(den, 1e-300)
+        assert np.all(err <= STAGE_TOL), err
+
+    g = case.ngg
+    close(s.download(0, _abi.F_SV)[:, g:-g, g:-g, g:-g], o.a["sv"][:, g:-g, g:-g, g:-g])
+    s.op(_abi.OP_ZERO_DQ)
+    o.op("zero_dq")
+    s.op(_abi.OP_CHEMISTRY)
+    o.op("chemistry")
+    close(s.download(0, _abi.F_DQ), o.a["dq"])
+    s.close()

@@ -143,6 +143,8 @@ struct Tab : corefl_chem_tables {
   double elec_first[COREFL_MAX_SPEC], elec_stop[COREFL_MAX_SPEC];
   // which of the usual control temperatures a reaction's rates take: 0 T, 1 sqrt(T Tve), 2 Tve, -1 another
   int tcf_set[COREFL_MAX_REAC], tcb_set[COREFL_MAX_REAC];
+  static_assert(COREFL_MAX_REAC <= 64, "one bit a reaction");
+  unsigned long long odd_orders;  // bit r: a stoichiometric coefficient of reaction r is negative or above 3
   Reac reac[COREFL_MAX_REAC];
 };
 void derive_tables(const corefl_chem_tables &in, Tab &out);

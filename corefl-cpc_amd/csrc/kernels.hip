@@ -4757,14 +4757,17 @@ __global__ __launch_bounds__(kFaceBlock) void k_bc_inflow(Zone z, const Tab *__r
 
 // project_to_interior in apply_wall, src/BoundCond.cu:3070-3087: a reference
 // node lying on another physical face moves one node inward along that axis.
+// (The face labels of a 2-D block are those of its one plane: the reference node of a face on the k axis is a
+// ghost.)
 DEV void project_to_interior(const Zone &z, int *ix) {
-  if (ix[0] <= 0 && z.bt_il[ix[1] + ix[2] * z.my] != 0)
+  const int k = z.mz > 1 ? ix[2] : 0;
+  if (ix[0] <= 0 && z.bt_il[ix[1] + k * z.my] != 0)
     ix[0] = 1;
-  else if (ix[0] >= z.mx - 1 && z.bt_ir[ix[1] + ix[2] * z.my] != 0)
+  else if (ix[0] >= z.mx - 1 && z.bt_ir[ix[1] + k * z.my] != 0)
     ix[0] = z.mx - 2;
-  if (ix[1] <= 0 && z.bt_jl[ix[0] + ix[2] * z.mx] != 0)
+  if (ix[1] <= 0 && z.bt_jl[ix[0] + k * z.mx] != 0)
     ix[1] = 1;
-  else if (ix[1] >= z.my - 1 && z.bt_jr[ix[0] + ix[2] * z.mx] != 0)
+  else if (ix[1] >= z.my - 1 && z.bt_jr[ix[0] + k * z.mx] != 0)
     ix[1] = z.my - 2;
   if (z.mz > 1) {
     if (ix[2] <= 0 && z.bt_kl[ix[0] + ix[1] * z.mx] != 0)

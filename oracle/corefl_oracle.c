@@ -2951,15 +2951,17 @@ static void bc_inflow(oc_zone *z, const oc_run *r, const oc_tables *tb, const oc
 }
 
 /* project_to_interior in apply_wall, src/BoundCond.cu:3070-3087: a reference
- * node on another physical face moves one node inward along that axis. */
+ * node on another physical face moves one node inward along that axis (the
+ * face labels of a 2-D block are those of its one plane). */
 static void project_to_interior(const oc_zone *z, int *ix) {
-  if (ix[0] <= 0 && z->btype_il[ix[1] + ix[2] * z->my] != 0)
+  const int k = z->mz > 1 ? ix[2] : 0;
+  if (ix[0] <= 0 && z->btype_il[ix[1] + k * z->my] != 0)
     ix[0] = 1;
-  else if (ix[0] >= z->mx - 1 && z->btype_ir[ix[1] + ix[2] * z->my] != 0)
+  else if (ix[0] >= z->mx - 1 && z->btype_ir[ix[1] + k * z->my] != 0)
     ix[0] = z->mx - 2;
-  if (ix[1] <= 0 && z->btype_jl[ix[0] + ix[2] * z->mx] != 0)
+  if (ix[1] <= 0 && z->btype_jl[ix[0] + k * z->mx] != 0)
     ix[1] = 1;
-  else if (ix[1] >= z->my - 1 && z->btype_jr[ix[0] + ix[2] * z->mx] != 0)
+  else if (ix[1] >= z->my - 1 && z->btype_jr[ix[0] + k * z->mx] != 0)
     ix[1] = z->my - 2;
   if (z->mz > 1) {
     if (ix[2] <= 0 && z->btype_kl[ix[0] + ix[1] * z->mx] != 0)

@@ -8,7 +8,7 @@ wall Tve from the wall temperature or the interior)."""
 import numpy as np
 import pytest
 
-from corefl_amd import CoreflError, Solver, _abi, channel_case, load_air5_tables, load_tables
+from corefl_amd import CoreflError, Solver, _abi, air5_box_case, channel_case, load_air5_tables, load_tables
 from oracle import Oracle, air5_tables
 
 pytestmark = pytest.mark.gpu
@@ -74,6 +74,29 @@ def test_channel_boundary_parity(tables, h2_oracle_tables, physics, subsonic):
             dg, do = s.step(), o.step(fixed=False)
             assert abs(dg - do) <= 1e-12 * do
     check(s, o, case, LONG_TOL, " after 11 steps")
+    s.close()
+
+
+@pytest.mark.parametrize("two_temperature", [False, True])
+@pytest.mark.parametrize("low,high", [(2, 21), (21, 2), (2, 3)])
+def test_k_walls_of_a_plane(two_temperature, low, high):
+    """Walls on the k faces of a one-plane block: their reference nodes are ghosts, and the labels of the other
+    faces beside them are those of the plane."""
+    tb, oc = load_air5_tables(two_temperature), air5_tables(two_temperature)
+    case = air5_box_case(19, 13, 1, seed=6, tables=tb, two_temperature=two_temperature)
+    end = (case.mx - 1, case.my - 1, 0)
+    case.boundaries = list(case.boundaries) + [(2, -1, low, (0, 0, 0), end), (2, 1, high, (0, 0, 0), end)]
+    case.conditions = [dict(label=2, kind=2, thermal_type=0, wall_temperature=1500.0),
+                       dict(label=21, kind=2, thermal_type=1), dict(label=3, kind=3)]
+    s = Solver(case.run, tb)
+    s.add_block(case)
+    o = Oracle(case, oc)
+    s.initialize()
+    o.initialize()
+    check(s, o, case, STAGE_TOL, " after initialize")
+    s.op(_abi.OP_BC)
+    o.op("bc")
+    check(s, o, case, STAGE_TOL, " after the boundary conditions")
     s.close()
 
 

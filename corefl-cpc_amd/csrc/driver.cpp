@@ -38,6 +38,7 @@ struct corefl_ctx {
     corefl::Zone z{};
     std::vector<Face> faces;
     std::vector<corefl_boundary> outflow;  // the outflow faces, launched together
+    bool k_faces = false;                  // boundary faces on the k axis (of a 2-D block: they read its ghost planes)
     std::vector<corefl::InnerDev> inner;
     std::vector<void *> allocs;
     int shape[3] = {0, 0, 0};  // tile shape of each direction's characteristic WENO sweep
@@ -403,8 +404,11 @@ int close_block(corefl_ctx *c, corefl_ctx::Block &b, bool planes) {
 }
 
 // Whether a stage inside a step leaves a 2-D block's ghost planes complete: the last one does; the 8th-order
-// viscous terms read them in every stage (the 2nd-order ones only as differences that are 0).
-bool stage_fills_planes(const Run &r, int rk) { return rk == 2 || r.viscous_order == 8; }
+// viscous terms read them in every stage (the 2nd-order ones only as differences that are 0), and so do the
+// characteristic inflow, symmetry and wall conditions of a face on the k axis.
+bool stage_fills_planes(const Run &r, const corefl_ctx::Block &b, int rk) {
+  return rk == 2 || r.viscous_order == 8 || b.k_faces;
+}
 
 // data_communication: inner faces of every block in block and face order,
 // src/DataCommunication.cu:6-35
@@ -555,7 +559,7 @@ int record_stage(corefl_ctx *c, int rk) {
     return ops(b, {COREFL_OP_CHEMISTRY, COREFL_OP_INVISCID_X, COREFL_OP_INVISCID_Y, COREFL_OP_INVISCID_Z,
                    COREFL_OP_UPDATE_RK, COREFL_OP_LIMIT_FLOW, COREFL_OP_BC});
   };
-  auto closing = [&](corefl_ctx::Block &b) -> int { return close_block(c, b, stage_fills_planes(r, rk)); };
+  auto closing = [&](corefl_ctx::Block &b) -> int { return close_block(c, b, stage_fills_planes(r, b, rk)); };
   if (inner && c->batched) {
     // the same stage with the block-local pointwise operators and the outflow faces of all blocks in one
     // launch each (blocks are independent between the flux exchange and the halo, so this is the
@@ -1299,6 +1303,7 @@ int corefl_block_add(corefl_ctx *c, const corefl_block_desc *d, int *block_id) {
       return fail(c, Status::Arg, "boundary face does not lie on the block face");
     b.faces.push_back(face);
     if (face.kind == COREFL_BC_OUTFLOW) b.outflow.push_back(bf);
+    b.k_faces = b.k_faces || bf.face == 2;
   }
   if (d->n_inner < 0 || (d->n_inner > 0 && !d->inner)) return fail(c, Status::Arg, "bad inner face list");
   for (int f = 0; f < d->n_inner; ++f) {
@@ -1608,7 +1613,7 @@ int run_stage(corefl_ctx *c, int rk, double dt, bool in_step) {
   }
   if ((st = op_all(c, COREFL_OP_HALO, rk, dt))) return st;
   for (auto &b : c->blocks)
-    if ((st = close_block(c, b, !in_step || stage_fills_planes(c->run, rk)))) return st;
+    if ((st = close_block(c, b, !in_step || stage_fills_planes(c->run, b, rk)))) return st;
   return 0;
 }
 

@@ -36,6 +36,19 @@ def plane_one_temperature(mx, my):
     return [air5_box_case(mx, my, 1, seed=4, tables=t)], t, STATE + (_abi.F_GAMMA, _abi.F_ACOUSTIC)
 
 
+def plane_k_faces(low, high):
+    """A plane with boundary faces on its k axis: those read the ghost planes in every stage."""
+    def make(mx, my):
+        t = load_air5_tables(False)
+        c = air5_box_case(mx, my, 1, seed=6, tables=t)
+        end = (mx - 1, my - 1, 0)
+        c.boundaries = list(c.boundaries) + [(2, -1, low, (0, 0, 0), end), (2, 1, high, (0, 0, 0), end)]
+        c.conditions = [dict(label=2, kind=2, thermal_type=0, wall_temperature=1500.0),
+                        dict(label=21, kind=2, thermal_type=1), dict(label=3, kind=3)]
+        return [c], t, STATE
+    return make
+
+
 def air_sod(mx, my):
     return [sod_case(mx, my)], None, STATE[:2]
 
@@ -52,8 +65,9 @@ def blocks(physics, visc):
 
 @pytest.mark.parametrize("make,mx,my", [
     (body_2d, 97, 33), (plane_8th, 33, 21), (plane_one_temperature, 65, 18), (air_sod, 101, 9),
+    (plane_k_faces(3, 21), 33, 21), (plane_k_faces(21, 2), 33, 21),
     (blocks("air", 0), 0, 0), (blocks("h2", 0), 0, 0), (blocks("h2", 8), 0, 0),
-], ids=["body", "plane8", "plane1t", "sod", "blocks_air", "blocks_h2", "blocks_h2_visc8"])
+], ids=["body", "plane8", "plane1t", "sod", "k_symmetry", "k_walls", "blocks_air", "blocks_h2", "blocks_h2_visc8"])
 def test_step_is_its_operators(make, mx, my):
     bl, tb, fields = make(mx, my)
     run = dict(bl[0].run, fixed_time_step=1)

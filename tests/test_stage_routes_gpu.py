@@ -5,8 +5,9 @@ above one launch's list, and two-temperature tables outside the usual ones again
 import numpy as np
 import pytest
 
-from corefl_amd import (Solver, _abi, air5_box_case, load_air5_tables, load_tables, multiblock_case, sod_case,
-                        square_ogrid_case)
+from corefl_amd import (Solver, _abi, air5_box_case, channel_case, load_air5_tables, load_tables, multiblock_case,
+                        sod_case, square_ogrid_case)
+from corefl_amd.cases import Case
 from oracle import Oracle, air5_tables
 
 pytestmark = pytest.mark.gpu
@@ -49,6 +50,43 @@ def plane_k_faces(low, high):
     return make
 
 
+def joined_planes(physics):
+    """A 2-D channel cut into 2 x 2 one-plane blocks joined at inner faces (their common lines belong to both)."""
+    def make(mx, my):
+        tt = physics == "air5"
+        t = None if physics == "air" else load_air5_tables(True) if tt else load_tables()
+        w = channel_case(mx, my, 1, physics=physics, seed=8)
+        g, ci, cj = w.ngg, mx // 2, my // 3
+        spans = [((0, ci), (0, cj)), ((ci, mx - 1), (0, cj)), ((0, ci), (cj, my - 1)), ((ci, mx - 1), (cj, my - 1))]
+        size = [(i1 - i0 + 1, j1 - j0 + 1) for (i0, i1), (j0, j1) in spans]
+        out = []
+        for n, ((i0, i1), (j0, j1)) in enumerate(spans):
+            m, faces, inner = size[n], [], []
+            cut = np.s_[..., j0:j1 + 1 + 2 * g, i0:i1 + 1 + 2 * g]
+            for axis in (0, 1):
+                for side in (-1, 1):
+                    at = 0 if side < 0 else m[axis] - 1
+                    lo, hi = [0, 0, 0], [m[0] - 1, m[1] - 1, 0]
+                    lo[axis] = hi[axis] = at
+                    high_block = bool(n & (1 << axis))
+                    if high_block == (side > 0):  # an outer side
+                        label = [f[2] for f in w.boundaries if f[0] == axis and f[1] == side][0]
+                        faces.append((axis, side, label, lo, hi))
+                        continue
+                    o = n ^ (1 << axis)
+                    src, tar = [1, m[0], -1, -m[1], 1, 1], [1, size[o][0], -1, -size[o][1], 1, 1]
+                    src[2 * axis:2 * axis + 2] = [at + 1] * 2
+                    tar[2 * axis:2 * axis + 2] = [1 if side > 0 else size[o][axis]] * 2
+                    inner.append((src, tar, o + 1))
+            c = Case(m[0], m[1], 1, g, *(np.ascontiguousarray(a[cut]) for a in (w.metric, w.jac, w.bv, w.sv)), faces,
+                     dict(w.run), inner=inner, conditions=w.conditions)
+            if tt:
+                c.tve = np.ascontiguousarray(w.tve[cut])
+            out.append(c)
+        return out, t, STATE + (_abi.F_TVE,) if tt else STATE if physics == "h2" else STATE[:2]
+    return make
+
+
 def air_sod(mx, my):
     return [sod_case(mx, my)], None, STATE[:2]
 
@@ -66,8 +104,10 @@ def blocks(physics, visc):
 @pytest.mark.parametrize("make,mx,my", [
     (body_2d, 97, 33), (plane_8th, 33, 21), (plane_one_temperature, 65, 18), (air_sod, 101, 9),
     (plane_k_faces(3, 21), 33, 21), (plane_k_faces(21, 2), 33, 21),
+    (joined_planes("air"), 41, 33), (joined_planes("air5"), 41, 33), (joined_planes("h2"), 41, 33),
     (blocks("air", 0), 0, 0), (blocks("h2", 0), 0, 0), (blocks("h2", 8), 0, 0),
-], ids=["body", "plane8", "plane1t", "sod", "k_symmetry", "k_walls", "blocks_air", "blocks_h2", "blocks_h2_visc8"])
+], ids=["body", "plane8", "plane1t", "sod", "k_symmetry", "k_walls", "joined_air",
+        "joined_body", "joined_h2", "blocks_air", "blocks_h2", "blocks_h2_visc8"])
 def test_step_is_its_operators(make, mx, my):
     bl, tb, fields = make(mx, my)
     run = dict(bl[0].run, fixed_time_step=1)

@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include <map>
 #include <string>
 #include <variant>
@@ -215,10 +217,13 @@ hipError_t launch_inviscid(const Zone &z, const Run &r, const Tab *tb, int dir, 
 hipError_t launch_shock_sensor(const Zone &z, const Run &r, hipStream_t s);
 hipError_t launch_reactors(const ReactorPool &p, int model, const Tab *tb, int max_steps, hipStream_t s);
 // the same step with one wave per slot, over slots [0, n_slots).  The servers take it while at most
-// kReactorWaveSlots slots are in flight: a wave per slot steps about 80 reactors a microsecond once the
-// GPU is full, a lane per slot takes 212 us a step however few of its lanes are used (up to 65,536), so
-// the lines cross near 16,000 slots (5000: 58 us against 212).
-constexpr int kReactorWaveSlots = 16384;
+// reactor_wave_slots slots are in flight.  With the GPU full a wave per slot takes a time in proportion to the
+// slots, a lane per slot nearly the same time for any number, and a lane's step grows with the species and the
+// reactions while a wave's has lanes to spare, so the lines cross later for the larger mechanism.  Fixed ROK4E
+// steps, wave against lane (us): 9 species and 19 reactions, 12,000 slots 187 / 204, 14,000 217 / 207; 9 and 6,
+// 8,000 87 / 101, 10,000 107 / 104; 5 and 17 (NASA-9), 6,000 99 / 115, 8,000 129 / 117; 5 and 5, 4,000 39 / 44,
+// 5,000 48 / 46.  SSP-RK3 crosses up to a fifth earlier, the point-implicit scheme later.
+inline int reactor_wave_slots(int ns, int n_reac) { return std::min(16384, ns * (700 + 35 * n_reac)); }
 hipError_t launch_reactors_wave(const ReactorPool &p, int model, const Tab *tb, int max_steps, int n_slots,
                                 hipStream_t s);
 hipError_t launch_reactor_admit(const ReactorPool &p, int model, const Tab *tb, const double *req, int n_req,

@@ -145,9 +145,11 @@ int corefl_serve_run_noalloc(const corefl_chem_tables *tables, const corefl_reac
   NA_HIP(hipMemcpy(d_rec, g_rec, static_cast<size_t>(n) * R * sizeof(double), hipMemcpyHostToDevice));
   // every slot's fields, its status included, are written by the admission: nothing stale is read
   NA_HIP(corefl::launch_reactor_admit(P, model, d_tab, d_rec, n, nullptr));
-  // the server's kernel choice: one wave per slot while few slots are in flight
+  // the server's kernel choice: one wave per slot while few slots are in flight (a small mechanism's line lies
+  // below COREFL_NOALLOC_MAX_REACTORS)
+  const int wave_slots = corefl::reactor_wave_slots(ns, tables->n_reac);
   for (int active = n; active > 0;) {
-    if (active <= corefl::kReactorWaveSlots)
+    if (active <= wave_slots)
       NA_HIP(corefl::launch_reactors_wave(P, model, d_tab, steps_per_launch, n, nullptr));
     else
       NA_HIP(corefl::launch_reactors(P, model, d_tab, steps_per_launch, nullptr));

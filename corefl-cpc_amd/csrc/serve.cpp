@@ -192,7 +192,7 @@ int corefl_serve_progress(corefl_server *s, int *pending) {
   if (s->in_flight > 0) {
     // few slots in flight: one wave per slot (latency); many: one lane per slot (throughput).  Both give
     // the same results bit for bit, so a request's result does not depend on the load.
-    if (s->in_flight <= corefl::kReactorWaveSlots)
+    if (s->in_flight <= corefl::reactor_wave_slots(s->ns, s->host.n_reac))
       SHIP(s, corefl::launch_reactors_wave(P, s->model, s->d_tables, s->steps_per_launch, s->high_water, s->stream));
     else
       SHIP(s, corefl::launch_reactors(P, s->model, s->d_tables, s->steps_per_launch, s->stream));

@@ -1,5 +1,8 @@
 """The size rules that split a kernel's work over more or fewer threads, against the oracle at sizes on
 both sides of each rule and at ragged ends of its tiles."""
+import re
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -25,14 +28,26 @@ def tables():
     return load_tables()
 
 
-@pytest.mark.parametrize("mx,my,mz", [
-    (16, 9, 5),        # one short chunk of k (4 nodes and 1), boundary closures from both ends
-    (21, 13, 18),      # the 4-node chunks with a remainder
-    (96, 70, 37),      # 16-node chunks, components over blocks, remainder of 5
-    (520, 510, 9),     # enough columns for all components in one block
+def column_split(mx, my, mz, fields):
+    """column_split of the kernels: (k nodes of a chunk, fields of a block)."""
+    src = (Path(__file__).parent.parent / "corefl-cpc_amd" / "csrc" / "kernels.hip").read_text()
+    most = int(re.search(r"constexpr long kColumnWaves = (\d+);", src)[1])
+    waves = (mx * my * -(-mz // 16) + 63) // 64
+    per_block = max(1, waves * fields // most) if waves * 2 < most else fields
+    return (4 if per_block == 1 and waves * fields < most // 2 else 16), per_block
+
+
+@pytest.mark.parametrize("mx,my,mz,chunk,per_block", [
+    (16, 9, 5, 4, 1),        # one short chunk of k (4 nodes and 1), boundary closures from both ends
+    (21, 13, 18, 4, 1),      # the 4-node chunks with a remainder
+    (96, 70, 37, 4, 1),      # the last size before the long chunks
+    (101, 67, 53, 16, 1),    # 16-node chunks, a component to a block, remainder of 5
+    (250, 170, 20, 16, 2),   # a few components to a block, the last block's fewer
+    (520, 510, 9, 16, 13),   # enough columns for all components in one block
 ])
-def test_viscous_column_splits(tables, h2_oracle_tables, mx, my, mz):
+def test_viscous_column_splits(tables, h2_oracle_tables, mx, my, mz, chunk, per_block):
     """8th-order viscous operator between walls, inflow, outflow and symmetry planes."""
+    assert column_split(mx, my, mz, 13) == (chunk, per_block)
     case = channel_case(mx, my, mz, physics="h2", seed=mx)
     s = Solver(case.run, tables)
     s.add_block(case)

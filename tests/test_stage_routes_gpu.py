@@ -1,12 +1,13 @@
 """What a step does differently from its operators one by one, against those operators bit for bit: on a 2-D
 block the ghost planes are completed only where a stage reads them, the x sweep stores dq instead of adding to a
-cleared one, the recorded step exchanges independent inner faces in one launch; then outflow faces in numbers
-above one launch's list, and two-temperature tables outside the usual ones against the oracle."""
+cleared one (or the viscous derivative stores it, in each of its splits), the recorded step exchanges independent
+inner faces in one launch; then outflow faces in numbers above one launch's list, and two-temperature tables
+outside the usual ones against the oracle."""
 import numpy as np
 import pytest
 
 from corefl_amd import (Solver, _abi, air5_box_case, channel_case, load_air5_tables, load_tables, multiblock_case,
-                        sod_case, square_ogrid_case)
+                        reacting_box_case, sod_case, square_ogrid_case)
 from corefl_amd.cases import Case
 from oracle import Oracle, air5_tables
 
@@ -91,6 +92,13 @@ def air_sod(mx, my):
     return [sod_case(mx, my)], None, STATE[:2]
 
 
+def box_8th(mx, my, mz):
+    def make(_mx, _my):
+        t = load_tables()
+        return [reacting_box_case(mx, my, mz, seed=9, tables=t)], t, STATE
+    return make
+
+
 def blocks(physics, visc):
     def make(_mx, _my):
         t = load_tables() if physics == "h2" else None
@@ -105,9 +113,11 @@ def blocks(physics, visc):
     (body_2d, 97, 33), (plane_8th, 33, 21), (plane_one_temperature, 65, 18), (air_sod, 101, 9),
     (plane_k_faces(3, 21), 33, 21), (plane_k_faces(21, 2), 33, 21),
     (joined_planes("air"), 41, 33), (joined_planes("air5"), 41, 33), (joined_planes("h2"), 41, 33),
+    (box_8th(101, 67, 53), 0, 0), (box_8th(250, 170, 20), 0, 0),
     (blocks("air", 0), 0, 0), (blocks("h2", 0), 0, 0), (blocks("h2", 8), 0, 0),
 ], ids=["body", "plane8", "plane1t", "sod", "k_symmetry", "k_walls", "joined_air",
-        "joined_body", "joined_h2", "blocks_air", "blocks_h2", "blocks_h2_visc8"])
+        "joined_body", "joined_h2", "box8_long_chunks", "box8_two_a_block", "blocks_air", "blocks_h2",
+        "blocks_h2_visc8"])
 def test_step_is_its_operators(make, mx, my):
     bl, tb, fields = make(mx, my)
     run = dict(bl[0].run, fixed_time_step=1)

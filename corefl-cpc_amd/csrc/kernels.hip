@@ -48,7 +48,8 @@ DEV double norm3(double a, double b, double c) { return sqrt(a * a + b * b + c *
 // 1/d and one exact-remainder correction (P. Markstein, Computation of
 // elementary functions on the IBM RISC System/6000 processor, 1990) give the
 // IEEE quotient's bits in 3 instructions instead of a division's eleven, for
-// normal x whose quotient is normal.
+// normal x whose quotient is normal.  An infinite x gives NaN instead of an
+// infinity, and a subnormal quotient may be off in its last bit.
 template <int D>
 DEV double div_by(double x) {
   constexpr double d = D, y = 1.0 / D;
@@ -57,6 +58,7 @@ DEV double div_by(double x) {
 }
 
 // the same for a divisor d whose rounded reciprocal rd serves several quotients
+// (also NaN for an infinite or zero d)
 DEV double div_rcp(double x, double d, double rd) {
   const double q = x * rd;
   return fma(fma(-d, q, x), rd, q);
@@ -998,7 +1000,8 @@ DEV void properties_store(const Zone &z, long p, bool with_transport, const Poin
 // elimination of the k gradient (k_k_gradient) gives them the plane's state, so
 // their properties are the plane's and are stored, not evaluated, for all of
 // them (with ngg = 3 that is six of seven planes; 1024x512 two-temperature air:
-// 920 + 182 us a stage -> 145 us, 395 us in the stage that fills the planes).  Tve is the one input that stays the ghost planes' own.
+// 920 + 182 us a stage -> 145 us, 395 us in the stage that fills the planes).
+// Tve is the one input that stays the ghost planes' own.
 // planes 0: plane 0 only (the ghost planes follow at the step's end).
 template <int M>
 __global__ __launch_bounds__(kBlock) void k_close_2d(Zone z, const Tab *__restrict__ tb, int transport_ghosts,
@@ -1269,16 +1272,14 @@ __global__ __launch_bounds__(kBlock) void k_vt_relax(Zone z, const Tab *__restri
 // indirectly.  Integer stoichiometric powers are evaluated as products (exact
 // for 1 and 2).
 // ---------------------------------------------------------------------------
-// reaction_temperature with smooth_reaction_temperature, src/FiniteRateChem.cu:1490-1503
-// One control temperature T^a Tve^b (smoothed) with what a reaction needs there.
-// Mechanisms use a few exponent pairs for all their reactions, so chem_rates
+// One control temperature T^a Tve^b (smoothed, reaction_temperature and
+// smooth_reaction_temperature, src/FiniteRateChem.cu:1490-1503) with what a
+// reaction needs there.  Mechanisms use a few exponent pairs for all their reactions, so chem_rates
 // evaluates the three usual ones once per point: (1, 0), (1/2, 1/2) and (0, 1).
 template <int M>
 struct CtrlTemp {
   double th, lt, it, g[kNs(M) > 0 ? kNs(M) : 1];
 };
-template <int M>
-DEV void thermo_gibbs(const Tab *__restrict__ tb, double t, double *g);
 template <int M>
 DEV void ctrl_at(const Tab *__restrict__ tb, double trx, bool want_g, CtrlTemp<M> &c) {
   c.th = 0.5 * (trx + 800.0 + sqrt((trx - 800.0) * (trx - 800.0) + 80.0 * 80.0));
@@ -1930,18 +1931,23 @@ __global__ __launch_bounds__(kReactorBlock) void k_reactors(ReactorPool P, const
 // fraction, ROK4E stages, h, cp and G/RT live on lane l, reaction r's constants
 // and rates of progress on lane r, row m of the iteration matrix in lane m's
 // registers (no LDS in the factorisation), so an operation over species is one
-// instruction instead of n_spec and nothing about the mechanism is read from
-// memory inside a step.  Values cross lanes by readlane (uniform source) or
-// through LDS where the source differs per lane.  Every sum runs in the order
-// of the one-lane kernel above, so a slot's result is the same bit for bit
-// under either kernel.
+// instruction instead of n_spec.  The reactions' constants, their lists, the
+// stoichiometry, the third bodies and the NASA-7 polynomials are held for the
+// whole launch; a step still reads the species' imw (uniform, cached), lists
+// beyond what a lane holds and NASA-9 polynomials.  Values cross lanes by
+// readlane (uniform source) or through LDS where the source differs per lane.
+// Every sum runs in the order of the one-lane kernel above, so a slot's result
+// is the same bit for bit under either kernel (where the quotients that this
+// kernel forms by div_rcp are normal: a partial density near underflow may
+// differ in its last bit).
 //
 // Bound by the latency of dependent FP64 operations while few waves share a
 // SIMD: a step is four source evaluations (log, three exponentials and the
 // Troe chain in sequence), three temperature solves, the LU factorisation and
-// its four solves.  A step takes 25 us with six reactors in flight against 49
-// with the state replicated in every lane, the tables read from memory and the
-// factors in LDS, and 58 us with 5000 in flight against 212 with a lane each.
+// its four solves.  A fixed ROK4E step of nine species takes 24 us alone
+// against 48 with the state replicated in every lane, the tables read from
+// memory and the factors in LDS, and 87 us with 5,000 in flight against 192
+// with a lane each.
 // ---------------------------------------------------------------------------
 constexpr int kWave = 64;
 

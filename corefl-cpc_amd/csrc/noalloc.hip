@@ -1,8 +1,8 @@
 // Allocation-free batch of served 0-D reactors (corefl_serve_run_noalloc).
 // No counterpart in the reference; for callers that cannot allocate device
 // memory (HIP graph capture, tight serving loops, harnesses that forbid it).
-// It runs the reactor server's kernels (admission, then k_reactors until
-// every request has reached t_end or failed) on one batch, with the chemistry
+// It runs the reactor server's kernels (admission, then k_reactors_wave or
+// k_reactors until every request has reached t_end or failed) on one batch, with the chemistry
 // tables, the slots and the admission records in the file-scope device array
 // `scratch` below instead of memory from corefl_serve_open.
 #include <hip/hip_runtime.h>
